@@ -93,8 +93,9 @@ int moearc_kv_append(moearc_ctx *c, void *k_pages, void *v_pages, const float *k
  * Refusals, in this order (kernels.cpp:1842-1852): any of c, out, q, k_pages, v_pages, block_table
  * null -> -1; kv_type not 0/1 -> -2; n_heads, n_kv_heads, head_dim, n_kv or page_tokens zero -> -2;
  * n_heads % n_kv_heads != 0 -> -2; kv_begin >= n_kv -> -2; head_dim > 1024 -> -2.
- * Paths: f16 KV with head_dim 64, a group of at most 16 heads and a power-of-two page size run the
- * split-K MFMA kernel; every other accepted shape runs a general f32 kernel. */
+ * Paths: head_dim 64 or 128 with a group of at most 16 heads, a power-of-two page size and a positive
+ * scale run the split-K MFMA kernels (f32 KV and head_dim 128 also need out, q and the pages 16-byte
+ * aligned); every other accepted shape runs a general f32 kernel. */
 int moearc_attn_decode(moearc_ctx *c, float *out, const float *q, const void *k_pages,
                        const void *v_pages, const unsigned int *block_table, const float *sinks,
                        unsigned long n_heads, unsigned long n_kv_heads, unsigned long head_dim,
@@ -129,10 +130,10 @@ int moearc_attn_decode_batched(moearc_ctx *c, void *out, unsigned int out_type, 
  * outputs), but the partial records of split spans go to a fixed 8 MiB array inside the code
  * object (MOEARC_DECODE_SCRATCH_FLOATS floats, one array per context on its device, held until the
  * context is destroyed) instead of the context's workspace, and no profiling event is recorded, so
- * the call makes no hipMalloc, hipFree, event or host allocation. Limit: n_heads x work items x 66
- * floats must fit the array (64 heads: up to 496 work items; the default split plan uses at most
- * 128); a larger call is refused with -2, checked for every launch of the call before anything is
- * enqueued. Calls of one context reuse the array in stream order; calls that overlap in time on one
+ * the call makes no hipMalloc, hipFree, event or host allocation. Limit: with f16 KV and head_dim 64,
+ * n_heads x work items x 66 floats must fit the array (64 heads: up to 496 work items; the default
+ * split plan uses at most 128); a larger call is refused with -2, checked for every launch of the call
+ * before anything is enqueued. (Other shapes are never refused for it: their splits grow to fit.) Calls of one context reuse the array in stream order; calls that overlap in time on one
  * context (e.g. graphs captured from it replayed on other streams concurrently) race. Nothing in the
  * array needs clearing between calls. */
 int moearc_attn_decode_batched_noalloc(moearc_ctx *c, void *out, unsigned int out_type, const float *q,

@@ -5,8 +5,9 @@
 // thread scores one key (a serial dot product over head_dim against q staged in LDS), the chunk's
 // max and sum are reduced across the work-group, and the P.V update is done with threads over the
 // head's channels, so the V reads of one key are coalesced. This path exists for coverage of the
-// reference's full argument space (its own tests use f32 KV, head_dim 128, page sizes 4 and 8);
-// the gpt-oss shape runs the split-K MFMA kernel in decode_splitk.hip.
+// reference's full argument space (head sizes other than 64 and 128, groups above 16, page sizes
+// that are no power of two, scales that are not positive, buffers aligned to less than 16 bytes);
+// every other call runs the split-K MFMA kernels in decode_splitk.hip.
 #include "common.h"
 
 #define GEN_THREADS 256

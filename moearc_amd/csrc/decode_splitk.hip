@@ -1,5 +1,5 @@
-// Split-K single-query paged attention for f16 KV with head_dim 64 (the gpt-oss shape: 64 query
-// heads over 8 KV heads), on gfx950 MFMA.
+// Split-K single-query paged attention on gfx950 MFMA: f16 or f32 KV, head_dim 64 (the gpt-oss shape:
+// 64 query heads over 8 KV heads) or 128 (Qwen3-30B-A3B: 32 over 4).
 //
 // Semantics are moearc_attn_decode's (kernels.cpp:1837-1919): for each query head,
 //     out = sum_j e^(s_j - M) V_j / (e^(sink - M) + sum_j e^(s_j - M)),  s_j = scale * q.K_j,
@@ -18,7 +18,8 @@
 // work-group writes per-head partial records (max, denominator, unnormalised output) and
 // moearc_attn_decode_merge, the next launch on the stream, combines them.
 //
-// Per 32-key tile (one wave), all operands in registers, no LDS:
+// Per 32-key tile (one wave), all operands in registers, no LDS. For f16 and 64 channels (the other
+// kinds differ in operand types and in P.V; see F16D128 and F32Kv):
 //   loads   K and V rows go from HBM straight into MFMA A-operand layout: lane (g, m) loads 16
 //           bytes, channels 8g..8g+7 (and 32+8g..) of key 16*blk + m.
 //   QK^T    S^T[32 keys x 16 heads] = K . Q^T, 2 key blocks x 2 channel halves of
@@ -34,6 +35,12 @@
 //           split p = p_hi + p_lo like q.
 // Heads beyond the group (columns 8..15 when the group is 8) are computed and discarded: MFMA
 // time is not the bound here, HBM is.
+//
+// The 128-channel and f32 kinds took the general kernel (decode_general.hip) before, a work-group per
+// query head with neither splits nor a shared KV read: four sequences of 2K-8K keys at 32 heads over
+// 4 KV heads of 128 f16 channels (34 MB) went from 2360 to 15.3 µs, 17 of 2K-30K reach 4.8 TB/s
+// (114.6 µs, a large copy's rate), eight of 3K-30K over f32 caches 5.2-5.4 TB/s (106.6 and 112 µs).
+// Their error against float64 is a quarter of that kernel's (2.8e-7 against 1.2e-6).
 //
 // Kernel arguments: the fields the first loads depend on (KV and block-table bases, q, sequence
 // 0's span and split, the geometry) lead the argument list as scalars, which the dispatcher
@@ -64,32 +71,23 @@ __device__ __forceinline__ float wave_max_16_32(float x) {
 
 __device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
 
-struct TileRegs {
-    u32x4_t k[2][2];  // [key block][channel half], A-operand layout
-    u32x4_t v[2][2];
-};
+// What the scores of a head start from: below any score in the log2 domain, and finite, so that a
+// tile of keys that all score -inf leaves weights of 0 and not NaN.
+#define M_START -3.0e38f
 
+template <int NO>
 struct SoftmaxState {
-    float m;        // reference max (log2 domain), uniform over the 4 lanes of a head
-    float l;        // running denominator in the m-frame, partial over this lane's keys
-    float4_t O[4];  // O^T[16*mb + 4g + r][n] in the m-frame
+    float m;         // reference max (log2 domain), uniform over the 4 lanes of a head
+    float l;         // running denominator in the m-frame, partial over this lane's keys
+    float4_t O[NO];  // unnormalised output in the m-frame, in the kind's accumulator order
 };
 
-__device__ __forceinline__ void process_tile(SoftmaxState &st, const TileRegs &r,
-                                             const half8_t (&qhi)[2], const half8_t (&qlo)[2],
-                                             const half8_t (&sel)[2], float c, uint32_t j0,
+// The softmax of one 32-key tile: S[blk] lane (g, n) element i is the raw score of key
+// j0 + 16 blk + 4g + i for head n, c the multiplier into the log2 domain. Moves the reference when
+// it must and turns S into the weights * 2^LOG2_PSCALE.
+template <int NO>
+__device__ __forceinline__ void softmax_tile(SoftmaxState<NO> &st, float4_t (&S)[2], float c, uint32_t j0,
                                              uint32_t te, uint32_t g) {
-    // QK^T: S[blk] lane (g, n) reg i = raw score of key j0 + 16*blk + 4g + i for head n
-    float4_t S[2];
-#pragma unroll
-    for (int blk = 0; blk < 2; ++blk) {
-        float4_t s = (float4_t){0.f, 0.f, 0.f, 0.f};
-        s = mfma16(as_half8(r.k[blk][0]), qhi[0], s);
-        s = mfma16(as_half8(r.k[blk][0]), qlo[0], s);
-        s = mfma16(as_half8(r.k[blk][1]), qhi[1], s);
-        s = mfma16(as_half8(r.k[blk][1]), qlo[1], s);
-        S[blk] = s;
-    }
     if (j0 + 32u > te) {  // the span's last, partial tile (uniform branch)
 #pragma unroll
         for (int i = 0; i < 8; ++i)
@@ -101,41 +99,305 @@ __device__ __forceinline__ void process_tile(SoftmaxState &st, const TileRegs &r
     // Move the reference only when some head's max outgrew it by more than the slack.
     if (__builtin_amdgcn_ballot_w64(tmax > st.m + RESCALE_SLACK) != 0) {
         const float m_new = fmaxf(st.m, tmax);
-        const float corr = exp2_fast(st.m - m_new);  // first tile: exp2(-inf) = 0
+        const float corr = exp2_fast(st.m - m_new);  // first tile: exp2 of a huge negative, 0
         st.m = m_new;
         st.l *= corr;
 #pragma unroll
-        for (int mb = 0; mb < 4; ++mb) st.O[mb] *= corr;
+        for (int mb = 0; mb < NO; ++mb) st.O[mb] *= corr;
     }
     const float bias = LOG2_PSCALE - st.m;
-    half8_t phi, plo;
     float psum = 0.f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         const float ps = exp2_fast(fmaf(S[i >> 2][i & 3], c, bias));
         psum += ps;
-        const _Float16 hi = (_Float16) ps;
-        phi[i] = hi;
-        plo[i] = (_Float16) (ps - (float) hi);
+        S[i >> 2][i & 3] = ps;
     }
     st.l += psum;
-    // V^T via the selection product, then P.V, one 16-channel block at a time
-#pragma unroll
-    for (int mb = 0; mb < 4; ++mb) {
-        const int hf = mb >> 1, sl = mb & 1;
-        const float4_t z = (float4_t){0.f, 0.f, 0.f, 0.f};
-        const float4_t t0 = mfma16(as_half8(r.v[0][hf]), sel[sl], z);  // keys 4g+i
-        const float4_t t1 = mfma16(as_half8(r.v[1][hf]), sel[sl], z);  // keys 16+4g+i
-        half8_t va;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            va[i] = (_Float16) t0[i];
-            va[4 + i] = (_Float16) t1[i];
-        }
-        st.O[mb] = mfma16(va, phi, st.O[mb]);
-        st.O[mb] = mfma16(va, plo, st.O[mb]);
-    }
 }
+
+// q as two f16 operands per 32 channels, q = (hi + lo) 2^(qexp - 1), and the score multiplier with
+// the power of two folded in: each head's q is normalised by a power of two (exact) so that the
+// split keeps full relative precision whatever q's magnitude.
+template <int NQ>
+struct SplitQuery {
+    half8_t hi[NQ], lo[NQ];
+    float c;
+    float v[8 * NQ];
+    // lane (g, n): channels 32 i + 8 g .. + 7 of head n, 0 for columns past the group
+    __device__ __forceinline__ void load(const float *qrow, uint32_t g, bool head_ok) {
+#pragma unroll
+        for (int i = 0; i < NQ; ++i) {
+            const float4_t x0 = *(const float4_t *) (qrow + 32 * i + 8 * g);
+            const float4_t x1 = *(const float4_t *) (qrow + 32 * i + 8 * g + 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[8 * i + e] = head_ok ? x0[e] : 0.f;
+                v[8 * i + 4 + e] = head_ok ? x1[e] : 0.f;
+            }
+        }
+    }
+    __device__ __forceinline__ void ready(float scale_log2e) {
+        float amax = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8 * NQ; ++i) amax = fmaxf(amax, fabsf(v[i]));
+        amax = wave_max_16_32(amax);
+        int qexp = 0;
+        if (amax > 0.f && amax < INFINITY) (void) frexpf(amax, &qexp);
+        c = ldexpf(scale_log2e, qexp - 1);  // score multiplier in the log2 domain
+#pragma unroll
+        for (int i = 0; i < NQ; ++i)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float x = ldexpf(v[8 * i + e], 1 - qexp);
+                const _Float16 h = (_Float16) x;
+                hi[i][e] = h;
+                lo[i][e] = (_Float16) (x - (float) h);
+            }
+    }
+};
+
+// ---- f16 cache, 64 channels ----------------------------------------------------------------------
+struct F16D64 {
+    static constexpr int D = 64, NO = 4;
+    using Elem = uint16_t;
+    struct Tile {
+        u32x4_t k[2][2];  // [key block][channel half], A-operand layout
+        u32x4_t v[2][2];
+    };
+    struct Query : SplitQuery<2> {
+        half8_t sel[2];  // selection operands: sel[s] lane (g, n) item i = 1 where 8g + i == 16s + n
+        __device__ __forceinline__ void ready(float scale_log2e, uint32_t g, uint32_t n) {
+            SplitQuery<2>::ready(scale_log2e);
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    sel[s][i] = (8u * g + i == 16u * s + n) ? (_Float16) 1.0f : (_Float16) 0.0f;
+        }
+    };
+    // row[blk]: the physical row of this lane's key 16 blk + m16
+    static __device__ __forceinline__ void load(Tile &r, const uint32_t (&row)[2], const Elem *k_pages,
+                                                const Elem *v_pages, uint64_t row_elems, uint32_t kvh, uint32_t g,
+                                                uint32_t) {
+#pragma unroll
+        for (int blk = 0; blk < 2; ++blk) {
+            const uint64_t off = (uint64_t) row[blk] * row_elems + (uint64_t) kvh * 64u + 8u * g;
+            const uint16_t *ks = k_pages + off;
+            const uint16_t *vs = v_pages + off;
+            r.k[blk][0] = *(const u32x4_t *) ks;
+            r.k[blk][1] = *(const u32x4_t *) (ks + 32);
+            r.v[blk][0] = *(const u32x4_t *) vs;
+            r.v[blk][1] = *(const u32x4_t *) (vs + 32);
+        }
+    }
+    static __device__ __forceinline__ void tile(SoftmaxState<NO> &st, Tile &r, const Query &q, uint32_t j0,
+                                                uint32_t te, uint32_t g, uint32_t) {
+        float4_t S[2];
+#pragma unroll
+        for (int blk = 0; blk < 2; ++blk) {
+            float4_t s = (float4_t){0.f, 0.f, 0.f, 0.f};
+            s = mfma16(as_half8(r.k[blk][0]), q.hi[0], s);
+            s = mfma16(as_half8(r.k[blk][0]), q.lo[0], s);
+            s = mfma16(as_half8(r.k[blk][1]), q.hi[1], s);
+            s = mfma16(as_half8(r.k[blk][1]), q.lo[1], s);
+            S[blk] = s;
+        }
+        softmax_tile(st, S, q.c, j0, te, g);
+        half8_t phi, plo;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float ps = S[i >> 2][i & 3];
+            const _Float16 hi = (_Float16) ps;
+            phi[i] = hi;
+            plo[i] = (_Float16) (ps - (float) hi);
+        }
+        // V^T via the selection product, then P.V, one 16-channel block at a time
+#pragma unroll
+        for (int mb = 0; mb < 4; ++mb) {
+            const int hf = mb >> 1, sl = mb & 1;
+            const float4_t z = (float4_t){0.f, 0.f, 0.f, 0.f};
+            const float4_t t0 = mfma16(as_half8(r.v[0][hf]), q.sel[sl], z);  // keys 4g+i
+            const float4_t t1 = mfma16(as_half8(r.v[1][hf]), q.sel[sl], z);  // keys 16+4g+i
+            half8_t va;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                va[i] = (_Float16) t0[i];
+                va[4 + i] = (_Float16) t1[i];
+            }
+            st.O[mb] = mfma16(va, phi, st.O[mb]);
+            st.O[mb] = mfma16(va, plo, st.O[mb]);
+        }
+    }
+    // O[mb] lane (g, n) element i: channel 16 mb + 4 g + i of head n
+    static __device__ __forceinline__ void put(float *row, const SoftmaxState<NO> &st, uint32_t g) {
+#pragma unroll
+        for (int mb = 0; mb < 4; ++mb) *(float4_t *) (row + 16u * mb + 4u * g) = st.O[mb];
+    }
+};
+
+// Row numbers of the keys a lane takes of V (16 blk + 4 g + r): lane 4 g + r holds key 4 g + r's.
+__device__ __forceinline__ uint32_t v_row(const uint32_t (&row)[2], int blk, uint32_t g, int r) {
+    return __shfl(row[blk], (int) (4u * g + r));
+}
+
+// ---- f16 cache, 128 channels: HBM-bound like the 64-channel kind, 512 bytes per key and KV head.
+// Scores as there, q in two f16 operands per 32 channels. For P.V, lane (g, m) loads channels
+// 8 m .. 8 m + 7 of key 16 blk + 4 g + r: a 16-lane group reads a whole 256-byte row, and element e
+// of the 16 lanes, widened to f32, is the A operand of a 16x16x4 f32 MFMA over keys {4 g + r} whose
+// B operand is the softmax register r as it stands: no transposition, weights in f32, at the price of
+// 4x the matrix time of the f16 product, which still leaves the matrix cores over half idle at the
+// HBM rate.
+struct F16D128 {
+    static constexpr int D = 128, NO = 8;
+    using Elem = uint16_t;
+    struct Tile {
+        u32x4_t k[2][4];  // [key block][channel quarter]
+        u32x4_t v[2][4];  // [key block][r]: channels 8 m .. of key 4 g + r
+    };
+    struct Query : SplitQuery<4> {
+        __device__ __forceinline__ void ready(float scale_log2e, uint32_t, uint32_t) { SplitQuery<4>::ready(scale_log2e); }
+    };
+    static __device__ __forceinline__ void load(Tile &r, const uint32_t (&row)[2], const Elem *k_pages,
+                                                const Elem *v_pages, uint64_t row_elems, uint32_t kvh, uint32_t g,
+                                                uint32_t m16) {
+#pragma unroll
+        for (int blk = 0; blk < 2; ++blk) {
+            const uint16_t *ks = k_pages + ((uint64_t) row[blk] * row_elems + (uint64_t) kvh * 128u + 8u * g);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) r.k[blk][i] = *(const u32x4_t *) (ks + 32 * i);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                r.v[blk][i] = *(const u32x4_t *) (v_pages + ((uint64_t) v_row(row, blk, g, i) * row_elems +
+                                                             (uint64_t) kvh * 128u + 8u * m16));
+        }
+    }
+    static __device__ __forceinline__ void tile(SoftmaxState<NO> &st, Tile &r, const Query &q, uint32_t j0,
+                                                uint32_t te, uint32_t g, uint32_t) {
+        float4_t S[2];
+#pragma unroll
+        for (int blk = 0; blk < 2; ++blk) {
+            float4_t s = (float4_t){0.f, 0.f, 0.f, 0.f}, t = s;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                s = mfma16(as_half8(r.k[blk][i]), q.hi[i], s);
+                t = mfma16(as_half8(r.k[blk][i]), q.lo[i], t);
+            }
+            // an infinite key (f16 overflow at the append) scores by q.hi's sign alone
+#pragma unroll
+            for (int i = 0; i < 4; ++i) S[blk][i] = fabsf(s[i]) == INFINITY ? s[i] : s[i] + t[i];
+        }
+        softmax_tile(st, S, q.c, j0, te, g);
+        if (j0 + 32u > te) {  // keys past the span repeat its last row: weight 0, and no 0 * inf either
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (j0 + 16u * (i >> 2) + 4u * g + (i & 3) >= te) r.v[i >> 2][i & 3] = (u32x4_t){0u, 0u, 0u, 0u};
+        }
+#pragma unroll
+        for (int blk = 0; blk < 2; ++blk)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const half8_t v = as_half8(r.v[blk][i]);
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    st.O[e] = __builtin_amdgcn_mfma_f32_16x16x4f32((float) v[e], S[blk][i], st.O[e], 0, 0, 0);
+            }
+    }
+    // O[e] lane (g, n) element i: channel 8 (4 g + i) + e of head n
+    static __device__ __forceinline__ void put(float *row, const SoftmaxState<NO> &st, uint32_t g) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int hf = 0; hf < 2; ++hf)
+                *(float4_t *) (row + 32u * g + 8u * i + 4u * hf) =
+                    (float4_t){st.O[4 * hf][i], st.O[4 * hf + 1][i], st.O[4 * hf + 2][i], st.O[4 * hf + 3][i]};
+    }
+};
+
+// ---- f32 cache, 64 or 128 channels: everything in f32, on 16x16x4 f32 MFMAs. Both contractions
+// take each lane's 16-byte loads as they come, four channels apart per instruction: scores with
+// lane (g, m) holding channels 16 i + 4 g .. + 3 of key m, outputs with channels 64 hf + 4 m .. + 3
+// of key 4 g + r (whole 256-byte row pieces per 16 lanes). 32 MFMAs per 16 keys and 64 channels:
+// the matrix cores could take about three times the HBM rate.
+template <int D_>
+struct F32Kv {
+    static constexpr int D = D_, NO = D / 16, NK = D / 16, NV = D / 64;
+    using Elem = float;
+    struct Tile {
+        float4_t k[2][NK];     // [key block][16 channels]
+        float4_t v[2][4][NV];  // [key block][r][64 channels]
+    };
+    struct Query {
+        float4_t v[NK];  // lane (g, n): channels 16 i + 4 g .. + 3 of head n
+        float c;
+        __device__ __forceinline__ void load(const float *qrow, uint32_t g, bool head_ok) {
+#pragma unroll
+            for (int i = 0; i < NK; ++i) {
+                const float4_t x = *(const float4_t *) (qrow + 16 * i + 4 * g);
+                v[i] = head_ok ? x : (float4_t){0.f, 0.f, 0.f, 0.f};
+            }
+        }
+        __device__ __forceinline__ void ready(float scale_log2e, uint32_t, uint32_t) { c = scale_log2e; }
+    };
+    static __device__ __forceinline__ void load(Tile &r, const uint32_t (&row)[2], const Elem *k_pages,
+                                                const Elem *v_pages, uint64_t row_elems, uint32_t kvh, uint32_t g,
+                                                uint32_t m16) {
+#pragma unroll
+        for (int blk = 0; blk < 2; ++blk) {
+            const float *ks = k_pages + ((uint64_t) row[blk] * row_elems + (uint64_t) kvh * D + 4u * g);
+#pragma unroll
+            for (int i = 0; i < NK; ++i) r.k[blk][i] = *(const float4_t *) (ks + 16 * i);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float *vs = v_pages + ((uint64_t) v_row(row, blk, g, i) * row_elems + (uint64_t) kvh * D + 4u * m16);
+#pragma unroll
+                for (int hf = 0; hf < NV; ++hf) r.v[blk][i][hf] = *(const float4_t *) (vs + 64 * hf);
+            }
+        }
+    }
+    static __device__ __forceinline__ void tile(SoftmaxState<NO> &st, Tile &r, const Query &q, uint32_t j0,
+                                                uint32_t te, uint32_t g, uint32_t) {
+        float4_t S[2];
+#pragma unroll
+        for (int blk = 0; blk < 2; ++blk) {
+            float4_t s = (float4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < NK; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    s = __builtin_amdgcn_mfma_f32_16x16x4f32(r.k[blk][i][e], q.v[i][e], s, 0, 0, 0);
+            S[blk] = s;
+        }
+        softmax_tile(st, S, q.c, j0, te, g);
+        if (j0 + 32u > te) {  // keys past the span repeat its last row: weight 0, and no 0 * inf either
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+#pragma unroll
+                for (int hf = 0; hf < NV; ++hf)
+                    if (j0 + 16u * (i >> 2) + 4u * g + (i & 3) >= te)
+                        r.v[i >> 2][i & 3][hf] = (float4_t){0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll
+        for (int blk = 0; blk < 2; ++blk)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int hf = 0; hf < NV; ++hf)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        st.O[4 * hf + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(r.v[blk][i][hf][e], S[blk][i],
+                                                                                st.O[4 * hf + e], 0, 0, 0);
+    }
+    // O[4 hf + e] lane (g, n) element i: channel 64 hf + 4 (4 g + i) + e of head n
+    static __device__ __forceinline__ void put(float *row, const SoftmaxState<NO> &st, uint32_t g) {
+#pragma unroll
+        for (int hf = 0; hf < NV; ++hf)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                *(float4_t *) (row + 64u * hf + 16u * g + 4u * i) =
+                    (float4_t){st.O[4 * hf][i], st.O[4 * hf + 1][i], st.O[4 * hf + 2][i], st.O[4 * hf + 3][i]};
+    }
+};
 
 // The fixed record array of the allocation-free entry point (moearc_attn_decode_batched_noalloc):
 // partial records live here instead of in the context's workspace. Each loaded instance of the code
@@ -169,17 +431,18 @@ __device__ __forceinline__ void store_out(void *out, uint32_t out_f16, uint64_t 
 
 // The split kernel. Geometry words: geo0 = pt_shift | n_kv_heads << 16, geo1 = nkb | group << 16,
 // nkb being the KV-head blocks (of KB heads) per work item.
-template <int KB, int WPK, int TILES>
-__device__ __forceinline__ void decode_body(const uint16_t *k_pages, const uint16_t *v_pages,
+template <class P, int KB, int WPK, int TILES>
+__device__ __forceinline__ void decode_body(const typename P::Elem *k_pages, const typename P::Elem *v_pages,
                                             const uint32_t *bt0, const float *q0, uint32_t kvb0,
                                             uint32_t nkv0, uint32_t slen0, uint32_t next0,
                                             uint32_t geo0, uint32_t geo1, const DecodeArgs &a) {
     constexpr int WAVES = KB * WPK;
+    constexpr uint32_t D = P::D;
     constexpr uint32_t CHUNK = 32u * TILES * WPK;  // keys of one chunk of the split
-    // a head's 64 partial outputs per row, rows 68 floats apart: the float4 writes of a 16-lane pass
-    // (16 heads, one channel quad each) then fall on 64 distinct banks (a 64-float stride put all
+    // a head's D partial outputs per row, rows D + 4 floats apart: the float4 writes of a 16-lane pass
+    // (16 heads, one channel quad each) then fall on 64 distinct banks (a stride of D floats put all
     // 16 heads on the same 16 banks)
-    constexpr uint32_t OROW = 68;
+    constexpr uint32_t OROW = D + 4u;
     __shared__ float o_lds[WAVES][16 * OROW];
     __shared__ float m_lds[WAVES][16];
     __shared__ float l_lds[WAVES][16];
@@ -202,7 +465,7 @@ __device__ __forceinline__ void decode_body(const uint16_t *k_pages, const uint1
         nkv = a.n_kv[b];
         slen = a.split_len[b];
         bt = a.block_tables + (uint64_t) b * a.bt_stride;
-        qb = a.q + (uint64_t) b * G * group * 64u;
+        qb = a.q + (uint64_t) b * G * group * D;
     }
     const uint32_t split = item - ib;
     const uint32_t nsplit = next - ib;
@@ -215,7 +478,7 @@ __device__ __forceinline__ void decode_body(const uint16_t *k_pages, const uint1
     const uint32_t g = lane >> 4, n = lane & 15u, m16 = lane & 15u;
     const bool head_ok = kvh_ok && n < group;
     const uint32_t h = kvh * group + (n < group ? n : 0u);
-    const uint64_t row_elems = (uint64_t) G * 64u;
+    const uint64_t row_elems = (uint64_t) G * D;
     const uint32_t pmask = (1u << sh) - 1u;
 
     // Block-table entries of this lane's keys in TILES tiles from key jw (j = jw + 32t + 16blk +
@@ -227,78 +490,37 @@ __device__ __forceinline__ void decode_body(const uint16_t *k_pages, const uint1
 #pragma unroll
             for (int blk = 0; blk < 2; ++blk) pid[t][blk] = bt[min(jw_ + 32u * t + 16u * blk + m16, te - 1u) >> sh];
     };
-    auto load_chunk = [&](uint32_t jw_, TileRegs (&r)[TILES], const uint32_t (&pid)[TILES][2]) {
+    auto load_chunk = [&](uint32_t jw_, typename P::Tile (&r)[TILES], const uint32_t (&pid)[TILES][2]) {
 #pragma unroll
-        for (int t = 0; t < TILES; ++t)
+        for (int t = 0; t < TILES; ++t) {
+            uint32_t row[2];
 #pragma unroll
             for (int blk = 0; blk < 2; ++blk) {
                 const uint32_t j = min(jw_ + 32u * t + 16u * blk + m16, te - 1u);
-                const uint32_t row = (pid[t][blk] << sh) | (j & pmask);
-                const uint64_t off = (uint64_t) row * row_elems + (uint64_t) kvh * 64u + 8u * g;
-                const uint16_t *ks = k_pages + off;
-                const uint16_t *vs = v_pages + off;
-                r[t].k[blk][0] = *(const u32x4_t *) ks;
-                r[t].k[blk][1] = *(const u32x4_t *) (ks + 32);
-                r[t].v[blk][0] = *(const u32x4_t *) vs;
-                r[t].v[blk][1] = *(const u32x4_t *) (vs + 32);
+                row[blk] = (pid[t][blk] << sh) | (j & pmask);
             }
+            P::load(r[t], row, k_pages, v_pages, row_elems, kvh, g, m16);
+        }
     };
 
-    SoftmaxState st;
-    st.m = -INFINITY;
+    SoftmaxState<P::NO> st;
+    st.m = M_START;
     st.l = 0.f;
 #pragma unroll
-    for (int mb = 0; mb < 4; ++mb) st.O[mb] = (float4_t){0.f, 0.f, 0.f, 0.f};
+    for (int mb = 0; mb < P::NO; ++mb) st.O[mb] = (float4_t){0.f, 0.f, 0.f, 0.f};
     uint32_t jw = tb + 32u * TILES * sub;   // this wave's first tile
     const bool active = kvh_ok && jw < te;  // uniform per wave
     if (active) {
         // ---- start-up: q and the first chunk's block-table entries leave together; the chunk's KV
         // loads leave as soon as the entries arrive, before the q arithmetic.
-        float qv[16];
-        const float *qrow = qb + (uint64_t) h * 64u;
-#pragma unroll
-        for (int hf = 0; hf < 2; ++hf) {
-            const float4_t x0 = *(const float4_t *) (qrow + 32 * hf + 8 * g);
-            const float4_t x1 = *(const float4_t *) (qrow + 32 * hf + 8 * g + 4);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                qv[8 * hf + i] = head_ok ? x0[i] : 0.f;
-                qv[8 * hf + 4 + i] = head_ok ? x1[i] : 0.f;
-            }
-        }
+        typename P::Query q;
+        q.load(qb + (uint64_t) h * D, g, head_ok);
         uint32_t pid[TILES][2];
         pages_of(jw, pid);
-        TileRegs r[TILES];
+        typename P::Tile r[TILES];
         load_chunk(jw, r, pid);
         __builtin_amdgcn_sched_barrier(0);
-
-        // Normalise each head's q by a power of two (exact) so that the hi/lo split keeps full
-        // relative precision whatever q's magnitude; the inverse power folds into the score
-        // multiplier.
-        float amax = 0.f;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(qv[i]));
-        amax = wave_max_16_32(amax);
-        int qexp = 0;
-        if (amax > 0.f && amax < INFINITY) (void) frexpf(amax, &qexp);
-        const float c = ldexpf(a.scale_log2e, qexp - 1);  // score multiplier in the log2 domain
-        half8_t qhi[2], qlo[2];
-#pragma unroll
-        for (int hf = 0; hf < 2; ++hf)
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const float x = ldexpf(qv[8 * hf + i], 1 - qexp);
-                const _Float16 hi = (_Float16) x;
-                qhi[hf][i] = hi;
-                qlo[hf][i] = (_Float16) (x - (float) hi);
-            }
-        // Selection operands: sel[s] lane (g, n) item i = 1 where 8g + i == 16s + n.
-        half8_t sel[2];
-#pragma unroll
-        for (int s = 0; s < 2; ++s)
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-                sel[s][i] = (8u * g + i == 16u * s + n) ? (_Float16) 1.0f : (_Float16) 0.0f;
+        q.ready(a.scale_log2e, g, n);
 
         // ---- key loop: every load of a chunk is issued before any of its tiles is computed, and
         // the next chunk's block-table entries leave before the computing starts. (The compiler
@@ -310,7 +532,7 @@ __device__ __forceinline__ void decode_body(const uint16_t *k_pages, const uint1
             pages_of(more ? jn : jw, pid);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int t = 0; t < TILES; ++t) process_tile(st, r[t], qhi, qlo, sel, c, jw + 32u * t, te, g);
+            for (int t = 0; t < TILES; ++t) P::tile(st, r[t], q, jw + 32u * t, te, g, n);
             if (!more) break;
             jw = jn;
             load_chunk(jw, r, pid);
@@ -322,11 +544,7 @@ __device__ __forceinline__ void decode_body(const uint16_t *k_pages, const uint1
     float l_run = st.l;
     l_run += __shfl_xor(l_run, 16);
     l_run += __shfl_xor(l_run, 32);
-    if (head_ok) {
-#pragma unroll
-        for (int mb = 0; mb < 4; ++mb)
-            *(float4_t *) (&o_lds[wave][n * OROW + 16u * mb + 4u * g]) = st.O[mb];
-    }
+    if (head_ok) P::put(&o_lds[wave][n * OROW], st, g);
     if (g == 0) {
         m_lds[wave][n] = head_ok && active ? st.m : -INFINITY;
         l_lds[wave][n] = head_ok && active ? l_run : 0.f;
@@ -334,14 +552,14 @@ __device__ __forceinline__ void decode_body(const uint16_t *k_pages, const uint1
     __syncthreads();
 
     // Threads take (KV head of the block, output element) pairs.
-    const uint32_t n_out = group * 64u;
+    const uint32_t n_out = group * D;
     const bool single = nsplit == 1u;
     const uint32_t H = G * group;
     for (uint32_t idx = threadIdx.x; idx < KB * n_out; idx += 64u * WAVES) {
         const uint32_t k2 = idx / n_out, e = idx - k2 * n_out;
         const uint32_t kv2 = kbi * KB + k2;
         if (kv2 >= G) break;
-        const uint32_t hn = e >> 6, d = e & 63u;
+        const uint32_t hn = e / D, d = e % D;
         float M = -INFINITY;
 #pragma unroll
         for (int w = 0; w < WPK; ++w) M = fmaxf(M, m_lds[w * KB + k2][hn]);
@@ -357,11 +575,11 @@ __device__ __forceinline__ void decode_body(const uint16_t *k_pages, const uint1
         const uint32_t hh = kv2 * group + hn;
         if (single) {
             const float sink2 = a.sinks ? a.sinks[hh] * MOEARC_LOG2E : -INFINITY;
-            store_out(a.out, a.out_f16, ((uint64_t) b * H + hh) * 64u + d, finish(sink2, M, L, acc));
+            store_out(a.out, a.out_f16, ((uint64_t) b * H + hh) * D + d, finish(sink2, M, L, acc));
         } else {
             // records, head-major: [head][work item], so a head's splits are contiguous
             const uint64_t r_i = (uint64_t) hh * a.n_items + item;
-            st_agent(a.rec_o + r_i * 64u + d, acc);
+            st_agent(a.rec_o + r_i * D + d, acc);
             if (d == 0) {
                 st_agent(a.rec_ml + 2u * r_i, M);
                 st_agent(a.rec_ml + 2u * r_i + 1u, L);
@@ -370,18 +588,26 @@ __device__ __forceinline__ void decode_body(const uint16_t *k_pages, const uint1
     }
 }
 
-#define DECODE_KERNEL(KB, WPK, TILES)                                                          \
-    extern "C" __global__ __launch_bounds__(64 * KB * WPK) void                               \
-        moearc_attn_decode_f16d64_k##KB##w##WPK##t##TILES(                                     \
-            const uint16_t *k_pages, const uint16_t *v_pages, const uint32_t *bt0,             \
+#define DECODE_KERNEL(NAME, P, KB, WPK, TILES, WAVES_EU)                                       \
+    extern "C" __global__ __launch_bounds__(64 * KB * WPK, WAVES_EU) void                     \
+        moearc_attn_decode_##NAME##_k##KB##w##WPK##t##TILES(                                   \
+            const P::Elem *k_pages, const P::Elem *v_pages, const uint32_t *bt0,               \
             const float *q0, uint32_t kvb0, uint32_t nkv0, uint32_t slen0, uint32_t next0,     \
             uint32_t geo0, uint32_t geo1, const DecodeArgs a) {                                \
-        decode_body<KB, WPK, TILES>(k_pages, v_pages, bt0, q0, kvb0, nkv0, slen0, next0,       \
-                                    geo0, geo1, a);                                            \
+        decode_body<P, KB, WPK, TILES>(k_pages, v_pages, bt0, q0, kvb0, nkv0, slen0, next0,    \
+                                       geo0, geo1, a);                                         \
     }
 
-DECODE_KERNEL(4, 2, 4)  // long spans: 8 waves, 256-key chunks, 32 KiB per wave in flight
-DECODE_KERNEL(1, 4, 1)  // short spans: 4 waves, 128-key chunks, many work-groups
+// Long spans: 8 waves, 32 KiB of K and V per wave in flight. Short spans: 4 waves on one KV head,
+// 128-key chunks, many work-groups. The last number is the least waves per SIMD (the 128-channel
+// f32 kind holds a 32 KiB tile per wave either way).
+DECODE_KERNEL(f16d64, F16D64, 4, 2, 4, 2)
+DECODE_KERNEL(f16d64, F16D64, 1, 4, 1, 4)
+DECODE_KERNEL(f16d128, F16D128, 1, 4, 1, 3)
+DECODE_KERNEL(f32d64, F32Kv<64>, 4, 2, 2, 2)
+DECODE_KERNEL(f32d64, F32Kv<64>, 1, 4, 1, 4)
+DECODE_KERNEL(f32d128, F32Kv<128>, 4, 2, 1, 2)
+DECODE_KERNEL(f32d128, F32Kv<128>, 1, 4, 1, 2)
 
 // (m, l, o) of two partial softmax sums over disjoint key sets, combined in the frame of the
 // larger max; a side that saw no keys has m = -inf and drops out.
@@ -395,25 +621,25 @@ __device__ __forceinline__ void merge_partial4(float &m, float &l, float4_t &o, 
     o = o * f1 + o2 * f2;
 }
 
-// Split merge. PARTS 256-thread work-groups per (query head, sequence), each owning 64 / PARTS
-// output channels (one: measured as fast as four at config 2's 128 splits, and a quarter of the
-// work-groups): lane (split group sg, channel quad c4) owns channels 4c4..4c4+3 of the part for
-// the splits sg, sg + NSG, ...; it issues every load of a round (a 16-byte piece of each of
-// MERGE_BATCH records and their (max, denominator) pairs) before using any, so up to
-// NSG * MERGE_BATCH splits cost one memory round trip, and a head's records are contiguous. The
-// split groups then combine by shuffles within a wave and through LDS across the four waves.
+// Split merge. One 256-thread work-group per (query head, sequence) (one measured as fast as four
+// at config 2's 128 splits, and a quarter of the work-groups): lane (split group sg, channel quad
+// c4) owns channels 4c4..4c4+3 for the splits sg, sg + NSG, ...; it issues every load of a round (a
+// 16-byte piece of each of MERGE_BATCH records and their (max, denominator) pairs) before using
+// any, so up to NSG * MERGE_BATCH splits cost one memory round trip, and a head's records are
+// contiguous. The split groups then combine by shuffles within a wave and through LDS across the
+// four waves.
 // Arguments: record bases, output, sinks and sequence 0's item count are preloaded scalars; the
 // struct carries the other sequences' item ranges.
 #define MERGE_BATCH 8
 
-template <int PARTS>
+template <uint32_t D>
 __device__ __forceinline__ void merge_body(const float *rec_o, const float *rec_ml, void *out,
                                            const float *sinks, uint32_t n_items, uint32_t next0,
                                            uint32_t n_heads, uint32_t out_f16, const MergeArgs &ma) {
-    constexpr uint32_t QUADS = 16 / PARTS, NSG = MOEARC_MERGE_THREADS / QUADS;
+    constexpr uint32_t QUADS = D / 4, NSG = MOEARC_MERGE_THREADS / QUADS;
     __shared__ float red[4][6][QUADS];  // [wave][m, l, o0..o3][channel quad]
     const uint32_t tid = threadIdx.x, c4 = tid % QUADS, sg = tid / QUADS, wave = tid >> 6;
-    const uint32_t b = blockIdx.y, h = blockIdx.x / PARTS, part = blockIdx.x % PARTS;
+    const uint32_t b = blockIdx.y, h = blockIdx.x;
     uint32_t ib0 = 0, ib1 = next0;
     if (b > 0) {
         ib0 = ma.item_begin[b];
@@ -424,7 +650,7 @@ __device__ __forceinline__ void merge_body(const float *rec_o, const float *rec_
     // the sink, requested with the records and first used at the end (without sinks the load reads
     // a record word, ignored)
     const float sink_raw = *(sinks ? sinks + h : rec_ml);
-    const uint32_t ch = 16u * part + 4u * c4;
+    const uint32_t ch = 4u * c4;
     const uint64_t base = (uint64_t) h * n_items + ib0;
     float m_t = -INFINITY, l_t = 0.f;
     float4_t o_t = (float4_t){0.f, 0.f, 0.f, 0.f};
@@ -434,7 +660,7 @@ __device__ __forceinline__ void merge_body(const float *rec_o, const float *rec_
 #pragma unroll
         for (int k = 0; k < MERGE_BATCH; ++k) {
             const uint64_t s = base + min(s0 + NSG * (uint32_t) k, nsplit - 1u);
-            v[k] = *(const float4_t *) (rec_o + s * 64u + ch);
+            v[k] = *(const float4_t *) (rec_o + s * D + ch);
             ml[k] = *(const float2_t *) (rec_ml + 2u * s);
         }
         __builtin_amdgcn_sched_barrier(0);  // every load of the round leaves before any is used
@@ -474,7 +700,7 @@ __device__ __forceinline__ void merge_body(const float *rec_o, const float *rec_
             merge_partial4(m_t, l_t, o_t, red[w][0][c4], red[w][1][c4],
                            (float4_t){red[w][2][c4], red[w][3][c4], red[w][4][c4], red[w][5][c4]});
         const float sink2 = sinks ? sink_raw * MOEARC_LOG2E : -INFINITY;
-        const uint64_t o = ((uint64_t) b * n_heads + h) * 64u + ch;
+        const uint64_t o = ((uint64_t) b * n_heads + h) * D + ch;
         float r4[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) r4[i] = finish(sink2, m_t, l_t, o_t[i]);
@@ -488,12 +714,13 @@ __device__ __forceinline__ void merge_body(const float *rec_o, const float *rec_
     }
 }
 
-#define MERGE_KERNEL(PARTS)                                                                    \
+#define MERGE_KERNEL(D)                                                                        \
     extern "C" __global__ __launch_bounds__(MOEARC_MERGE_THREADS) void                        \
-        moearc_attn_decode_merge_p##PARTS(const float *rec_o, const float *rec_ml, void *out,  \
-                                          const float *sinks, uint32_t n_items, uint32_t next0, \
-                                          uint32_t n_heads, uint32_t out_f16, const MergeArgs ma) { \
-        merge_body<PARTS>(rec_o, rec_ml, out, sinks, n_items, next0, n_heads, out_f16, ma);    \
+        moearc_attn_decode_merge_d##D(const float *rec_o, const float *rec_ml, void *out,      \
+                                      const float *sinks, uint32_t n_items, uint32_t next0,    \
+                                      uint32_t n_heads, uint32_t out_f16, const MergeArgs ma) { \
+        merge_body<D>(rec_o, rec_ml, out, sinks, n_items, next0, n_heads, out_f16, ma);        \
     }
 
-MERGE_KERNEL(1)
+MERGE_KERNEL(64)
+MERGE_KERNEL(128)

@@ -15,13 +15,14 @@
 // Partial results of a split decode, written by the split kernel when a sequence's span is split
 // across work items (one work item = one split of one sequence) and combined by the merge kernel.
 // Head-major, so the records of one query head are contiguous:
-//   rec_o[(h * n_items + item) * 64 + d]   un-normalised output (f32)
+//   rec_o[(h * n_items + item) * D + d]    un-normalised output (f32), D = 64 or 128 channels
 //   rec_ml[(h * n_items + item) * 2 + 0/1] running max (log2 domain) / denominator (f32)
 #define MOEARC_MERGE_THREADS 256
 
 // Floats of the code object's fixed record array (moearc_decode_scratch, 8 MiB), which the
 // allocation-free decode entry point uses in place of the context's workspace: n_heads * work items
-// * 66 floats must fit (64 heads: up to 496 work items; the planner's default is at most 128).
+// * (head_dim + 2) floats must fit (64 heads of 64: up to 496 work items; the planner's default is at
+// most 128).
 #define MOEARC_DECODE_SCRATCH_FLOATS (1u << 21)
 
 // Kernel arguments of the split-K decode that are not preloaded scalars (the leading kernel
@@ -31,10 +32,10 @@
 // KV-head block kbi, so consecutive work-groups -- which the dispatcher places on consecutive XCDs
 // -- take consecutive KV-head blocks of the same split.
 struct DecodeArgs {
-    const float *q;               // [n_seqs][n_heads][64] f32
+    const float *q;               // [n_seqs][n_heads][D] f32
     const uint32_t *block_tables; // row b at block_tables + b * bt_stride
     const float *sinks;           // [n_heads] or null
-    void *out;                    // [n_seqs][n_heads][64], f32 or f16
+    void *out;                    // [n_seqs][n_heads][D], f32 or f16
     float *rec_o;                 // partial records (see above)
     float *rec_ml;
     uint64_t bt_stride;

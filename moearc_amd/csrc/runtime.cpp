@@ -84,8 +84,8 @@ struct moearc_ctx {
     hipFunction_t f_rope_sums64 = nullptr;  // the same from the q/k/v product's split-K sums
     bool block_fused = true;  // MOEARC_BLOCK_FUSED=0: the attention block's fused steps as separate launches
     hipFunction_t f_dec_general = nullptr;
-    hipFunction_t f_dec_fast[2] = {};  // split kernels (kDecodeVariants)
-    hipFunction_t f_dec_merge = nullptr;
+    hipFunction_t f_dec_fast[4][2] = {};  // split kernels (kDecodeVariants): kind x variant
+    hipFunction_t f_dec_merge[2] = {};    // head_dim 64, 128
     unsigned merge_threads = 0;  // the merge kernel's launch bound (its work-group size)
     hipFunction_t f_mv[7][4] = {};  // matvec: format (F32 F16 Q8_0 Q4_K Q5_K Q6_K MXFP4) x pieces per lane 1/2/4/8
     hipFunction_t f_add = nullptr, f_read_floor = nullptr, f_mfma_floor = nullptr;
@@ -275,26 +275,46 @@ struct SpanList {
     SeqSpan at(size_t i) const { return kv_begin ? SeqSpan{kv_begin[i], n_kv[i]} : SeqSpan{begin0, end0}; }
 };
 
-// The split-K kernel masks keys with -inf scores before multiplying by scale*log2(e) and takes
-// its running maximum on raw scores, so it needs a positive, finite scale; any other scale runs on
-// the general kernel.
-bool fast_decode_ok(unsigned long n_heads, unsigned long n_kv_heads, unsigned long head_dim,
-                    unsigned long page_tokens, unsigned int kv_type, float scale) {
-    return kv_type == 1u && head_dim == 64 && n_heads / n_kv_heads <= 16 && n_kv_heads <= 0xFFFFul &&
-           is_pow2(page_tokens) && page_tokens <= (1ul << 30) && scale > 0.f && scale <= 3.0e38f;
+// The split kernels' cache layouts: f16 and f32 entries, heads of 64 and 128 channels.
+enum DecodeKind { kF16D64, kF16D128, kF32D64, kF32D128, kNumDecodeKinds, kGeneral = -1 };
+
+// The split-K kernels mask keys with -inf scores before multiplying by scale*log2(e) and take
+// their running maximum on raw scores, so they need a positive, finite scale; they load rows in
+// 16-byte pieces and hold the query heads of a KV head in 16 matrix columns. Any other call runs on
+// the general kernel, a serial scan per head: four sequences of 2K-8K keys at 32 heads over 4 KV
+// heads of 128 f16 channels take it 2370 µs.
+DecodeKind decode_kind(const void *out, const float *q, const void *k_pages, const void *v_pages, unsigned long n_heads,
+                       unsigned long n_kv_heads, unsigned long head_dim, unsigned long page_tokens,
+                       unsigned int kv_type, float scale) {
+    if ((head_dim != 64 && head_dim != 128) || n_heads / n_kv_heads > 16 || n_kv_heads > 0xFFFFul ||
+        !is_pow2(page_tokens) || page_tokens > (1ul << 30) || !(scale > 0.f && scale <= 3.0e38f))
+        return kGeneral;
+    if (kv_type == 1u && head_dim == 64) return kF16D64;
+    if (((uintptr_t) out | (uintptr_t) q | (uintptr_t) k_pages | (uintptr_t) v_pages) % 16 != 0) return kGeneral;
+    return kv_type == 1u ? kF16D128 : head_dim == 64 ? kF32D64 : kF32D128;
 }
 
-// Split-K decode variants (moearc_attn_decode_f16d64_k<kb>w<wpk>t<tiles>): kb KV heads x wpk
-// waves per work-group, each wave computing `tiles` 32-key tiles per chunk with all of their loads
-// in flight; the work-group count the split length aims for.
+unsigned long kind_dim(DecodeKind k) { return k == kF16D64 || k == kF32D64 ? 64 : 128; }
+
+// Split-K decode variants (moearc_attn_decode_<kind>_k<kb>w<wpk>t<tiles>): kb KV heads x wpk waves
+// per work-group, each wave computing `tiles` 32-key tiles per chunk with all of their loads in
+// flight; the work-group count the split length aims for. Each kind has a short-span variant, 4
+// waves on one KV head, whose target is what its registers let the device hold at once (104, 168, 128
+// and 230 VGPRs: 4, 3, 4 and 2 work-groups per CU). All but the 128-channel f16 kind have a long-span
+// one, 8 waves (2 per SIMD, one work-group per CU) with 32 KiB each in flight. That kind's (4x2x2)
+// measured no better at any size, 22.5 against 19.3-20.0 µs over 32K keys of 4 KV heads and 114.9
+// against 114.5 over 17 sequences of 2K-30K; the f32 kinds' long-span shapes win from 8 such
+// sequences on (105.9 against 109.9 µs at 128 channels) and tie below.
 struct DecodeVariant {
     const char *name;
     unsigned kb, wpk, tiles, target_wgs;
 };
 constexpr int kNumDecodeVariants = 2;
-constexpr DecodeVariant kDecodeVariants[kNumDecodeVariants] = {
-    {"4x2x4", 4, 2, 4, 256},  // 8 waves (2 per SIMD at 214 VGPRs): one work-group per CU
-    {"1x4x1", 1, 4, 1, 1024}, // 4 waves, many small work-groups: short spans, windows
+constexpr DecodeVariant kDecodeVariants[kNumDecodeKinds][kNumDecodeVariants] = {
+    {{"4x2x4", 4, 2, 4, 256}, {"1x4x1", 1, 4, 1, 1024}},
+    {{"1x4x1", 1, 4, 1, 768}, {"1x4x1", 1, 4, 1, 768}},
+    {{"4x2x2", 4, 2, 2, 256}, {"1x4x1", 1, 4, 1, 1024}},
+    {{"4x2x1", 4, 2, 1, 256}, {"1x4x1", 1, 4, 1, 512}},
 };
 
 // Variant and keys per split. The long-span variant reads 512 contiguous bytes of every key row
@@ -305,19 +325,20 @@ constexpr DecodeVariant kDecodeVariants[kNumDecodeVariants] = {
 // work-group count (all resident at once: a second round of work-groups would start only as the
 // first finishes and double the time); ragged spans make the count a step function of the length,
 // hence the search.
-void plan_split(const moearc_ctx *c, const SeqSpan *spans, size_t cnt, unsigned long G, int &variant,
-                uint32_t &split_len) {
+void plan_split(const moearc_ctx *c, DecodeKind kind, const SeqSpan *spans, size_t cnt, unsigned long G,
+                int &variant, uint32_t &split_len) {
+    const DecodeVariant *const dv = kDecodeVariants[kind];
     uint64_t keys = 0, longest = 0;
     for (size_t i = 0; i < cnt; ++i) {
         keys += (uint64_t) (spans[i].end - spans[i].begin);
         longest = std::max<uint64_t>(longest, spans[i].end - spans[i].begin);
     }
-    auto nkb_of = [&](int v) { return (G + kDecodeVariants[v].kb - 1) / kDecodeVariants[v].kb; };
-    auto chunk_of = [&](int v) { return 32ull * kDecodeVariants[v].wpk * kDecodeVariants[v].tiles; };
+    auto nkb_of = [&](int v) { return (G + dv[v].kb - 1) / dv[v].kb; };
+    auto chunk_of = [&](int v) { return 32ull * dv[v].wpk * dv[v].tiles; };
     variant = keys * nkb_of(0) / chunk_of(0) >= 192 ? 0 : 1;
     if (c->decode_variant_override >= 0) variant = c->decode_variant_override;
     const uint64_t quantum = chunk_of(variant), nkb = nkb_of(variant);
-    const uint64_t target = kDecodeVariants[variant].target_wgs;
+    const uint64_t target = dv[variant].target_wgs;
     auto wgs_at = [&](uint64_t len) {
         uint64_t items = 0;
         for (size_t i = 0; i < cnt; ++i) items += (spans[i].end - spans[i].begin + len - 1) / len;
@@ -334,6 +355,9 @@ void plan_split(const moearc_ctx *c, const SeqSpan *spans, size_t cnt, unsigned 
     len = (len + quantum - 1) / quantum * quantum;
     split_len = (uint32_t) std::min<uint64_t>(len, 0x40000000ull);
 }
+
+// Floats of one head's record of one work item: D outputs, max and denominator.
+uint64_t record_floats(DecodeKind kind) { return kind_dim(kind) + 2; }
 
 // Launch layouts. The leading scalars are the kernel's preloaded arguments (the code object is
 // built with kernarg preloading of 14 dwords); the struct follows at its natural alignment, as the
@@ -379,11 +403,27 @@ uint64_t group_items(const SeqSpan *sub, size_t cnt, uint32_t split_len) {
     return items;
 }
 
+// The plan of a launch group whose records go to `rs`. Calls that the general kernel used to serve,
+// which keeps no records, are never refused for want of record space: their splits grow until the
+// records fit (one split per sequence needs none).
+void plan_group(const moearc_ctx *c, DecodeKind kind, const SeqSpan *sub, size_t cnt, unsigned long n_heads,
+                unsigned long G, const RecordSpace &rs, int &variant, uint32_t &split_len) {
+    plan_split(c, kind, sub, cnt, G, variant, split_len);
+    if (!rs.fixed || kind == kF16D64) return;
+    for (;;) {
+        const uint64_t items = group_items(sub, cnt, split_len);
+        if (items <= cnt || (uint64_t) n_heads * items * record_floats(kind) <= rs.cap || split_len >= 0x40000000u)
+            return;
+        split_len *= 2u;
+    }
+}
+
 int decode_launch_body(moearc_ctx *c, void *out, unsigned int out_f16, const float *q,
                        const void *k_pages, const void *v_pages, const unsigned int *block_tables,
                        unsigned long bt_stride, const SpanList &spans, const float *sinks,
                        unsigned long n_heads, unsigned long n_kv_heads, unsigned long head_dim,
-                       unsigned long page_tokens, float scale, unsigned int kv_type, RecordSpace rs);
+                       unsigned long page_tokens, float scale, unsigned int kv_type, RecordSpace rs,
+                       DecodeKind kind);
 
 int decode_launch(moearc_ctx *c, void *out, unsigned int out_f16, const float *q,
                   const void *k_pages, const void *v_pages, const unsigned int *block_tables,
@@ -392,15 +432,27 @@ int decode_launch(moearc_ctx *c, void *out, unsigned int out_f16, const float *q
                   unsigned long page_tokens, float scale, unsigned int kv_type, RecordSpace rs = {}) {
     // A fixed record buffer must hold every launch group's records: checked for all groups before
     // anything is enqueued, so a refusal leaves the stream untouched.
-    if (rs.fixed && fast_decode_ok(n_heads, n_kv_heads, head_dim, page_tokens, kv_type, scale)) {
+    const DecodeKind kind =
+        decode_kind(out, q, k_pages, v_pages, n_heads, n_kv_heads, head_dim, page_tokens, kv_type, scale);
+    // Under stream capture the kinds that the general kernel used to serve keep their records in the
+    // context's fixed array: that kernel needed no memory, so a captured call of theirs must neither
+    // allocate nor leave a graph with the address of a workspace that a later call may replace.
+    if (!rs.fixed && kind != kGeneral && kind != kF16D64) {
+        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(c->stream, &status) == hipSuccess && status == hipStreamCaptureStatusActive) {
+            rs.fixed = c->scratch;
+            rs.cap = c->scratch_floats;
+        }
+    }
+    if (rs.fixed && kind != kGeneral) {
         SeqSpan sub[MOEARC_MAX_SEQS_PER_LAUNCH];
         for (size_t s0 = 0; s0 < spans.n; s0 += MOEARC_MAX_SEQS_PER_LAUNCH) {
             const size_t cnt = group_spans(spans, s0, sub);
             int variant = 0;
             uint32_t split_len = 0;
-            plan_split(c, sub, cnt, n_kv_heads, variant, split_len);
+            plan_group(c, kind, sub, cnt, n_heads, n_kv_heads, rs, variant, split_len);
             const uint64_t items = group_items(sub, cnt, split_len);
-            if (items > cnt && (uint64_t) n_heads * items * 66u > rs.cap) return ERR_ARG;
+            if (items > cnt && (uint64_t) n_heads * items * record_floats(kind) > rs.cap) return ERR_ARG;
         }
     }
     // With profiling on, the whole call (split and merge launches, SWA and full layers alike) is
@@ -408,7 +460,7 @@ int decode_launch(moearc_ctx *c, void *out, unsigned int out_f16, const float *q
     // (kernels.cpp:1905-1916); its kernels are timed on their own only with
     // MOEARC_PROFILE_KERNELS=1. The allocation-free entry point records no events.
     hipEvent_t call0 = nullptr;
-    if (!rs.fixed && tracks(c, "attn_decode") && (call0 = take_event(c))) {
+    if (tracks(c, "attn_decode") && (call0 = take_event(c))) {
         if (hipEventRecord(call0, c->stream) != hipSuccess) {
             c->event_pool.push_back(call0);
             call0 = nullptr;
@@ -417,7 +469,7 @@ int decode_launch(moearc_ctx *c, void *out, unsigned int out_f16, const float *q
     ++c->scope_depth;
     const int rc_all = decode_launch_body(c, out, out_f16, q, k_pages, v_pages, block_tables,
                                           bt_stride, spans, sinks, n_heads, n_kv_heads, head_dim,
-                                          page_tokens, scale, kv_type, rs);
+                                          page_tokens, scale, kv_type, rs, kind);
     --c->scope_depth;
     if (call0) record_bracket(c, call0, "attn_decode", n_heads, head_dim);
     return rc_all;
@@ -427,8 +479,9 @@ int decode_launch_body(moearc_ctx *c, void *out, unsigned int out_f16, const flo
                        const void *k_pages, const void *v_pages, const unsigned int *block_tables,
                        unsigned long bt_stride, const SpanList &spans, const float *sinks,
                        unsigned long n_heads, unsigned long n_kv_heads, unsigned long head_dim,
-                       unsigned long page_tokens, float scale, unsigned int kv_type, RecordSpace rs) {
-    const bool fast_shape = fast_decode_ok(n_heads, n_kv_heads, head_dim, page_tokens, kv_type, scale);
+                       unsigned long page_tokens, float scale, unsigned int kv_type, RecordSpace rs,
+                       DecodeKind kind) {
+    const uint64_t rec_floats = kind == kGeneral ? 0 : record_floats(kind);
     SeqSpan sub[MOEARC_MAX_SEQS_PER_LAUNCH];
     for (size_t s0 = 0; s0 < spans.n; s0 += MOEARC_MAX_SEQS_PER_LAUNCH) {
         const size_t cnt = group_spans(spans, s0, sub);
@@ -438,8 +491,8 @@ int decode_launch_body(moearc_ctx *c, void *out, unsigned int out_f16, const flo
         const unsigned int *btb = block_tables + s0 * bt_stride;
         int variant = 0;
         uint32_t split_len = 0;
-        if (fast_shape) plan_split(c, sub, cnt, n_kv_heads, variant, split_len);
-        if (!fast_shape) {
+        if (kind != kGeneral) plan_group(c, kind, sub, cnt, n_heads, n_kv_heads, rs, variant, split_len);
+        if (kind == kGeneral) {
             DecodeGeneralArgs a{};
             a.q = qb;
             a.k_pages = k_pages;
@@ -465,7 +518,7 @@ int decode_launch_body(moearc_ctx *c, void *out, unsigned int out_f16, const flo
             if (rc) return rc;
             continue;
         }
-        const DecodeVariant &dv = kDecodeVariants[variant];
+        const DecodeVariant &dv = kDecodeVariants[kind][variant];
         const size_t nkb = (n_kv_heads + dv.kb - 1) / dv.kb;
         DecodeLaunch L{};
         DecodeArgs &a = L.a;
@@ -495,13 +548,13 @@ int decode_launch_body(moearc_ctx *c, void *out, unsigned int out_f16, const flo
             const size_t rec = (size_t) n_heads * items;
             float *ws = rs.fixed;
             if (ws) {
-                if (rec * 66 > rs.cap) return ERR_ARG;  // checked for every group before the first launch
+                if (rec * rec_floats > rs.cap) return ERR_ARG;  // checked for every group before the first launch
             } else {
-                if (ensure_workspace(c, rec * 66)) return ERR;
+                if (ensure_workspace(c, rec * rec_floats)) return ERR;
                 ws = c->ws;
             }
             a.rec_o = ws;
-            a.rec_ml = ws + rec * 64;
+            a.rec_ml = ws + rec * head_dim;
         }
         a.n_items = items;
         L.k_pages = (const uint16_t *) k_pages;
@@ -514,7 +567,7 @@ int decode_launch_body(moearc_ctx *c, void *out, unsigned int out_f16, const flo
         L.next0 = a.item_begin[1];
         L.geo0 = log2u(page_tokens) | (uint32_t) n_kv_heads << 16;
         L.geo1 = (uint32_t) nkb | (uint32_t) (n_heads / n_kv_heads) << 16;
-        const int rc = launch(c, c->f_dec_fast[variant], (unsigned) wgs, 64u * dv.kb * dv.wpk, L,
+        const int rc = launch(c, c->f_dec_fast[kind][variant], (unsigned) wgs, 64u * dv.kb * dv.wpk, L,
                               "attn_decode.split", n_heads, head_dim);
         if (rc) return rc;
         if (any_split) {
@@ -529,7 +582,7 @@ int decode_launch_body(moearc_ctx *c, void *out, unsigned int out_f16, const flo
             M.out_f16 = out_f16;
             for (size_t i = 0; i <= MOEARC_MAX_SEQS_PER_LAUNCH; ++i) M.m.item_begin[i] = a.item_begin[i];
             M.m.item_begin[MOEARC_MAX_SEQS_PER_LAUNCH + 1] = items;
-            const int rm = launch2d(c, c->f_dec_merge, (unsigned) n_heads, (unsigned) cnt, c->merge_threads,
+            const int rm = launch2d(c, c->f_dec_merge[head_dim == 64 ? 0 : 1], (unsigned) n_heads, (unsigned) cnt, c->merge_threads,
                                     M, "attn_decode.merge", n_heads, head_dim);
             if (rm) return rm;
         }
@@ -603,9 +656,16 @@ moearc_ctx *moearc_ctx_create(void) {
         {&c->f_rope_qkv64, "moearc_rope_qkv_chunk64_k"},
         {&c->f_rope_sums64, "moearc_rope_qkv_sums64_k"},
         {&c->f_dec_general, "moearc_attn_decode_general_k"},
-        {&c->f_dec_fast[0], "moearc_attn_decode_f16d64_k4w2t4"},
-        {&c->f_dec_fast[1], "moearc_attn_decode_f16d64_k1w4t1"},
-        {&c->f_dec_merge, "moearc_attn_decode_merge_p1"},
+        {&c->f_dec_fast[kF16D64][0], "moearc_attn_decode_f16d64_k4w2t4"},
+        {&c->f_dec_fast[kF16D64][1], "moearc_attn_decode_f16d64_k1w4t1"},
+        {&c->f_dec_fast[kF16D128][0], "moearc_attn_decode_f16d128_k1w4t1"},
+        {&c->f_dec_fast[kF16D128][1], "moearc_attn_decode_f16d128_k1w4t1"},
+        {&c->f_dec_fast[kF32D64][0], "moearc_attn_decode_f32d64_k4w2t2"},
+        {&c->f_dec_fast[kF32D64][1], "moearc_attn_decode_f32d64_k1w4t1"},
+        {&c->f_dec_fast[kF32D128][0], "moearc_attn_decode_f32d128_k4w2t1"},
+        {&c->f_dec_fast[kF32D128][1], "moearc_attn_decode_f32d128_k1w4t1"},
+        {&c->f_dec_merge[0], "moearc_attn_decode_merge_d64"},
+        {&c->f_dec_merge[1], "moearc_attn_decode_merge_d128"},
         {&c->f_add, "moearc_add_k"},
         {&c->f_read_floor, "moearc_read_floor_k"},
         {&c->f_mfma_floor, "moearc_mfma_floor_k"},
@@ -642,13 +702,15 @@ moearc_ctx *moearc_ctx_create(void) {
             return release(c);
         }
     }
-    int merge_threads = 0;
-    if (hipFuncGetAttribute(&merge_threads, HIP_FUNC_ATTRIBUTE_MAX_THREADS_PER_BLOCK, c->f_dec_merge) !=
-            hipSuccess || merge_threads != MOEARC_MERGE_THREADS) {
-        std::fprintf(stderr, "moearc: cannot read the merge kernel's work-group size\n");
-        return release(c);
+    for (hipFunction_t f : c->f_dec_merge) {
+        int merge_threads = 0;
+        if (hipFuncGetAttribute(&merge_threads, HIP_FUNC_ATTRIBUTE_MAX_THREADS_PER_BLOCK, f) != hipSuccess ||
+            merge_threads != MOEARC_MERGE_THREADS) {
+            std::fprintf(stderr, "moearc: cannot read the merge kernel's work-group size\n");
+            return release(c);
+        }
+        c->merge_threads = (unsigned) merge_threads;
     }
-    c->merge_threads = (unsigned) merge_threads;
     if (const char *pp = std::getenv("MOEARC_PREFILL_PRECISE")) c->prefill_precise = pp[0] == '1';
     if (const char *bf = std::getenv("MOEARC_BLOCK_FUSED")) c->block_fused = bf[0] != '0';
     for (int i = 0; i < 8; ++i) {
@@ -683,7 +745,7 @@ moearc_ctx *moearc_ctx_create(void) {
     c->profiling = (ev && ev[0] == '1') || c->profile_kernels;
     if (const char *w = std::getenv("MOEARC_DECODE_VARIANT")) {
         for (int i = 0; i < kNumDecodeVariants; ++i)
-            if (std::strcmp(w, kDecodeVariants[i].name) == 0) c->decode_variant_override = i;
+            if (std::strcmp(w, kDecodeVariants[kF16D64][i].name) == 0) c->decode_variant_override = i;
     }
     if (const char *s = std::getenv("MOEARC_DECODE_SPLIT")) c->split_override = std::strtoul(s, nullptr, 10);
     if (const char *pb = std::getenv("MOEARC_PF_BOOST")) {
