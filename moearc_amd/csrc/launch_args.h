@@ -109,6 +109,23 @@ struct PrefillArgs {
                                   // for boost_a * its chunks - boost_b * its partner's chunks
 };
 
+// A prefill whose query tiles alone leave compute units idle is split along the keys: tile t (of at
+// most MOEARC_PF_MAX_TILES) is cut into item_begin[t + 1] - item_begin[t] pieces of nearly equal
+// chunk counts, each a work-group per KV head that leaves the partial results of its 256 rows, and
+// moearc_attn_prefill_merge_k combines them:
+//   rec_o[((item * n_kv_heads + kvh) * 256 + row) * 64 + d]  un-normalised output (f32)
+//   rec_ml[((item * n_kv_heads + kvh) * 256 + row) * 2 + 0/1] reference max / row sum in its frame
+// A tile of one piece is finished by its work-group and has no records.
+#define MOEARC_PF_MAX_TILES 64
+#define MOEARC_PF_RECORD_FLOATS (MOEARC_PREFILL_FAST_ROWS * 66u)  // one item's records of one KV head
+struct PrefillSplitArgs {
+    PrefillArgs a;
+    float *rec_o, *rec_ml;
+    uint32_t n_items;
+    uint32_t tile_tokens;         // query tokens per tile
+    uint16_t item_begin[MOEARC_PF_MAX_TILES + 4];  // entries n_qtiles .. the end: n_items
+};
+
 // RoPE parameters (moearc_rope, moearc_rope_kv_append_chunk): theta_scale = freq_base^(-2/n_dims),
 // computed on the host; neox selects the (p, p + n_dims/2) pairing, else (2p, 2p + 1).
 // Heads per thread of the RoPE kernels (grid y runs over groups of this many heads).

@@ -79,8 +79,13 @@ typedef uint32_t u32x8_t __attribute__((ext_vector_type(8)));
         "s64", "s65", "s66", "s67", "s68", "s69", "s70", "s71", "s72", "s73", "s74", "s75", "s76",    \
         "s77", "s78", "s79", "s80", "s81", "s82", "s83", "s84", "s85", "s86", "vcc", "scc", "memory"
 
-template <int GROUP>
-__device__ __forceinline__ void prefill_fast_body(const PrefillArgs &a) {
+// SPLIT: the work-group takes a piece of its tile's key range (sp, launch_args.h), and leaves partial
+// records unless the piece is the whole range. For chunks whose tiles leave CUs idle: a work-group's
+// time is its chunk count (0.59 us per 32-key chunk alone on a CU) and about 10 us around it, so 200
+// tokens behind 16301 keys (56 work-groups of 516 chunks) took 306 us and take 74.8 in 504 pieces,
+// 16 behind 24000 443 -> 30.6, 300 behind 4000 84 -> 43.6 (64 query heads over 8 KV heads).
+template <int GROUP, bool SPLIT>
+__device__ __forceinline__ void prefill_fast_body(const PrefillArgs &a, const PrefillSplitArgs *sp) {
     constexpr uint32_t TOK = MOEARC_PREFILL_FAST_ROWS / GROUP;  // query tokens per work-group
     __shared__ __attribute__((aligned(1024))) uint8_t tiles[PFF_NBUF * PFF_BUF];
 
@@ -90,7 +95,17 @@ __device__ __forceinline__ void prefill_fast_body(const PrefillArgs &a) {
     const uint32_t kvh = blockIdx.x % G;
     const uint32_t jj = blockIdx.x / G;
     const uint32_t nqt = a.n_qtiles, hq = (nqt + 1u) >> 1;
-    const uint32_t qt = jj < hq ? nqt - 1u - jj : jj - hq;
+    uint32_t qt = jj < hq ? nqt - 1u - jj : jj - hq;
+    uint32_t item = 0, piece = 0, pieces = 1;
+    if constexpr (SPLIT) {
+        // the tile that holds this item: lane t compares with tile t's first item (longest tiles first)
+        item = sp->n_items - 1u - jj;
+        const uint32_t first = sp->item_begin[lane];
+        qt = __builtin_popcountll(__builtin_amdgcn_ballot_w64(lane < nqt && first <= item)) - 1u;
+        const uint32_t i0 = sp->item_begin[qt];
+        piece = item - i0;
+        pieces = sp->item_begin[qt + 1u] - i0;
+    }
     const uint32_t q0 = qt * TOK, q_end = min(q0 + TOK, a.n_q);
     const uint32_t h = lane >> 5, n = lane & 31u;
     const uint32_t p_last = a.pos0 + q_end - 1u;
@@ -99,8 +114,13 @@ __device__ __forceinline__ void prefill_fast_body(const PrefillArgs &a) {
     };
     // Chunks of 32 keys from the one holding the first row's window start to the one holding the
     // last row's position; tiles of two chunks from there (the last tile may hold one chunk only).
-    const uint32_t key0 = win(a.pos0 + q0) / 32u * 32u;  // first key of chunk 0
-    const uint32_t nc = (p_last - key0) / 32u + 1u;      // 32-key chunks
+    uint32_t key0 = win(a.pos0 + q0) / 32u * 32u;  // first key of chunk 0
+    uint32_t nc = (p_last - key0) / 32u + 1u;      // 32-key chunks
+    if constexpr (SPLIT) {
+        const uint32_t c0 = nc * piece / pieces, c1 = nc * (piece + 1u) / pieces;  // the host bounds nc below 2^22
+        key0 += 32u * c0;
+        nc = c1 - c0;
+    }
     const uint32_t ntiles = (nc + 1u) >> 1;
 
     // ---- pair balance: the dispatcher puts work-groups i and i + pair_half on one CU, and the issue
@@ -108,7 +128,12 @@ __device__ __forceinline__ void prefill_fast_body(const PrefillArgs &a) {
     // alone at half occupancy. The second raises its waves' priority for boost_a * (its chunks) -
     // boost_b * (its partner's chunks) chunks and returns to the default at that tile step.
     uint32_t btile = 0;
-    if (a.pair_half && blockIdx.x >= a.pair_half) {
+    if constexpr (SPLIT) {  // pieces of nearly equal length
+        if (a.pair_half && blockIdx.x >= a.pair_half) {
+            btile = min(ntiles, (uint32_t) ((a.boost_a - a.boost_b) * 0.5f * (float) nc));
+            if (btile) __builtin_amdgcn_s_setprio(1);
+        }
+    } else if (a.pair_half && blockIdx.x >= a.pair_half) {
         const uint32_t pb = blockIdx.x - a.pair_half, pjj = pb / G;
         const uint32_t pqt = pjj < hq ? nqt - 1u - pjj : pjj - hq;
         const uint32_t pq0 = pqt * TOK, pq_end = min(pq0 + TOK, a.n_q);
@@ -283,8 +308,16 @@ __device__ __forceinline__ void prefill_fast_body(const PrefillArgs &a) {
         const float sink2 = a.sinks ? a.sinks[hh] * MOEARC_LOG2E : -INFINITY;
         const float Mt = fmaxf(m_run[X], sink2);
         const float fm = __builtin_amdgcn_exp2f(m_run[X] - Mt);
-        const float inv = fm / (L * fm + __builtin_amdgcn_exp2f(sink2 - Mt + PF_LOG2_PSCALE));
+        float inv = fm / (L * fm + __builtin_amdgcn_exp2f(sink2 - Mt + PF_LOG2_PSCALE));
         const uint32_t rho = 32u * X + n;  // row of the wave
+        if constexpr (SPLIT) {
+            if (pieces > 1u) {
+                inv = 1.f;
+                if (h == 0 && tok_of(X) < q_end)
+                    *(float2_t *) (sp->rec_ml + 2u * (((uint64_t) item * G + kvh) * MOEARC_PREFILL_FAST_ROWS + 64u * wave + rho)) =
+                        (float2_t){m_run[X], L};
+            }
+        }
 #pragma unroll
         for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
@@ -297,6 +330,19 @@ __device__ __forceinline__ void prefill_fast_body(const PrefillArgs &a) {
             }
     }
     // (the reads below follow the writes in this wave's LDS order; other waves' rows are not read)
+    if constexpr (SPLIT) {
+        if (pieces > 1u) {
+#pragma unroll
+            for (int k = 0; k < 16; ++k) {  // lane L: row 4k + (L >> 4), channels 4 (L & 15) .. + 3
+                const uint32_t rho = 4u * k + (lane >> 4), c = lane & 15u, r = 64u * wave + rho;
+                const float4_t v = *(const __attribute__((address_space(3))) float4_t *) (uintptr_t) (
+                    stage + rho * 256u + 16u * (c ^ (rho & 15u)));
+                float *dst = sp->rec_o + ((((uint64_t) item * G + kvh) * MOEARC_PREFILL_FAST_ROWS + r) * 64u + 4u * c);
+                if (q0 + r / GROUP < q_end) store_through16(dst, __builtin_bit_cast(u32x4_t, v));
+            }
+            return;
+        }
+    }
     auto out_row = [&](uint32_t rho) -> int64_t {  // element offset of a staged row, -1 past the chunk
         const uint32_t r = 64u * wave + rho, tk = q0 + r / GROUP;
         return tk < q_end ? (int64_t) (((uint64_t) tk * a.n_heads + kvh * GROUP + r % GROUP) * 64u) : -1;
@@ -342,10 +388,72 @@ __device__ __forceinline__ void prefill_fast_body(const PrefillArgs &a) {
 #define PREFILL_FAST_KERNEL(GRP)                                                                 \
     extern "C" __global__ __launch_bounds__(MOEARC_PREFILL_THREADS)                              \
         __attribute__((amdgpu_waves_per_eu(2, 2))) void moearc_attn_prefill_g##GRP(const PrefillArgs a) { \
-        prefill_fast_body<GRP>(a);                                                               \
+        prefill_fast_body<GRP, false>(a, nullptr);                                               \
+    }                                                                                            \
+    extern "C" __global__ __launch_bounds__(MOEARC_PREFILL_THREADS)                              \
+        __attribute__((amdgpu_waves_per_eu(2, 2))) void moearc_attn_prefill_split_g##GRP(const PrefillSplitArgs s) { \
+        prefill_fast_body<GRP, true>(s.a, &s);                                                   \
     }
 
 PREFILL_FAST_KERNEL(1)
 PREFILL_FAST_KERNEL(2)
 PREFILL_FAST_KERNEL(4)
 PREFILL_FAST_KERNEL(8)
+
+// Combines the pieces of split tiles (launch_args.h): 16 lanes per (token, head) row, lane c taking
+// channels 4c .. + 3 of each piece's record, eight pieces' loads in flight; then the sink, the
+// normalisation and the store as the unsplit kernel's. Rows of unsplit tiles are left alone.
+// Bound by the records' traffic: 33 MB of 504 pieces in 10-11 us.
+extern "C" __global__ __launch_bounds__(256) void moearc_attn_prefill_merge_k(const PrefillSplitArgs s) {
+    constexpr uint32_t B = 8;
+    const PrefillArgs &a = s.a;
+    const uint64_t row = (uint64_t) blockIdx.x * 16u + (threadIdx.x >> 4);
+    const uint32_t c = threadIdx.x & 15u, H = a.n_heads, G = a.n_kv_heads, group = a.group;
+    if (row >= (uint64_t) a.n_q * H) return;
+    const uint32_t tk = (uint32_t) (row / H), hd = (uint32_t) (row % H), kvh = hd / group;
+    const uint32_t qt = tk / s.tile_tokens, i0 = s.item_begin[qt], n = s.item_begin[qt + 1u] - i0;
+    if (n <= 1u) return;
+    const uint32_t r = (tk - qt * s.tile_tokens) * group + hd % group;
+    const float sink2 = a.sinks ? a.sinks[hd] * MOEARC_LOG2E : -INFINITY;
+    float m = PF_M_INIT, l = 0.f;
+    float4_t o = (float4_t){0.f, 0.f, 0.f, 0.f};
+    for (uint32_t p0 = 0; p0 < n; p0 += B) {
+        float4_t v[B];
+        float2_t ml[B];
+#pragma unroll
+        for (uint32_t k = 0; k < B; ++k) {
+            const uint64_t at = ((uint64_t) (i0 + min(p0 + k, n - 1u)) * G + kvh) * MOEARC_PREFILL_FAST_ROWS + r;
+            v[k] = *(const float4_t *) (s.rec_o + at * 64u + 4u * c);
+            ml[k] = *(const float2_t *) (s.rec_ml + 2u * at);
+        }
+        float mn = m;
+#pragma unroll
+        for (uint32_t k = 0; k < B; ++k) mn = fmaxf(mn, ml[k][0]);  // repeats of the last are harmless
+        const float corr = __builtin_amdgcn_exp2f(m - mn);
+        l *= corr;
+        o *= corr;
+#pragma unroll
+        for (uint32_t k = 0; k < B; ++k) {
+            const float f = p0 + k < n ? __builtin_amdgcn_exp2f(ml[k][0] - mn) : 0.f;
+            l = fmaf(ml[k][1], f, l);
+            o += v[k] * f;
+        }
+        m = mn;
+    }
+    const float Mt = fmaxf(m, sink2);
+    const float fm = __builtin_amdgcn_exp2f(m - Mt);
+    o *= fm / (l * fm + __builtin_amdgcn_exp2f(sink2 - Mt + PF_LOG2_PSCALE));
+    if (!a.out_f16) {
+        *(float4_t *) ((float *) a.out + row * 64u + 4u * c) = o;
+        return;
+    }
+    typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+    half4_t hi, lo;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        hi[i] = (_Float16) o[i];
+        lo[i] = (_Float16) (o[i] - (float) hi[i]);  // as moearc_split_f16_k
+    }
+    *(half4_t *) ((_Float16 *) a.out + row * 64u + 4u * c) = hi;
+    if (a.out_lo) *(half4_t *) ((_Float16 *) a.out_lo + row * 64u + 4u * c) = lo;
+}

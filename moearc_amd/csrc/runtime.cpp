@@ -99,7 +99,9 @@ struct moearc_ctx {
     hipFunction_t f_mm_reduce = nullptr;
     hipFunction_t f_mm_reduce4 = nullptr;  // four elements per lane, when every address allows
     hipFunction_t f_prefill[4] = {};      // group 1, 2, 4, 8
-    hipFunction_t f_prefill_precise[4] = {};  // the same with p split into f16 hi + lo
+    hipFunction_t f_prefill_split[4] = {};    // group 1, 2, 4, 8: pieces of a tile's key range
+    hipFunction_t f_prefill_merge = nullptr;
+    hipFunction_t f_prefill_precise[4] = {};  // group 1, 2, 4, 8: p split into f16 hi + lo
     bool prefill_precise = false;         // MOEARC_PREFILL_PRECISE=1: p split into f16 hi + lo
     bool profiling = false;        // MOEARC_PROFILE_EVENTS=1: one event bracket per tracked call
     bool profile_kernels = false;  // MOEARC_PROFILE_KERNELS=1: also every kernel inside a call
@@ -119,6 +121,10 @@ struct moearc_ctx {
     std::vector<Pending> pending;
     std::vector<KernelTime> totals;
     std::vector<hipEvent_t> event_pool;
+    // a split prefill's records (eager calls only: captured ones use the fixed array, so no graph
+    // holds an address that a later call may replace)
+    float *pf_ws = nullptr;
+    size_t pf_ws_floats = 0;
     // split-K workspace: the partial records of the split kernel (per query head and work item)
     float *ws = nullptr;
     size_t ws_floats = 0;
@@ -246,18 +252,25 @@ int launch(moearc_ctx *c, hipFunction_t f, unsigned grid, unsigned block, const 
     return launch2d(c, f, grid, 1, block, args, what, r, m, 0, kernel);
 }
 
-int ensure_workspace(moearc_ctx *c, size_t floats) {
-    if (floats <= c->ws_floats) return OK;
-    if (c->ws) {
+int ensure_floats(moearc_ctx *c, float *&ws, size_t &have, size_t floats) {
+    if (floats <= have) return OK;
+    if (ws) {
         // the previous workspace may still be read by queued launches
         if (hipStreamSynchronize(c->stream) != hipSuccess) return ERR;
-        if (hipFree(c->ws) != hipSuccess) return ERR;
-        c->ws = nullptr;
-        c->ws_floats = 0;
+        if (hipFree(ws) != hipSuccess) return ERR;
+        ws = nullptr;
+        have = 0;
     }
-    if (hipMalloc((void **) &c->ws, floats * sizeof(float)) != hipSuccess) return ERR;
-    c->ws_floats = floats;
+    if (hipMalloc((void **) &ws, floats * sizeof(float)) != hipSuccess) return ERR;
+    have = floats;
     return OK;
+}
+
+int ensure_workspace(moearc_ctx *c, size_t floats) { return ensure_floats(c, c->ws, c->ws_floats, floats); }
+
+bool capturing(moearc_ctx *c) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(c->stream, &status) == hipSuccess && status == hipStreamCaptureStatusActive;
 }
 
 // ---- decode dispatch ----------------------------------------------------------------------------
@@ -437,12 +450,9 @@ int decode_launch(moearc_ctx *c, void *out, unsigned int out_f16, const float *q
     // Under stream capture the kinds that the general kernel used to serve keep their records in the
     // context's fixed array: that kernel needed no memory, so a captured call of theirs must neither
     // allocate nor leave a graph with the address of a workspace that a later call may replace.
-    if (!rs.fixed && kind != kGeneral && kind != kF16D64) {
-        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(c->stream, &status) == hipSuccess && status == hipStreamCaptureStatusActive) {
-            rs.fixed = c->scratch;
-            rs.cap = c->scratch_floats;
-        }
+    if (!rs.fixed && kind != kGeneral && kind != kF16D64 && capturing(c)) {
+        rs.fixed = c->scratch;
+        rs.cap = c->scratch_floats;
     }
     if (rs.fixed && kind != kGeneral) {
         SeqSpan sub[MOEARC_MAX_SEQS_PER_LAUNCH];
@@ -600,7 +610,7 @@ moearc_ctx *release(moearc_ctx *c) {
         (void) hipEventDestroy(p.stop);
     }
     for (auto e : c->event_pool) (void) hipEventDestroy(e);
-    for (void *p : {(void *) c->ws, (void *) c->blk_ws, (void *) c->mm_ws, (void *) c->mm_part,
+    for (void *p : {(void *) c->ws, (void *) c->pf_ws, (void *) c->blk_ws, (void *) c->mm_ws, (void *) c->mm_part,
                     (void *) c->err_word})
         if (p) (void) hipFree(p);
     if (c->module) (void) hipModuleUnload(c->module);
@@ -666,6 +676,7 @@ moearc_ctx *moearc_ctx_create(void) {
         {&c->f_dec_fast[kF32D128][1], "moearc_attn_decode_f32d128_k1w4t1"},
         {&c->f_dec_merge[0], "moearc_attn_decode_merge_d64"},
         {&c->f_dec_merge[1], "moearc_attn_decode_merge_d128"},
+        {&c->f_prefill_merge, "moearc_attn_prefill_merge_k"},
         {&c->f_add, "moearc_add_k"},
         {&c->f_read_floor, "moearc_read_floor_k"},
         {&c->f_mfma_floor, "moearc_mfma_floor_k"},
@@ -713,11 +724,10 @@ moearc_ctx *moearc_ctx_create(void) {
     }
     if (const char *pp = std::getenv("MOEARC_PREFILL_PRECISE")) c->prefill_precise = pp[0] == '1';
     if (const char *bf = std::getenv("MOEARC_BLOCK_FUSED")) c->block_fused = bf[0] != '0';
-    for (int i = 0; i < 8; ++i) {
-        const bool precise = i >= 4;
+    for (int i = 0; i < 12; ++i) {
         char name[64];
-        std::snprintf(name, sizeof(name), "moearc_attn_prefill_%sg%d", precise ? "precise_" : "", 1 << (i & 3));
-        hipFunction_t *slot = precise ? &c->f_prefill_precise[i & 3] : &c->f_prefill[i & 3];
+        std::snprintf(name, sizeof(name), "moearc_attn_prefill_%sg%d", i < 4 ? "" : i < 8 ? "precise_" : "split_", 1 << (i & 3));
+        hipFunction_t *slot = (i < 4 ? c->f_prefill : i < 8 ? c->f_prefill_precise : c->f_prefill_split) + (i & 3);
         if (hipModuleGetFunction(slot, c->module, name) != hipSuccess) {
             std::fprintf(stderr, "moearc: code object %s lacks kernel %s\n", co.c_str(), name);
             return release(c);
@@ -1369,6 +1379,65 @@ bool prefill_is_fast(const moearc_ctx *c, float scale) {
     return !c->prefill_precise && c2 > 0.0f && c2 <= 3.0e38f;
 }
 
+// How a prefill whose query tiles leave compute units idle is cut along the keys: the pieces of tile t
+// are the items [begin[t], begin[t + 1]).
+struct PrefillPlan {
+    uint32_t items = 0;  // 0: not split
+    uint16_t begin[MOEARC_PF_MAX_TILES + 4];
+};
+
+// Chooses the pieces from what the launch would take, in µs: a work-group takes PF_CHUNK1 per 32-key
+// chunk alone on a CU and PF_CHUNK2 beside another (200 tokens behind 16301, 56 work-groups: 306 µs for
+// 516 chunks; 2048 behind 2048, 512: 107 µs for 193 per CU); every piece writes and reads 66 KB of
+// records, about PF_PIECE of the whole device, and the merge is a launch more (PF_MERGE). Candidates
+// are the shortest pieces for which the launch has at most 64, 128, 256 or 512 work-groups.
+// `max_records`: pieces x KV heads that the record space holds.
+void plan_prefill(const PrefillArgs &a, uint32_t tile_tokens, uint32_t n_cu, uint64_t max_records, PrefillPlan &plan) {
+    constexpr float PF_CHUNK1 = 0.59f, PF_CHUNK2 = 1.10f, PF_PIECE = 0.033f, PF_MERGE = 5.f;
+    const uint32_t T = a.n_qtiles, G = a.n_kv_heads;
+    if (!n_cu || T > MOEARC_PF_MAX_TILES || (uint64_t) T * G >= 2ull * n_cu) return;
+    uint32_t nc[MOEARC_PF_MAX_TILES], most = 0;
+    uint64_t total = 0;
+    for (uint32_t t = 0; t < T; ++t) {
+        const uint32_t q0 = t * tile_tokens, p0 = a.pos0 + q0, p1 = a.pos0 + std::min(q0 + tile_tokens, a.n_q) - 1u;
+        const uint32_t first = a.n_swa && p0 + 1u > a.n_swa ? p0 + 1u - a.n_swa : 0u;
+        nc[t] = (p1 - first / 32u * 32u) / 32u + 1u;
+        most = std::max(most, nc[t]);
+        total += nc[t];
+    }
+    if (most < 16u || most >= 1u << 22) return;  // nothing to gain over the merge; 32-bit products of chunks and pieces
+    float best = 0.9f * (T * G <= n_cu ? PF_CHUNK1 * most : std::max(PF_CHUNK1 * most, 0.5f * PF_CHUNK2 * total * G / n_cu));
+    uint32_t len = 0;
+    for (uint32_t wgs : {n_cu / 4, n_cu / 2, n_cu, 2 * n_cu}) {
+        if (wgs <= T * G) continue;
+        auto pieces_at = [&](uint32_t l) {
+            uint64_t n = 0;
+            for (uint32_t t = 0; t < T; ++t) n += (nc[t] + l - 1u) / l;
+            return n;
+        };
+        uint32_t lo = 4, hi = most;
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi) / 2;
+            if (pieces_at(mid) * G <= wgs) hi = mid;
+            else lo = mid + 1;
+        }
+        const uint64_t n = pieces_at(lo) * G;
+        if (n > wgs || n > max_records) continue;
+        const float t = (n <= n_cu ? PF_CHUNK1 : PF_CHUNK2) * lo + PF_MERGE + PF_PIECE * n;
+        if (t < best) {
+            best = t;
+            len = lo;
+        }
+    }
+    if (!len) return;
+    uint32_t at = 0;
+    for (uint32_t t = 0; t < MOEARC_PF_MAX_TILES + 4; ++t) {
+        plan.begin[t] = (uint16_t) at;
+        if (t < T) at += (nc[t] + len - 1u) / len;
+    }
+    plan.items = at;
+}
+
 // moearc_attn_prefill's checks and launch; out_lo (f16 output, default kernels only) also takes
 // the low halves of the chunk product's activation split.
 int prefill_launch(moearc_ctx *c, void *out, unsigned int out_type, uint16_t *out_lo, const void *q,
@@ -1418,6 +1487,40 @@ int prefill_launch(moearc_ctx *c, void *out, unsigned int out_type, uint16_t *ou
     a.boost_a = c->pf_boost_a;
     a.boost_b = c->pf_boost_b;
     if (wgs > 0x7FFFFFFFull) return ERR_ARG;
+    PrefillPlan plan;
+    const bool fixed = !precise && capturing(c);
+    if (!precise)
+        plan_prefill(a, rows_per_tile / (uint32_t) group, c->n_cu,
+                     fixed ? c->scratch_floats / MOEARC_PF_RECORD_FLOATS : ~0ull, plan);
+    if (plan.items) {
+        const uint64_t n = (uint64_t) plan.items * n_kv_heads;
+        PrefillSplitArgs s{};
+        a.pair_half = n > c->n_cu ? c->n_cu : 0u;
+        s.a = a;
+        if (!fixed && ensure_floats(c, c->pf_ws, c->pf_ws_floats, n * MOEARC_PF_RECORD_FLOATS)) return ERR;
+        s.rec_o = fixed ? c->scratch : c->pf_ws;
+        s.rec_ml = s.rec_o + n * MOEARC_PREFILL_FAST_ROWS * 64u;
+        s.n_items = plan.items;
+        s.tile_tokens = rows_per_tile / (uint32_t) group;
+        std::memcpy(s.item_begin, plan.begin, sizeof(plan.begin));
+        // one bracket for the call (the pieces and their merge), as for a single launch
+        hipEvent_t call0 = nullptr;
+        if (tracks(c, "attn_prefill") && (call0 = take_event(c))) {
+            if (hipEventRecord(call0, c->stream) != hipSuccess) {
+                c->event_pool.push_back(call0);
+                call0 = nullptr;
+            }
+        }
+        const bool own = c->scope_depth == 0;
+        ++c->scope_depth;
+        int rc = launch(c, c->f_prefill_split[gi], (unsigned) n, MOEARC_PREFILL_THREADS, s, "attn_prefill", n_heads, head_dim);
+        if (rc == OK)
+            rc = launch(c, c->f_prefill_merge, (unsigned) ((n_q * n_heads + 15) / 16), 256, s, nullptr, n_heads, head_dim,
+                        "attn_prefill.merge");
+        --c->scope_depth;
+        if (call0) record_bracket(c, call0, own ? "attn_prefill" : "kernel attn_prefill", n_heads, head_dim);
+        return rc;
+    }
     return launch(c, f, (unsigned) wgs, MOEARC_PREFILL_THREADS, a, "attn_prefill",
                   n_heads, head_dim);
 }
