@@ -207,6 +207,7 @@ struct MatvecArgs {
 // segments in order.
 #define MOEARC_MM_TOKENS 64    // tokens per work-group
 #define MOEARC_MM_MAX_SEG 3
+#define MOEARC_MM_SMALL_WAVES 8 // waves per work-group of matmul_small.hip
 struct MatmulSeg {
     const uint8_t *w;
     const float *bias;         // [rows] or null
@@ -220,11 +221,13 @@ struct MatmulSeg {
 struct MatmulArgs {
     MatmulSeg seg[MOEARC_MM_MAX_SEG];
     const uint16_t *xh, *xl;   // [n_tok][cols] f16: x = hi + lo to within 2^-22 |x|
-    const float *xs;           // [n_tok][cols / 32] block sums of x (Q4_K, Q5_K), else unread
+    const float *xs;           // [n_tok][cols / 32] block sums of x (Q4_K, Q5_K), else unread;
+                               // matmul_small.hip: x itself, f32 [n_tok][cols]
     float *part;               // split launches (grid z > 1): slice z's sums, [t][r] per matrix
     uint64_t part_stride;      // floats per slice: the sum of n_tok * rows over the matrices
     uint32_t n_seg, cols, n_tok;
     uint32_t accumulate;       // 1: y[t][r] += the result (the residual add), else y[t][r] = it
     uint32_t kb_per;           // k-blocks (of 32) per k-slice: work-group z takes blocks kb_per * z ..
+                               // (matmul_small.hip: wave w, kb_per * w ..)
     uint32_t pad;
 };

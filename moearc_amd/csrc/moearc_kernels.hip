@@ -8,4 +8,5 @@
 #include "rope.hip"
 #include "matvec.hip"
 #include "matmul.hip"
+#include "matmul_small.hip"
 #include "matmul2.hip"

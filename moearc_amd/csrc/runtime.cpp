@@ -90,6 +90,8 @@ struct moearc_ctx {
     hipFunction_t f_mv[7][4] = {};  // matvec: format (F32 F16 Q8_0 Q4_K Q5_K Q6_K MXFP4) x pieces per lane 1/2/4/8
     hipFunction_t f_add = nullptr, f_read_floor = nullptr, f_mfma_floor = nullptr;
     hipFunction_t f_mm[6][2] = {}, f_split = nullptr, f_split8 = nullptr, f_bsums = nullptr;  // Q8_0 F16 Q4_K Q5_K MXFP4 Q6_K x 16 / 32 rows per wave
+    hipFunction_t f_mm_small[6][4] = {};  // the same formats x 16 / 32 / 48 / 64 tokens, from f32 activations
+    unsigned long mm_small = 64;  // MOEARC_MM_SMALL: most tokens that run on them (0: none)
     hipFunction_t f_mm2[6] = {};  // Q8_0, F16, Q4_K, Q5_K, Q6_K, MXFP4: 128 x 128 tiles on the 32x32x16 MFMA
     hipFunction_t f_mm2w[3] = {};  // Q8_0, F16, MXFP4 on 128 tokens x 256 rows, eight waves
     uint16_t *mm_ws = nullptr;  // f16 hi / lo split of a chunk's activations
@@ -733,6 +735,16 @@ moearc_ctx *moearc_ctx_create(void) {
             return release(c);
         }
     }
+    constexpr const char *kMmNames[6] = {"q8_0", "f16", "q4_k", "q5_k", "mxfp4", "q6_k"};  // mm_index's order
+    for (int t = 0; t < 6; ++t)
+        for (int i = 0; i < 4; ++i) {
+            char name[64];
+            std::snprintf(name, sizeof(name), "moearc_matmul_small_%s_t%d_k", kMmNames[t], i + 1);
+            if (hipModuleGetFunction(&c->f_mm_small[t][i], c->module, name) != hipSuccess) {
+                std::fprintf(stderr, "moearc: code object %s lacks kernel %s\n", co.c_str(), name);
+                return release(c);
+            }
+        }
     for (int t = 0; t < 7; ++t) {
         for (int i = 0; i < 4; ++i) {
             if ((1u << i) > moearc_mv_ppl_max(kMvTypes[t])) continue;
@@ -771,6 +783,7 @@ moearc_ctx *moearc_ctx_create(void) {
             c->n_cu = (unsigned) ncu;
     }
     if (const char *s = std::getenv("MOEARC_MM_WIDE")) c->mm_wide = std::strtoul(s, nullptr, 10) ? 1 : 0;
+    if (const char *s = std::getenv("MOEARC_MM_SMALL")) c->mm_small = std::min(64ul, std::strtoul(s, nullptr, 10));
     if (const char *s = std::getenv("MOEARC_MM_SPLIT_WG")) c->mm_split_wg = (int) std::min(8ul, std::strtoul(s, nullptr, 10));
     return c;
 }
@@ -1590,6 +1603,45 @@ struct MmSums {
 // y = W x for n_mat matrices of one weight type over the same chunk x, given as its f16 split
 // (xh, xl) of n_tok x n_cols, in one launch (plus the split-K reduction, unless `sums` takes the
 // slices' sums instead; y is then not written).
+// Whether a product of a few tokens runs from the f32 activations in one launch, 16 weight rows per
+// work-group, the reduction cut over its 8 waves (matmul_small.hip): rows of at least one window (eight
+// k-blocks), and up to 32 tokens (gpt-oss attn_q, 4096 x 2880 Q8_0: 8.8 us at 8 tokens, 11.8 at 32,
+// against 21.9 and 23.4 in three launches) or, where the row tiles fit the device in one round (one
+// work-group per CU then), 64 (17.4 us at 63 and 64 against 27.1, and 21.7 on the 128 x 128 tiles). The
+// 5120 rows of a gpt-oss block's q, k and v are 320 tiles: 64 tokens of the block take 70 us that way
+// and 58 on the 128 x 128 tiles.
+bool mm_takes_f32(const moearc_ctx *c, unsigned long n_tok, unsigned long n_cols, uint64_t tiles16) {
+    return n_tok <= c->mm_small && n_cols >= 256 && (n_tok <= 32 || tiles16 <= 256);
+}
+
+int mm_small_launch(moearc_ctx *c, unsigned ty, const MmMat *m, unsigned n_mat, const float *x, unsigned long n_tok,
+                    unsigned long n_cols, const char *what, bool accumulate = false) {
+    if (n_mat == 0 || n_mat > MOEARC_MM_MAX_SEG) return ERR;
+    MatmulArgs a{};
+    a.accumulate = accumulate ? 1u : 0u;
+    a.xs = x;
+    a.cols = (uint32_t) n_cols;
+    a.n_tok = (uint32_t) n_tok;
+    a.n_seg = n_mat;
+    uint64_t tile_end = 0, rows = 0;
+    for (unsigned i = 0; i < n_mat; ++i) {
+        MatmulSeg &g = a.seg[i];
+        g.w = static_cast<const uint8_t *>(m[i].w);
+        g.bias = m[i].bias;
+        g.y = m[i].y;
+        g.row_bytes = (uint64_t) n_cols / moearc_mv_be(ty) * moearc_mv_bb(ty);
+        g.rows = (uint32_t) m[i].rows;
+        g.y_stride = (uint32_t) m[i].y_stride;
+        rows += m[i].rows;
+        tile_end += (m[i].rows + 15) / 16;
+        g.tile_end = (uint32_t) tile_end;
+    }
+    const uint64_t nb = n_cols / 32, gran = (ty == 12u || ty == 13u || ty == 14u) ? 8 : 1;
+    a.kb_per = (uint32_t) (((nb + MOEARC_MM_SMALL_WAVES - 1) / MOEARC_MM_SMALL_WAVES + gran - 1) / gran * gran);
+    hipFunction_t f = c->f_mm_small[mm_index(ty)][(n_tok - 1) / 16];
+    return launch2d(c, f, (unsigned) tile_end, 1, 64 * MOEARC_MM_SMALL_WAVES, a, what, rows, n_tok);
+}
+
 int mm_launch(moearc_ctx *c, unsigned ty, const MmMat *m, unsigned n_mat, const uint16_t *xh, const uint16_t *xl,
               const float *xs, unsigned long n_tok, unsigned long n_cols, const char *what,
               bool accumulate = false, MmSums *sums = nullptr) {
@@ -1609,8 +1661,9 @@ int mm_launch(moearc_ctx *c, unsigned ty, const MmMat *m, unsigned n_mat, const 
         tiles128 += (m[i].rows + 127) / 128;
         tiles256 += (m[i].rows + 255) / 256;
     }
-    // Every format over chunks of at least 64 tokens: 128 x 128 tiles on the 32x32x16 MFMA
-    // (matmul2.hip; Q8_0 and MXFP4 weights arrive there in pairs of k-blocks, so their rows must
+    // Every format over chunks of more than 32 tokens: 128 x 128 tiles on the 32x32x16 MFMA (matmul2.hip;
+    // 33 to 63 tokens of a gpt-oss block's q, k and v, too many rows for matmul_small.hip, took 70-79 us
+    // per block on the 16 x 16 x 32 kernels and take 57-58; Q8_0 and MXFP4 weights arrive there in pairs of k-blocks, so their rows must
     // hold an even number of them). Otherwise 32 rows per wave halves the activation loads per MFMA, but only
     // pays while the launch still has about two work-groups per CU; shorter chunks take 16.
     hipFunction_t f;
@@ -1618,7 +1671,7 @@ int mm_launch(moearc_ctx *c, unsigned ty, const MmMat *m, unsigned n_mat, const 
     unsigned gy;
     const bool pairs = ty == 8u || ty == 39u;
     const bool mm2 = (ty == 1u || ty == 12u || ty == 13u || ty == 14u || (pairs && (n_cols / 32) % 2 == 0)) &&
-                     n_tok >= 64;
+                     n_tok > 32;
     // F16, Q8_0 and MXFP4 take work-groups of eight waves over 128 tokens x 256 rows (one per CU)
     // when those tiles alone cover every CU in whole rounds, the last at least three quarters
     // full: each k-block's copies into LDS then serve twice the rows, and the copies' volume is
@@ -1785,10 +1838,11 @@ int moearc_matmul_q(moearc_ctx *c, unsigned int type_id, float *y, const void *w
     if (!c || !y || !w || !x) return ERR;
     if (const int rc = mm_check(type_id, w, n_tok, n_rows, n_cols)) return rc;
     if (n_rows == 0 || n_tok == 0) return OK;
+    const MmMat mat{w, bias, y, n_rows, n_rows};
+    if (mm_takes_f32(c, n_tok, n_cols, (n_rows + 15) / 16)) return mm_small_launch(c, type_id, &mat, 1, x, n_tok, n_cols, "matmul");
     uint16_t *xh, *xl;
     float *xs;
     if (const int rc = mm_split(c, x, n_tok * n_cols, &xh, &xl, &xs, mm_needs_sums(type_id))) return rc;
-    const MmMat mat{w, bias, y, n_rows, n_rows};
     return mm_launch(c, type_id, &mat, 1, xh, xl, xs, n_tok, n_cols, "matmul");
 }
 
@@ -1873,11 +1927,14 @@ int moearc_attn_block_chunk(moearc_ctx *c, const moearc_attn_block *b, float *h,
                         mm_check(b->w_type[0], b->w[0], n_tok, q_rows, E) == OK &&
                         mm_check(b->w_type[1], b->w[1], n_tok, kv_rows, E) == OK &&
                         mm_check(b->w_type[2], b->w[2], n_tok, kv_rows, E) == OK;
+    const bool small = mm_takes_f32(c, n_tok, E, (q_rows + 15) / 16 + 2 * ((kv_rows + 15) / 16)),
+               small_out = (small || n_tok <= 32) && mm_takes_f32(c, n_tok, q_rows, (E + 15) / 16);
     if (mm_qkv) {
-        uint16_t *xh, *xl;
-        float *xs;
+        uint16_t *xh = nullptr, *xl = nullptr;
+        float *xs = nullptr;
         const bool sums = mm_needs_sums(b->w_type[0]) || mm_needs_sums(b->w_type[1]) || mm_needs_sums(b->w_type[2]);
-        if (const int rc = mm_split(c, x, n_tok * E, &xh, &xl, &xs, sums)) return rc;
+        if (!small)
+            if (const int rc = mm_split(c, x, n_tok * E, &xh, &xl, &xs, sums)) return rc;
         float *outs[3] = {q, k, v};
         const unsigned long rows[3] = {q_rows, kv_rows, kv_rows};
         // the projections of one weight type in one launch (a block's q, k and v usually share it)
@@ -1891,9 +1948,10 @@ int moearc_attn_block_chunk(moearc_ctx *c, const moearc_attn_block *b, float *h,
                 done[j] = true;
                 mats[n++] = MmMat{b->w[j], b->bias[j], outs[j], rows[j], rows[j]};
             }
-            if (const int rc = mm_launch(c, b->w_type[i], mats, n, xh, xl, xs, n_tok, E, "attn_qkv_mm", false,
-                                         rope_one && n == 3 ? &qkv_sums : nullptr))
-                return rc;
+            const int rc = small ? mm_small_launch(c, b->w_type[i], mats, n, x, n_tok, E, "attn_qkv_mm")
+                                 : mm_launch(c, b->w_type[i], mats, n, xh, xl, xs, n_tok, E, "attn_qkv_mm", false,
+                                             rope_one && n == 3 ? &qkv_sums : nullptr);
+            if (rc) return rc;
         }
     } else {
         float *outs[3] = {q, k, v};
@@ -1968,7 +2026,7 @@ int moearc_attn_block_chunk(moearc_ctx *c, const moearc_attn_block *b, float *h,
     // default prefill kernels, the prefill writes the product's f16 hi + lo activation split
     // itself, in place of an f32 output and a split launch (the same halves).
     const bool proj_mm = n_tok >= 2 && mm_check(b->w_type[3], b->w[3], n_tok, E, q_rows) == OK;
-    const bool att_split = c->block_fused && proj_mm && !mm_needs_sums(b->w_type[3]) && prefill_is_fast(c, b->scale);
+    const bool att_split = c->block_fused && proj_mm && !small_out && !mm_needs_sums(b->w_type[3]) && prefill_is_fast(c, b->scale);
     uint16_t *axh = nullptr, *axl = nullptr;
     float *axs = nullptr;
     if (att_split)
@@ -1987,11 +2045,12 @@ int moearc_attn_block_chunk(moearc_ctx *c, const moearc_attn_block *b, float *h,
     // h += W_o attn (+ bias_o), the residual add folded into the product's store
     (void) proj;
     if (proj_mm) {
+        const MmMat mat{b->w[3], b->bias[3], h, E, E};
+        if (small_out) return mm_small_launch(c, b->w_type[3], &mat, 1, att, n_tok, q_rows, "attn_proj_mm", true);
         uint16_t *xh = axh, *xl = axl;
         float *xs = axs;
         if (!att_split)
             if (const int rc = mm_split(c, att, nq, &xh, &xl, &xs, mm_needs_sums(b->w_type[3]))) return rc;
-        const MmMat mat{b->w[3], b->bias[3], h, E, E};
         return mm_launch(c, b->w_type[3], &mat, 1, xh, xl, xs, n_tok, q_rows, "attn_proj_mm", true);
     }
     std::vector<MvJob> jobs;
