@@ -1,11 +1,10 @@
-// Chunk-form projections on v_mfma_f32_32x32x16_f16, for F16, Q8_0, Q4_K, Q5_K, Q6_K and MXFP4
-// weights: Y[t][r] = sum_c W[r][c] X[t][c] (+ bias[r]) for the tokens of a prompt chunk -- the GEMM
+// Chunk-form projections on v_mfma_f32_32x32x16_f16, for F16, Q8_0, Q6_K and MXFP4 weights (Q4_K and
+// Q5_K: matmul2k.hip): Y[t][r] = sum_c W[r][c] X[t][c] (+ bias[r]) for the tokens of a prompt chunk -- the GEMM
 // that the reference's prefill performs as one matvec per token (moe.rs:1942-1959, 2063-2071;
 // kernels.cpp:1046-1111). Precision is matmul.hip's: X is split into f16 hi + lo on the host side of
 // the launch (x - hi - lo <= 2^-22 |x|), a block's payload enters the MFMA as exact f16 integers
 // (E2M1 code points for MXFP4), each 32-wide block's (Q6_K: 16-wide group's) f32 sum q . (hi + lo)
-// is scaled by the block's factor in f32 (and, for Q4_K and Q5_K, its min times the activation's
-// block sum subtracted); F16 weights enter as they are. Activations must stay below 65504.
+// is scaled by the block's factor in f32; F16 weights enter as they are. Activations must stay below 65504.
 //
 // The product is computed transposed, D[token][row] = X . W^T, so that the weight rows are the MFMA's
 // N side: lane l holds D column l % 32 -- one weight row -- in all 16 of its accumulators, and a
@@ -47,12 +46,7 @@ constexpr uint32_t MM2_NBUF = 3u;
 // wave 0, 64 .. 127 from wave 1, ...), and 256 bytes per remaining wave that it fills with the same
 // tails as the wave it repeats (so every wave issues the same copies; nothing reads them)
 
-// Q4_K, Q5_K (per work-group, after the activation buffers): the k-blocks' per-token block sums
-// (128 floats, three buffers), each pair of sub-blocks' 32 payload bytes per row (the low nibbles
-// are the pair's first sub-block, the high ones its second; three buffers) and each super-block's
-// header per row (d, dmin, the 12 scale bytes; Q5_K: and the 32 bytes of fifth bits; two buffers)
-constexpr uint32_t MM2_KXS = MM2_TOK * 4u;
-// (The per-row buffers' sizes follow the tile's row count: mm2_body's KPAIR_B, KHDR_B, QUAD6_B,
+// (The per-row buffers' sizes follow the tile's row count: mm2_body's QUAD6_B,
 // HDR6_B and XPAIR_B.)
 // Q6_K (per work-group, after the activation buffers): each half super-block's (four k-blocks')
 // 64 bytes of ql and 32 of qh per row (two buffers), and each super-block's 16 scale bytes per row
@@ -151,16 +145,48 @@ __device__ __forceinline__ uint32_t mm2_lds4(uint32_t off) {
     return *(const __attribute__((address_space(3))) uint32_t *) (uintptr_t) off;
 }
 
+// D[token][row] of a wave: lane l holds rows r + 32 rt, tokens t0 + tl + 32 tt + 8 (j / 4) + j % 4 -- 32
+// consecutive rows per store instruction
+__device__ __forceinline__ void mm2_store(const MatmulArgs &a, const MmSegView &sg, const mm2_f32x16 (&acc)[2][2], uint32_t t0,
+                                          uint32_t row, uint32_t tl) {
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) {
+        const uint32_t r = row + 32u * rt;
+        if (r >= sg.rows) continue;
+        if (gridDim.z > 1) {  // one slice of a split launch: its sums, for the reduction
+#pragma unroll
+            for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+                for (int j = 0; j < 16; ++j) {
+                    const uint32_t t = t0 + tl + 32u * tt + 8u * (j >> 2) + (j & 3);
+                    if (t < a.n_tok)
+                        a.part[blockIdx.z * a.part_stride + sg.part_off + (uint64_t) t * sg.rows + r] = acc[tt][rt][j];
+                }
+            continue;
+        }
+        const float bias = sg.bias ? sg.bias[r] : 0.f;
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                const uint32_t t = t0 + tl + 32u * tt + 8u * (j >> 2) + (j & 3);
+                if (t < a.n_tok) {
+                    float *yp = sg.y + (uint64_t) t * sg.y_stride + r;
+                    const float v = acc[tt][rt][j] + bias;
+                    *yp = a.accumulate ? *yp + v : v;
+                }
+            }
+    }
+}
+
 template <uint32_t TY, bool WIDE = false>
 __device__ __forceinline__ void mm2_body(const MatmulArgs &a) {
-    constexpr bool Q8 = TY == 8, Q4K = TY == 12 || TY == 13, Q5K = TY == 13, Q6K = TY == 14, MX = TY == 39;
-    constexpr uint32_t KSB = Q5K ? 176u : 144u, KQS = Q5K ? 48u : 16u;  // super-block bytes, qs offset
+    constexpr bool Q8 = TY == 8, Q6K = TY == 14, MX = TY == 39;
     // WIDE: eight waves over 128 tokens x 256 rows, one work-group per CU; the per-wave tiles and
-    // steps are the same, each k-block's copies are shared by twice the rows. The K-quants, built
-    // this way (their per-row buffers and header copies below follow ROWS and RQ), measured no gain
-    // (Q4_K, Q5_K within noise, Q6_K 6% slower): the two waves of a SIMD then belong to one
-    // work-group and meet at every barrier, and in their VALU-heavy steps they contend where two
-    // work-groups' waves would interleave.
+    // steps are the same, each k-block's copies are shared by twice the rows. Q6_K, built
+    // this way (its per-row buffers and header copies below follow ROWS and RQ), measured 6% slower:
+    // the two waves of a SIMD then belong to one work-group and meet at every barrier, and in their
+    // VALU-heavy steps they contend where two work-groups' waves would interleave.
     static_assert(!WIDE || TY == 1 || TY == 8 || TY == 39, "wide tiles: F16, Q8_0 and MXFP4");
     constexpr uint32_t NW = WIDE ? 8u : 4u;                 // waves
     constexpr uint32_t ROWS = WIDE ? 2u * MM2_ROWS : MM2_ROWS;  // weight rows per work-group
@@ -168,15 +194,13 @@ __device__ __forceinline__ void mm2_body(const MatmulArgs &a) {
     constexpr uint32_t NAI = 16u / NW;                      // activation copies per wave and step
     constexpr uint32_t QTAIL = ROWS * 64u, QPAIR = QTAIL + NW * 256u;
     // the per-row weight buffers at this tile's row count
-    constexpr uint32_t KPAIR_B = ROWS * 32u, KHDR_B = ROWS * (Q5K ? 48u : 16u);
     constexpr uint32_t QUAD6_B = ROWS * 96u, HDR6_B = ROWS * 20u, XPAIR_B = ROWS * 36u;
     // LDS: per buffer a k-block's activation tile and (F16) its weight tile; then (Q8_0) the pair
-    // buffers, (Q4_K) the block sums, pair and header buffers
+    // buffers
     constexpr uint32_t BUF = MM2_ACT + (TY == 1 ? ROWS * 64u : 0u);
     constexpr uint32_t QBASE = MM2_NBUF * BUF;
-    constexpr uint32_t KXS = QBASE, KPAIR = KXS + MM2_NBUF * MM2_KXS, KHDR = KPAIR + MM2_NBUF * KPAIR_B;
     constexpr uint32_t K6Q = QBASE, K6H = K6Q + 2u * QUAD6_B;
-    constexpr uint32_t EXTRA = Q8 ? MM2_NBUF * QPAIR : Q4K ? KHDR - QBASE + 2u * KHDR_B
+    constexpr uint32_t EXTRA = Q8 ? MM2_NBUF * QPAIR
                              : Q6K ? 2u * QUAD6_B + 2u * HDR6_B : MX ? MM2_NBUF * XPAIR_B : 0u;
     __shared__ __attribute__((aligned(1024))) uint8_t tiles[QBASE + EXTRA];
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
@@ -230,41 +254,8 @@ __device__ __forceinline__ void mm2_body(const MatmulArgs &a) {
                            wsrc[i] + 64u * b);
         }
     };
-    // Q4_K: per k-block b (into buffers buf, qb and the header buffer of b's super-block) the block
-    // sums of the tile's tokens, b's pair of sub-blocks, b's super-block header -- three copies for
-    // every block, whichever of them repeat the previous block's bytes, so each step issues the
-    // same count. Waves from 2 on copy the same sums as waves 0 and 1, waves from RQ on the same
-    // headers as waves 0 .. RQ - 1 (the same bytes to the same places). Pair slot q = 64 wave + lane
-    // holds row q / 2's 16-byte chunk (q & 1) ^ ((row >> 3) & 1) of the pair's 32 payload bytes
-    // (qs[32 g .. 32 g + 31]).
     const uint32_t k_row = (64u * wave + lane) >> 1;
-    const uint8_t *k_psrc = sg.w + (uint64_t) min(r0 + k_row, sg.rows - 1u) * sg.row_bytes + KQS +
-                            16u * ((lane & 1u) ^ ((k_row >> 3) & 1u));
     const uint8_t *k_hsrc = sg.w + (uint64_t) min(r0 + 64u * (wave % RQ) + lane, sg.rows - 1u) * sg.row_bytes;
-    const float *k_xsrc = a.xs + (uint64_t) min(t0 + 64u * (wave & 1u) + lane, a.n_tok - 1u) * (a.cols / 32u) + kb0;
-    // Q5_K header slots: instruction i of wave w fills slots 64 s .. + 63, s = min(2 w + i, 3 RQ - 1)
-    // (the last waves repeat the last 64 slots); slot q is row q / 3's 16-byte chunk q % 3
-    auto k5slot = [&](uint32_t i) { return 64u * min(2u * wave + i, 3u * RQ - 1u); };
-    const uint8_t *k5hsrc[2];
-#pragma unroll
-    for (uint32_t i = 0; i < 2; ++i) {
-        const uint32_t q = k5slot(i) + lane;
-        k5hsrc[i] = sg.w + (uint64_t) min(r0 + q / 3u, sg.rows - 1u) * sg.row_bytes + 16u * (q % 3u);
-    }
-    auto kcopy = [&](uint32_t b, uint32_t buf, uint32_t qb) {
-        const uint32_t kb = kb0 + b;  // super-block kb / 8, pair (kb % 8) / 2
-        mm2_copy4(__builtin_amdgcn_readfirstlane(lds0 + KXS + buf * MM2_KXS + (wave & 1u) * 256u), k_xsrc + b);
-        mm2_copy16(__builtin_amdgcn_readfirstlane(lds0 + KPAIR + qb * KPAIR_B + wave * 1024u),
-                   k_psrc + KSB * (uint64_t) (kb >> 3) + 32u * ((kb & 7u) >> 1));
-        const uint32_t hbase = lds0 + KHDR + ((b >> 3) & 1u) * KHDR_B;
-        if constexpr (Q5K) {
-#pragma unroll
-            for (uint32_t i = 0; i < 2; ++i)
-                mm2_copy16(__builtin_amdgcn_readfirstlane(hbase + 16u * k5slot(i)), k5hsrc[i] + KSB * (uint64_t) (kb >> 3));
-        } else {
-            mm2_copy16(__builtin_amdgcn_readfirstlane(hbase + (wave % RQ) * 1024u), k_hsrc + KSB * (uint64_t) (kb >> 3));
-        }
-    };
     // Q8_0: the weights of blocks b, b + 1 (b even) into pair buffer qb
     auto qcopy = [&](uint32_t b, uint32_t qb) {
         const uint32_t base = lds0 + QBASE + qb * QPAIR;
@@ -358,7 +349,7 @@ __device__ __forceinline__ void mm2_body(const MatmulArgs &a) {
         mm2_copy4(__builtin_amdgcn_readfirstlane(lds0 + QBASE + qb * XPAIR_B + ROWS * 32u + (wave % RQ) * 256u),
                   x_tsrc + po);
     };
-    // block b from activation buffer buf and (Q8_0, Q4_K) pair buffer qb, b odd: the pair's second block
+    // block b from activation buffer buf and (Q8_0, MXFP4) pair buffer qb, b odd: the pair's second block
     auto compute = [&](uint32_t buf, uint32_t qb, bool odd, uint32_t b) {
         half8_t ah[2][2], al[2][2], bw[2][2];
         float d[2];
@@ -475,66 +466,6 @@ __device__ __forceinline__ void mm2_body(const MatmulArgs &a) {
                     for (int j = 0; j < 16; ++j)
                         acc[tt][rt][j] = fmaf(ds[rt][1], sg1[j], fmaf(ds[rt][0], sg0[j], acc[tt][rt][j]));
                 }
-            return;
-        }
-        if constexpr (Q4K) {
-            // this lane's 16 payload bytes of the pair (its k of both sub-blocks) and the
-            // super-block header (d, dmin, 12 scale bytes) of each row tile: both stay in their
-            // buffers for every step that reads them
-            const uint32_t sb = b & 7u;  // sub-block within the super-block (slices start on one)
-            float d1[2], m1[2];
-#pragma unroll
-            for (int rt = 0; rt < 2; ++rt) {
-                const uint32_t rl = 64u * (wave >> 1) + 32u * rt + n;
-                const u32x4_t kq = mm2_lds16(lds0 + KPAIR + qb * KPAIR_B + 32u * rl + 16u * (h ^ ((rl >> 3) & 1u)));
-                const uint32_t hrow = lds0 + KHDR + ((b >> 3) & 1u) * KHDR_B + (Q5K ? 48u : 16u) * rl;
-                const u32x4_t hd = mm2_lds16(hrow);
-                // get_scale_min_k4 (reference.rs:150-160) over the 12 scale bytes hd.y .. hd.w
-                // (a mask, not a branch or a select: those split the step and its registers spill)
-                const uint32_t i = 8u * (sb & 3u);
-                const uint32_t a1 = hd[1] >> i, a2 = hd[2] >> i, a3 = hd[3] >> i;
-                const uint32_t lo = sb < 4u ? ~0u : 0u;  // uniform
-                const uint32_t sc = ((a1 & 63u) & lo) | (((a3 & 15u) | (((a1 >> 6) & 3u) << 4)) & ~lo);
-                const uint32_t mn = ((a2 & 63u) & lo) | ((((a3 >> 4) & 15u) | (((a2 >> 6) & 3u) << 4)) & ~lo);
-                d1[rt] = (float) __builtin_bit_cast(_Float16, (uint16_t) (hd[0] & 0xFFFFu)) * (float) sc;
-                m1[rt] = (float) __builtin_bit_cast(_Float16, (uint16_t) (hd[0] >> 16)) * (float) mn;
-                const uint32_t sh = odd ? 4u : 0u;  // the pair's first sub-block: low nibbles
-                // Q5_K: element e's fifth bit is bit sb of qh[e]; this lane's elements 16 h ..
-                // + 15 have qh[16 h .. 16 h + 15], the header's chunk 1 + h
-                u32x4_t qh = {};
-                if constexpr (Q5K) qh = mm2_lds16(hrow + 16u + 16u * h);
-#pragma unroll
-                for (int s = 0; s < 2; ++s) {
-                    uint32_t w0 = (kq[2 * s] >> sh) & 0x0F0F0F0Fu, w1 = (kq[2 * s + 1] >> sh) & 0x0F0F0F0Fu;
-                    if constexpr (Q5K) {
-                        w0 |= ((qh[2 * s] >> sb) & 0x01010101u) << 4;
-                        w1 |= ((qh[2 * s + 1] >> sb) & 0x01010101u) << 4;
-                    }
-                    bw[rt][s] = mm2_u4_to_f16(mm2_u32x2{w0, w1});
-                }
-            }
-#pragma unroll
-            for (int tt = 0; tt < 2; ++tt) {
-                // the block sums of this lane's accumulators: element j is token 8 (j / 4) + 4 h + j % 4
-                float4_t xs[4];
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    xs[q] = *(const __attribute__((address_space(3))) float4_t *) (uintptr_t) (
-                        lds0 + KXS + buf * MM2_KXS + 4u * (64u * (wave & 1u) + 32u * tt + 8u * q + 4u * h));
-#pragma unroll
-                for (int rt = 0; rt < 2; ++rt) {
-                    mm2_f32x16 sblk = {};
-#pragma unroll
-                    for (int s = 0; s < 2; ++s) {
-                        sblk = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[tt][s], bw[rt][s], sblk, 0, 0, 0);
-                        sblk = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[tt][s], bw[rt][s], sblk, 0, 0, 0);
-                    }
-                    // d1 * (sum q x) - m1 * (sum x): the reference's sub-block regrouped
-#pragma unroll
-                    for (int j = 0; j < 16; ++j)
-                        acc[tt][rt][j] = fmaf(-m1[rt], xs[j >> 2][j & 3], fmaf(d1[rt], sblk[j], acc[tt][rt][j]));
-                }
-            }
             return;
         }
 #pragma unroll
@@ -663,11 +594,9 @@ __device__ __forceinline__ void mm2_body(const MatmulArgs &a) {
     } else {
     copy(0, 0);
     if constexpr (Q8) qcopy(0, 0);
-    if constexpr (Q4K) kcopy(0, 0, 0);
     if constexpr (Q6K) k6copy(0);
     if constexpr (MX) xcopy(0, 0);
     copy(min(1u, nb - 1u), 1);
-    if constexpr (Q4K) kcopy(min(1u, nb - 1u), 1, 0);
     if constexpr (Q6K) k6copy(min(1u, nb - 1u));
     if constexpr (MX) xcopy(min(1u, nb - 1u), 0);
     auto step = [&](uint32_t b, uint32_t buf, uint32_t qb, bool odd) {
@@ -676,10 +605,6 @@ __device__ __forceinline__ void mm2_body(const MatmulArgs &a) {
         __builtin_amdgcn_sched_barrier(0);
         if (Q6K)
             __builtin_amdgcn_s_waitcnt(mm2_vmcnt_lgkm0(NAI + 5u));  // NAI + 3 quads + header 2
-        else if (Q5K)
-            __builtin_amdgcn_s_waitcnt(mm2_vmcnt_lgkm0(NAI + 4u));  // NAI + sums + pair + header 2
-        else if (Q4K)
-            __builtin_amdgcn_s_waitcnt(mm2_vmcnt_lgkm0(NAI + 3u));  // NAI + sums + pair + header
         else if (!Q8)
             __builtin_amdgcn_s_waitcnt(mm2_vmcnt_lgkm0(NAI + 2u));  // F16: NAI + 2 copies; MXFP4: 4 + 2
         else if (odd)
@@ -691,8 +616,7 @@ __device__ __forceinline__ void mm2_body(const MatmulArgs &a) {
         copy(min(b + 2u, nb - 1u), (buf + 2u) % 3u);
         if constexpr (Q8)
             if (!odd) qcopy(min(b + 2u, nb - 2u), (qb + 1u) % 3u);
-        if constexpr (Q4K) kcopy(min(b + 2u, nb - 1u), (buf + 2u) % 3u, (qb + 1u) % 3u);
-        if constexpr (Q6K) k6copy(min(b + 2u, nb - 1u));
+            if constexpr (Q6K) k6copy(min(b + 2u, nb - 1u));
         if constexpr (MX) xcopy(min(b + 2u, nb - 1u), (qb + 1u) % 3u);
         __builtin_amdgcn_sched_barrier(0);
         compute(buf, qb, odd, b);
@@ -714,36 +638,7 @@ __device__ __forceinline__ void mm2_body(const MatmulArgs &a) {
     __builtin_amdgcn_s_waitcnt(mm2_vmcnt(0));  // no copy outlives the work-group
     }
 
-    // D[token][row]: lane l holds row r0 + 64 (w >> 1) + 32 rt + n, tokens 8 (j / 4) + 4 h + j % 4 of
-    // tile tt -- 32 consecutive rows per store instruction
-#pragma unroll
-    for (int rt = 0; rt < 2; ++rt) {
-        const uint32_t r = r0 + 64u * (wave >> 1) + 32u * rt + n;
-        if (r >= sg.rows) continue;
-        if (gridDim.z > 1) {  // one slice of a split launch: its sums, for the reduction
-#pragma unroll
-            for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-                for (int j = 0; j < 16; ++j) {
-                    const uint32_t t = t0 + 64u * (wave & 1u) + 32u * tt + 8u * (j >> 2) + 4u * h + (j & 3);
-                    if (t < a.n_tok)
-                        a.part[blockIdx.z * a.part_stride + sg.part_off + (uint64_t) t * sg.rows + r] = acc[tt][rt][j];
-                }
-            continue;
-        }
-        const float bias = sg.bias ? sg.bias[r] : 0.f;
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                const uint32_t t = t0 + 64u * (wave & 1u) + 32u * tt + 8u * (j >> 2) + 4u * h + (j & 3);
-                if (t < a.n_tok) {
-                    float *yp = sg.y + (uint64_t) t * sg.y_stride + r;
-                    const float v = acc[tt][rt][j] + bias;
-                    *yp = a.accumulate ? *yp + v : v;
-                }
-            }
-    }
+    mm2_store(a, sg, acc, t0, r0 + 64u * (wave >> 1) + n, 64u * (wave & 1u) + 4u * h);
 }
 
 }  // namespace
@@ -753,10 +648,6 @@ extern "C" __global__ void __launch_bounds__(256) moearc_matmul2_f16_k(MatmulArg
 extern "C" __global__ void __launch_bounds__(512) moearc_matmul2w_q8_0_k(MatmulArgs a) { mm2_body<8, true>(a); }
 extern "C" __global__ void __launch_bounds__(512) moearc_matmul2w_f16_k(MatmulArgs a) { mm2_body<1, true>(a); }
 extern "C" __global__ void __launch_bounds__(512) moearc_matmul2w_mxfp4_k(MatmulArgs a) { mm2_body<39, true>(a); }
-extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
-moearc_matmul2_q4_k_k(MatmulArgs a) { mm2_body<12>(a); }
-extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
-moearc_matmul2_q5_k_k(MatmulArgs a) { mm2_body<13>(a); }
 extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 moearc_matmul2_q6_k_k(MatmulArgs a) { mm2_body<14>(a); }
 extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))

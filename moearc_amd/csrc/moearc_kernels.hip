@@ -10,3 +10,4 @@
 #include "matmul.hip"
 #include "matmul_small.hip"
 #include "matmul2.hip"
+#include "matmul2k.hip"
