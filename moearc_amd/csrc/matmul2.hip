@@ -145,41 +145,93 @@ __device__ __forceinline__ uint32_t mm2_lds4(uint32_t off) {
     return *(const __attribute__((address_space(3))) uint32_t *) (uintptr_t) off;
 }
 
-// D[token][row] of a wave: lane l holds rows r + 32 rt, tokens t0 + tl + 32 tt + 8 (j / 4) + j % 4 -- 32
+// D[token][row] of a wave's row tile: lane l holds row r, tokens t0 + tl + 32 tt + 8 (j / 4) + j % 4 -- 32
 // consecutive rows per store instruction
-__device__ __forceinline__ void mm2_store(const MatmulArgs &a, const MmSegView &sg, const mm2_f32x16 (&acc)[2][2], uint32_t t0,
-                                          uint32_t row, uint32_t tl) {
-#pragma unroll
-    for (int rt = 0; rt < 2; ++rt) {
-        const uint32_t r = row + 32u * rt;
-        if (r >= sg.rows) continue;
-        if (gridDim.z > 1) {  // one slice of a split launch: its sums, for the reduction
-#pragma unroll
-            for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-                for (int j = 0; j < 16; ++j) {
-                    const uint32_t t = t0 + tl + 32u * tt + 8u * (j >> 2) + (j & 3);
-                    if (t < a.n_tok)
-                        a.part[blockIdx.z * a.part_stride + sg.part_off + (uint64_t) t * sg.rows + r] = acc[tt][rt][j];
-                }
-            continue;
-        }
-        const float bias = sg.bias ? sg.bias[r] : 0.f;
+__device__ __forceinline__ void mm2_store(const MatmulArgs &a, const MmSegView &sg, const mm2_f32x16 &v0, const mm2_f32x16 &v1,
+                                          uint32_t t0, uint32_t r, uint32_t tl) {
+    if (r >= sg.rows) return;
+    if (gridDim.z > 1) {  // one slice of a split launch: its sums, for the reduction
 #pragma unroll
         for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
             for (int j = 0; j < 16; ++j) {
                 const uint32_t t = t0 + tl + 32u * tt + 8u * (j >> 2) + (j & 3);
-                if (t < a.n_tok) {
-                    float *yp = sg.y + (uint64_t) t * sg.y_stride + r;
-                    const float v = acc[tt][rt][j] + bias;
-                    *yp = a.accumulate ? *yp + v : v;
-                }
+                if (t < a.n_tok)
+                    a.part[blockIdx.z * a.part_stride + sg.part_off + (uint64_t) t * sg.rows + r] = tt ? v1[j] : v0[j];
             }
+        return;
+    }
+    const float bias = sg.bias ? sg.bias[r] : 0.f;
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const uint32_t t = t0 + tl + 32u * tt + 8u * (j >> 2) + (j & 3);
+            if (t < a.n_tok) {
+                float *yp = sg.y + (uint64_t) t * sg.y_stride + r;
+                const float v = (tt ? v1[j] : v0[j]) + bias;
+                *yp = a.accumulate ? *yp + v : v;
+            }
+        }
+}
+
+// The results of a work-group whose k-slice was cut between two groups of four waves (group = 0, 1; `wave`
+// within it): each group takes one of the waves' row tiles, adds the other group's sums to its own in LDS
+// and stores them. lds: 64 KiB that no wave reads and no copy fills any more once all have met here (each wave has
+// waited for its own).
+__device__ __forceinline__ void mm2_store_halves(const MatmulArgs &a, const MmSegView &sg, mm2_f32x16 (&acc)[2][2], uint32_t group,
+                                                 uint32_t wave, uint32_t lane, uint32_t lds, uint32_t t0, uint32_t r, uint32_t tl) {
+    __syncthreads();
+    // [taking group][wave][tt][quad][lane]: 16 bytes per lane, consecutive
+    auto slot = [&](uint32_t to, int tt, int q) {
+        return (__attribute__((address_space(3))) float4_t *) (uintptr_t) (
+            lds + (((to * 4u + wave) * 2u + (uint32_t) tt) * 4u + (uint32_t) q) * 1024u + 16u * lane);
+    };
+    auto put = [&](const mm2_f32x16 &v, uint32_t to, int tt) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) *slot(to, tt, q) = (float4_t){v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+    };
+    auto add = [&](mm2_f32x16 &v, int tt) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float4_t o = *slot(group, tt, q);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[4 * q + e] += o[e];
+        }
+    };
+    if (group == 0u) {
+        put(acc[0][1], 1u, 0);
+        put(acc[1][1], 1u, 1);
+    } else {
+        put(acc[0][0], 0u, 0);
+        put(acc[1][0], 0u, 1);
+    }
+    __syncthreads();
+    if (group == 0u) {
+        add(acc[0][0], 0);
+        add(acc[1][0], 1);
+        mm2_store(a, sg, acc[0][0], acc[1][0], t0, r, tl);
+    } else {
+        add(acc[0][1], 0);
+        add(acc[1][1], 1);
+        mm2_store(a, sg, acc[0][1], acc[1][1], t0, r + 32u, tl);
     }
 }
 
-template <uint32_t TY, bool WIDE = false>
+// The k-blocks [kb0, kb0 + nb) of wave group `group` (of KS) of this work-group's k-slice, cut on a multiple
+// of GRAN; most: the larger group's count, which is the steps (barriers) that every wave goes through.
+struct Mm2Span {
+    uint32_t kb0, nb, most;
+};
+template <uint32_t KS, uint32_t GRAN>
+__device__ __forceinline__ Mm2Span mm2_span(const MatmulArgs &a, uint32_t group) {
+    const uint32_t kb0 = blockIdx.z * a.kb_per, nb = min(a.kb_per, a.cols / 32u - kb0);
+    if constexpr (KS == 1) return Mm2Span{kb0, nb, nb};
+    const uint32_t first = min(nb, (nb / 2u + GRAN - 1u) / GRAN * GRAN);
+    return group ? Mm2Span{kb0 + first, nb - first, max(first, nb - first)} : Mm2Span{kb0, first, max(first, nb - first)};
+}
+
+template <uint32_t TY, bool WIDE = false, uint32_t KS = 1>
 __device__ __forceinline__ void mm2_body(const MatmulArgs &a) {
     constexpr bool Q8 = TY == 8, Q6K = TY == 14, MX = TY == 39;
     // WIDE: eight waves over 128 tokens x 256 rows, one work-group per CU; the per-wave tiles and
@@ -188,6 +240,12 @@ __device__ __forceinline__ void mm2_body(const MatmulArgs &a) {
     // the two waves of a SIMD then belong to one work-group and meet at every barrier, and in their
     // VALU-heavy steps they contend where two work-groups' waves would interleave.
     static_assert(!WIDE || TY == 1 || TY == 8 || TY == 39, "wide tiles: F16, Q8_0 and MXFP4");
+    // KS = 2: eight waves, one work-group per CU; waves 0-3 and 4-7 are two such work-groups with LDS of
+    // their own that share one tile, take half of its reduction each and add up in LDS: 64 KiB there in
+    // place of a slice's partial sums in memory and a second launch to add them (256 tiles: 6-11% of the
+    // call). Grids of about one tile per CU run it; smaller ones, sliced, gain nothing by it: 128 tokens x
+    // 4096 x 2880 Q8_0 25.1 against 24.5 us, so their time is not the waves' steps.
+    static_assert(!WIDE || KS == 1, "one way of using eight waves");
     constexpr uint32_t NW = WIDE ? 8u : 4u;                 // waves
     constexpr uint32_t ROWS = WIDE ? 2u * MM2_ROWS : MM2_ROWS;  // weight rows per work-group
     constexpr uint32_t RQ = ROWS / 64u;                     // 64-row quarters: per-row copies by waves w % RQ
@@ -202,16 +260,19 @@ __device__ __forceinline__ void mm2_body(const MatmulArgs &a) {
     constexpr uint32_t K6Q = QBASE, K6H = K6Q + 2u * QUAD6_B;
     constexpr uint32_t EXTRA = Q8 ? MM2_NBUF * QPAIR
                              : Q6K ? 2u * QUAD6_B + 2u * HDR6_B : MX ? MM2_NBUF * XPAIR_B : 0u;
-    __shared__ __attribute__((aligned(1024))) uint8_t tiles[QBASE + EXTRA];
+    __shared__ __attribute__((aligned(1024))) uint8_t tiles[KS * (QBASE + EXTRA)];
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t wave8 = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t group = KS == 2 ? wave8 >> 2 : 0u, wave = wave8 - 4u * group;
     const uint32_t n = lane & 31u, h = lane >> 5;
     const MmSegView sg = mm_seg(a, blockIdx.x);
     const uint32_t t0 = blockIdx.y * MM2_TOK, r0 = sg.tile * ROWS;
     // this work-group's k-slice: blocks kb0 .. kb0 + nb (Q8_0: both even)
-    const uint32_t kb0 = blockIdx.z * a.kb_per, nb = min(a.kb_per, a.cols / 32u - kb0);
-    const uint32_t lds0 =
+    const Mm2Span span = mm2_span<KS, Q6K ? 8u : Q8 || MX ? 2u : 1u>(a, group);
+    const uint32_t kb0 = span.kb0, nb = span.nb;
+    const uint32_t lds_all =
         __builtin_amdgcn_readfirstlane((uint32_t) (uintptr_t) (__attribute__((address_space(3))) uint8_t *) tiles);
+    const uint32_t lds0 = lds_all + group * (QBASE + EXTRA);
 
     // Activation copies: instruction i of wave w fills region R = NAI w + i (1 KiB): half R >> 3,
     // tokens 16 (R & 7) .. + 15; lane L writes slot L of the region = chunk position L & 3 of token
@@ -592,6 +653,7 @@ __device__ __forceinline__ void mm2_body(const MatmulArgs &a) {
         if (b + 1u < nb) pstep(b + 1u, 1u);
         __builtin_amdgcn_s_waitcnt(mm2_vmcnt(0));  // no copy outlives the work-group
     } else {
+    if (KS == 1 || nb > 0u) {  // (the last k-slice may leave group 1 without a block)
     copy(0, 0);
     if constexpr (Q8) qcopy(0, 0);
     if constexpr (Q6K) k6copy(0);
@@ -635,10 +697,19 @@ __device__ __forceinline__ void mm2_body(const MatmulArgs &a) {
     if (b + 2u < nb) step(b + 2u, 2, 1, false);
     if (b + 3u < nb) step(b + 3u, 0, 1, true);
     if (b + 4u < nb) step(b + 4u, 1, 2, false);
+    }
+    if constexpr (KS == 2)
+        for (uint32_t i = nb; i < span.most; ++i) __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_s_waitcnt(mm2_vmcnt(0));  // no copy outlives the work-group
     }
 
-    mm2_store(a, sg, acc, t0, r0 + 64u * (wave >> 1) + n, 64u * (wave & 1u) + 4u * h);
+    const uint32_t r = r0 + 64u * (wave >> 1) + n, tl = 64u * (wave & 1u) + 4u * h;
+    if constexpr (KS == 2) {
+        mm2_store_halves(a, sg, acc, group, wave, lane, lds_all, t0, r, tl);
+    } else {
+        mm2_store(a, sg, acc[0][0], acc[1][0], t0, r, tl);
+        mm2_store(a, sg, acc[0][1], acc[1][1], t0, r + 32u, tl);
+    }
 }
 
 }  // namespace
@@ -652,3 +723,10 @@ extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_pe
 moearc_matmul2_q6_k_k(MatmulArgs a) { mm2_body<14>(a); }
 extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 moearc_matmul2_mxfp4_k(MatmulArgs a) { mm2_body<39>(a); }
+#define MM2_HALVES(NAME, TY)                                                                     \
+    extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))   \
+    moearc_matmul2x_##NAME##_k(MatmulArgs a) { mm2_body<TY, false, 2>(a); }
+MM2_HALVES(q8_0, 8)
+MM2_HALVES(f16, 1)
+MM2_HALVES(q6_k, 14)
+MM2_HALVES(mxfp4, 39)

@@ -27,23 +27,27 @@ namespace {
 // LDS: three activation buffers as in matmul2.hip; two buffers of a pair of sub-blocks' 32 payload
 // bytes per row (low nibbles: the first sub-block); two of a super-block's header per row (d, dmin,
 // the 12 scale bytes; Q5_K: and the 32 bytes of fifth bits); one super-block's sums per token.
-template <uint32_t TY>
+template <uint32_t TY, uint32_t KS = 1>  // KS: as mm2_body's
 __device__ __forceinline__ void mm2k_body(const MatmulArgs &a) {
     constexpr bool Q5K = TY == 13;
     constexpr uint32_t SB = Q5K ? 176u : 144u, QS = Q5K ? 48u : 16u;  // super-block bytes, offset of its nibbles
     constexpr uint32_t HDR = Q5K ? 48u : 16u, NHDR = Q5K ? 2u : 1u;   // header bytes per row, copies per wave
     constexpr uint32_t PAIR = MM2_ROWS * 32u;
     constexpr uint32_t PAIR0 = MM2_NBUF * MM2_ACT, HDR0 = PAIR0 + 2u * PAIR, SUM0 = HDR0 + 2u * MM2_ROWS * HDR;
-    __shared__ __attribute__((aligned(1024))) uint8_t tiles[SUM0 + MM2_TOK * 32u];
+    constexpr uint32_t LDS = SUM0 + MM2_TOK * 32u;
+    __shared__ __attribute__((aligned(1024))) uint8_t tiles[KS * LDS];
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t wave8 = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t group = KS == 2 ? wave8 >> 2 : 0u, wave = wave8 - 4u * group;
     const uint32_t n = lane & 31u, h = lane >> 5;
     const MmSegView sg = mm_seg(a, blockIdx.x);
     const uint32_t t0 = blockIdx.y * MM2_TOK, r0 = sg.tile * MM2_ROWS;
     // this work-group's k-slice: whole super-blocks, k-blocks kb0 .. kb0 + nb
-    const uint32_t kb0 = blockIdx.z * a.kb_per, nb = min(a.kb_per, a.cols / 32u - kb0), nsb = nb >> 3;
-    const uint32_t lds0 =
+    const Mm2Span span = mm2_span<KS, 8>(a, group);
+    const uint32_t kb0 = span.kb0, nb = span.nb, nsb = nb >> 3;
+    const uint32_t lds_all =
         __builtin_amdgcn_readfirstlane((uint32_t) (uintptr_t) (__attribute__((address_space(3))) uint8_t *) tiles);
+    const uint32_t lds0 = lds_all + group * LDS;
 
     // ---- copy sources. Activations as in matmul2.hip: instruction i of wave w fills region R = 4 w + i.
     const uint16_t *xsrc[4];
@@ -102,10 +106,12 @@ __device__ __forceinline__ void mm2k_body(const MatmulArgs &a) {
 #pragma unroll
             for (int j = 0; j < 16; ++j) acc[tt][rt][j] = 0.f;
 
-    copy_hdr(0u, 0u);
-    copy_pair(0u, 0u);
-    copy_act(0u, 0u);
-    copy_act(min(1u, nb - 1u), MM2_ACT);
+    if (KS == 1 || nsb > 0u) {  // (the last k-slice may leave group 1 without a super-block)
+        copy_hdr(0u, 0u);
+        copy_pair(0u, 0u);
+        copy_act(0u, 0u);
+        copy_act(1u, MM2_ACT);
+    }
     uint32_t bufo = 0u;              // k-block b's activation buffer, b % 3, as an offset
     for (uint32_t sb = 0; sb < nsb; ++sb) {
         const uint32_t hpar = sb & 1u;
@@ -211,8 +217,16 @@ __device__ __forceinline__ void mm2k_body(const MatmulArgs &a) {
             bufo = bufo == 2u * MM2_ACT ? 0u : bufo + MM2_ACT;
         }
     }
+    if constexpr (KS == 2)
+        for (uint32_t i = nb; i < span.most; ++i) __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_s_waitcnt(mm2_vmcnt(0));  // no copy outlives the work-group
-    mm2_store(a, sg, acc, t0, r0 + 64u * (wave >> 1) + n, 64u * (wave & 1u) + 4u * h);
+    const uint32_t r = r0 + 64u * (wave >> 1) + n, tl = 64u * (wave & 1u) + 4u * h;
+    if constexpr (KS == 2) {
+        mm2_store_halves(a, sg, acc, group, wave, lane, lds_all, t0, r, tl);
+    } else {
+        mm2_store(a, sg, acc[0][0], acc[1][0], t0, r, tl);
+        mm2_store(a, sg, acc[0][1], acc[1][1], t0, r + 32u, tl);
+    }
 }
 
 }  // namespace
@@ -221,6 +235,10 @@ extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_pe
 moearc_matmul2_q4_k_k(MatmulArgs a) { mm2k_body<12>(a); }
 extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 moearc_matmul2_q5_k_k(MatmulArgs a) { mm2k_body<13>(a); }
+extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+moearc_matmul2x_q4_k_k(MatmulArgs a) { mm2k_body<12, 2>(a); }
+extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+moearc_matmul2x_q5_k_k(MatmulArgs a) { mm2k_body<13, 2>(a); }
 
 // The f16 hi / lo split of x (as moearc_split_f16_k) and, in the same pass, each super-block's eight
 // 32-wide sums as two f16 pieces for the mins' MFMA: piece 0 f16(v), piece 1 f16((v - f32(piece 0)) *

@@ -93,6 +93,7 @@ struct moearc_ctx {
     hipFunction_t f_mm_small[6][4] = {};  // the same formats x 16 / 32 / 48 / 64 tokens, from f32 activations
     unsigned long mm_small = 64;  // MOEARC_MM_SMALL: most tokens that run on them (0: none)
     hipFunction_t f_mm2[6] = {};  // Q8_0, F16, Q4_K, Q5_K, Q6_K, MXFP4: 128 x 128 tiles on the 32x32x16 MFMA
+    hipFunction_t f_mm2x[6] = {};  // the same, eight waves, each four on half of the reduction
     hipFunction_t f_mm2w[3] = {};  // Q8_0, F16, MXFP4 on 128 tokens x 256 rows, eight waves
     uint16_t *mm_ws = nullptr;  // f16 hi / lo split of a chunk's activations
     size_t mm_ws_halves = 0;
@@ -700,6 +701,12 @@ moearc_ctx *moearc_ctx_create(void) {
         {&c->f_mm2[3], "moearc_matmul2_q5_k_k"},
         {&c->f_mm2[4], "moearc_matmul2_q6_k_k"},
         {&c->f_mm2[5], "moearc_matmul2_mxfp4_k"},
+        {&c->f_mm2x[0], "moearc_matmul2x_q8_0_k"},
+        {&c->f_mm2x[1], "moearc_matmul2x_f16_k"},
+        {&c->f_mm2x[2], "moearc_matmul2x_q4_k_k"},
+        {&c->f_mm2x[3], "moearc_matmul2x_q5_k_k"},
+        {&c->f_mm2x[4], "moearc_matmul2x_q6_k_k"},
+        {&c->f_mm2x[5], "moearc_matmul2x_mxfp4_k"},
         {&c->f_mm2w[0], "moearc_matmul2w_q8_0_k"},
         {&c->f_mm2w[1], "moearc_matmul2w_f16_k"},
         {&c->f_mm2w[2], "moearc_matmul2w_mxfp4_k"},
@@ -1735,7 +1742,18 @@ int mm_launch(moearc_ctx *c, unsigned ty, const MmMat *m, unsigned n_mat, const 
     uint64_t slices = 1, kb_per = nb;
     const uint64_t aim = c->mm_split_wg >= 0 ? (uint64_t) c->mm_split_wg : (gy <= 2 || wide) ? 1 : 2;
     if (tiles <= kMmCUs && nb >= 8 && aim) {
-        const uint64_t want = std::max<uint64_t>(1, std::min<uint64_t>(aim * kMmCUs / tiles, nb / 4));
+        uint64_t want = std::max<uint64_t>(1, std::min<uint64_t>(aim * kMmCUs / tiles, nb / 4));
+        // Tiles that fill three quarters of the CUs or more by themselves are not sliced: eight waves to
+        // a work-group keep two per SIMD, the two fours halve the reduction between them and meet in LDS, and
+        // there are no partial sums to write, read and add (1000 x 4096 x 2048 Q4_K, 256 tiles: 67 -> 60.5 us,
+        // 1000 x 4096 x 2880 Q8_0 77.4 -> 72.5 and F16 75 -> 69, 900 MXFP4 86 -> 80; 192 tiles 66.1 -> 65.3;
+        // 160 tiles lose, 48.2 -> 55 and, Q6_K, 65 -> 77). Two slices of such halves tie with four of four
+        // waves (128 tiles: 48.5 against 49.9, 44.6 against 45.0, 39.5 against 39.4).
+        if (mm2 && !wide && c->mm_split_wg < 0 && tiles >= kMmCUs * 3 / 4 && nb >= 2 * gran) {
+            want = 1;
+            f = c->f_mm2x[mm2_i];
+            threads = 512;
+        }
         kb_per = (nb + want - 1) / want;
         kb_per = (kb_per + gran - 1) / gran * gran;
         slices = (nb + kb_per - 1) / kb_per;
