@@ -429,7 +429,8 @@ __device__ __forceinline__ void store_out(void *out, uint32_t out_f16, uint64_t 
     else ((float *) out)[o] = r;
 }
 
-// The split kernel. Geometry words: geo0 = pt_shift | n_kv_heads << 16, geo1 = nkb | group << 16,
+// The split kernel. Geometry words: geo0 = pt_shift | MOEARC_DECODE_UNIFORM if
+// every sequence has the same number of items | n_kv_heads << 16, geo1 = nkb | group << 16,
 // nkb being the KV-head blocks (of KB heads) per work item.
 template <class P, int KB, int WPK, int TILES>
 __device__ __forceinline__ void decode_body(const typename P::Elem *k_pages, const typename P::Elem *v_pages,
@@ -449,28 +450,40 @@ __device__ __forceinline__ void decode_body(const typename P::Elem *k_pages, con
 
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t sh = geo0 & 0xFFFFu, G = geo0 >> 16;
+    const uint32_t sh = geo0 & (MOEARC_DECODE_UNIFORM - 1u), G = geo0 >> 16;
     const uint32_t nkb = geo1 & 0xFFFFu, group = geo1 >> 16;
     const uint32_t kbi = blockIdx.x % nkb;
     const uint32_t item = blockIdx.x / nkb;
     // Sequence 0 comes from the preloaded arguments; later sequences search the struct.
-    uint32_t b = 0, ib = 0, next = next0, kvb = kvb0, nkv = nkv0, slen = slen0;
+    uint32_t b = 0, ib = 0, next = next0, kvb = kvb0, nkv = nkv0;
     const uint32_t *bt = bt0;
     const float *qb = q0;
     if (item >= next) {
-        do ++b; while (item >= a.item_begin[b + 1]);
-        ib = a.item_begin[b];
-        next = a.item_begin[b + 1];
-        kvb = a.kv_begin[b];
-        nkv = a.n_kv[b];
-        slen = a.split_len[b];
+        // Where every sequence has as many splits as sequence 0 (windows: one), the item's number gives
+        // the sequence; else a walk along item_begin, 40 ns per sequence of a chain that ends in the first
+        // loads: 32 windows of 128 keys 6.07 -> 4.90 us, 24 at 128 channels 8.08 -> 7.43. (A lane per
+        // sequence and a ballot, one vector round trip, lost up to 1.1 us to the walk at 2-24 ragged
+        // sequences of 128 channels.)
+        if (geo0 & MOEARC_DECODE_UNIFORM) {
+            b = next0 == 1u ? item : item / next0;
+            ib = b * next0;
+            next = ib + next0;
+            kvb = a.kv_begin[b];
+            nkv = a.n_kv[b];
+        } else {
+            do ++b; while (item >= a.item_begin[b + 1]);
+            ib = a.item_begin[b];
+            next = a.item_begin[b + 1];
+            kvb = a.kv_begin[b];
+            nkv = a.n_kv[b];
+        }
         bt = a.block_tables + (uint64_t) b * a.bt_stride;
         qb = a.q + (uint64_t) b * G * group * D;
     }
     const uint32_t split = item - ib;
     const uint32_t nsplit = next - ib;
-    const uint32_t tb = kvb + split * slen;
-    const uint32_t te = min(nkv, tb + slen);
+    const uint32_t tb = kvb + split * slen0;
+    const uint32_t te = min(nkv, tb + slen0);
     const uint32_t kl = wave % KB, sub = wave / KB;
     const uint32_t kvh_raw = kbi * KB + kl;
     const bool kvh_ok = kvh_raw < G;

@@ -25,6 +25,10 @@
 // most 128).
 #define MOEARC_DECODE_SCRATCH_FLOATS (1u << 21)
 
+// Set in the split kernel's geometry word geo0 (above the page shift, at most 30) when every sequence
+// of the launch has as many work items as sequence 0.
+#define MOEARC_DECODE_UNIFORM 0x8000u
+
 // Kernel arguments of the split-K decode that are not preloaded scalars (the leading kernel
 // arguments carry the KV and block-table bases, q, sequence 0's span, split and item count, and
 // the geometry). Passed by value; the per-sequence arrays let one launch serve a ragged batch.
@@ -47,7 +51,6 @@ struct DecodeArgs {
                                                          // n_seqs .. the end: the work-item count
     uint32_t kv_begin[MOEARC_MAX_SEQS_PER_LAUNCH];       // key span [kv_begin, n_kv)
     uint32_t n_kv[MOEARC_MAX_SEQS_PER_LAUNCH];
-    uint32_t split_len[MOEARC_MAX_SEQS_PER_LAUNCH];      // keys per split (a multiple of the chunk)
 };
 
 // The merge kernel's per-sequence item ranges (sequence 0's end is a preloaded argument). One

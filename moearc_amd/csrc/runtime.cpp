@@ -544,14 +544,15 @@ int decode_launch_body(moearc_ctx *c, void *out, unsigned int out_f16, const flo
         a.scale_log2e = scale * 1.4426950408889634f;
         a.n_seqs = (uint32_t) cnt;
         uint32_t items = 0;
+        bool uniform = true;  // as many splits in every sequence
         for (size_t i = 0; i < cnt; ++i) {
             a.item_begin[i] = items;
             a.kv_begin[i] = sub[i].begin;
             a.n_kv[i] = sub[i].end;
-            a.split_len[i] = split_len;
             const uint64_t n_split = (sub[i].end - sub[i].begin + (uint64_t) split_len - 1) / split_len;
             if (items + n_split > 0x7FFFFFFFull) return ERR_ARG;
             items += (uint32_t) n_split;
+            uniform = uniform && items == (i + 1) * (uint64_t) n_split;
         }
         for (size_t i = cnt; i <= MOEARC_MAX_SEQS_PER_LAUNCH; ++i) a.item_begin[i] = items;
         const size_t wgs = (size_t) items * nkb;
@@ -576,9 +577,9 @@ int decode_launch_body(moearc_ctx *c, void *out, unsigned int out_f16, const flo
         L.q0 = qb;
         L.kvb0 = a.kv_begin[0];
         L.nkv0 = a.n_kv[0];
-        L.slen0 = a.split_len[0];
+        L.slen0 = split_len;
         L.next0 = a.item_begin[1];
-        L.geo0 = log2u(page_tokens) | (uint32_t) n_kv_heads << 16;
+        L.geo0 = log2u(page_tokens) | (uniform ? MOEARC_DECODE_UNIFORM : 0u) | (uint32_t) n_kv_heads << 16;
         L.geo1 = (uint32_t) nkb | (uint32_t) (n_heads / n_kv_heads) << 16;
         const int rc = launch(c, c->f_dec_fast[kind][variant], (unsigned) wgs, 64u * dv.kb * dv.wpk, L,
                               "attn_decode.split", n_heads, head_dim);
