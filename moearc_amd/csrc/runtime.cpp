@@ -124,13 +124,17 @@ struct moearc_ctx {
     std::vector<Pending> pending;
     std::vector<KernelTime> totals;
     std::vector<hipEvent_t> event_pool;
-    // a split prefill's records (eager calls only: captured ones use the fixed array, so no graph
-    // holds an address that a later call may replace)
+    // a split prefill's records (eager calls only: captured ones are not split, so no graph holds an
+    // address that a later call may replace or that a graph on another stream shares)
     float *pf_ws = nullptr;
     size_t pf_ws_floats = 0;
     // split-K workspace: the partial records of the split kernel (per query head and work item)
     float *ws = nullptr;
     size_t ws_floats = 0;
+    // the same for the 128-channel and f32 caches, eager calls only: their growth leaves the address
+    // alone that a captured 64-channel f16 call may hold
+    float *ws_kinds = nullptr;
+    size_t ws_kinds_floats = 0;
     int decode_variant_override = -1;  // MOEARC_DECODE_VARIANT, e.g. "4x2x4"
     unsigned long split_override = 0;  // MOEARC_DECODE_SPLIT (keys per split)
     float *blk_ws = nullptr;  // attention-block chunk: q, k, v, f16 q, attention output, projection
@@ -268,8 +272,6 @@ int ensure_floats(moearc_ctx *c, float *&ws, size_t &have, size_t floats) {
     have = floats;
     return OK;
 }
-
-int ensure_workspace(moearc_ctx *c, size_t floats) { return ensure_floats(c, c->ws, c->ws_floats, floats); }
 
 bool capturing(moearc_ctx *c) {
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
@@ -450,12 +452,14 @@ int decode_launch(moearc_ctx *c, void *out, unsigned int out_f16, const float *q
     // anything is enqueued, so a refusal leaves the stream untouched.
     const DecodeKind kind =
         decode_kind(out, q, k_pages, v_pages, n_heads, n_kv_heads, head_dim, page_tokens, kv_type, scale);
-    // Under stream capture the kinds that the general kernel used to serve keep their records in the
-    // context's fixed array: that kernel needed no memory, so a captured call of theirs must neither
-    // allocate nor leave a graph with the address of a workspace that a later call may replace.
+    // Under stream capture the kinds that the general kernel used to serve keep no records (one split
+    // per sequence): that kernel needed no memory, so a captured call of theirs must neither allocate,
+    // nor leave a graph with the address of a workspace that a later call may replace, nor share memory
+    // with a graph that another stream replays at the same time. A program that captures long spans of
+    // these kinds takes the allocation-free entry point, whose array one stream owns.
     if (!rs.fixed && kind != kGeneral && kind != kF16D64 && capturing(c)) {
         rs.fixed = c->scratch;
-        rs.cap = c->scratch_floats;
+        rs.cap = 0;
     }
     if (rs.fixed && kind != kGeneral) {
         SeqSpan sub[MOEARC_MAX_SEQS_PER_LAUNCH];
@@ -564,8 +568,9 @@ int decode_launch_body(moearc_ctx *c, void *out, unsigned int out_f16, const flo
             if (ws) {
                 if (rec * rec_floats > rs.cap) return ERR_ARG;  // checked for every group before the first launch
             } else {
-                if (ensure_workspace(c, rec * rec_floats)) return ERR;
-                ws = c->ws;
+                float *&own = kind == kF16D64 ? c->ws : c->ws_kinds;
+                if (ensure_floats(c, own, kind == kF16D64 ? c->ws_floats : c->ws_kinds_floats, rec * rec_floats)) return ERR;
+                ws = own;
             }
             a.rec_o = ws;
             a.rec_ml = ws + rec * head_dim;
@@ -614,7 +619,7 @@ moearc_ctx *release(moearc_ctx *c) {
         (void) hipEventDestroy(p.stop);
     }
     for (auto e : c->event_pool) (void) hipEventDestroy(e);
-    for (void *p : {(void *) c->ws, (void *) c->pf_ws, (void *) c->blk_ws, (void *) c->mm_ws, (void *) c->mm_part,
+    for (void *p : {(void *) c->ws, (void *) c->ws_kinds, (void *) c->pf_ws, (void *) c->blk_ws, (void *) c->mm_ws, (void *) c->mm_part,
                     (void *) c->err_word})
         if (p) (void) hipFree(p);
     if (c->module) (void) hipModuleUnload(c->module);
@@ -1413,8 +1418,7 @@ struct PrefillPlan {
 // 516 chunks; 2048 behind 2048, 512: 107 µs for 193 per CU); every piece writes and reads 66 KB of
 // records, about PF_PIECE of the whole device, and the merge is a launch more (PF_MERGE). Candidates
 // are the shortest pieces for which the launch has at most 64, 128, 256 or 512 work-groups.
-// `max_records`: pieces x KV heads that the record space holds.
-void plan_prefill(const PrefillArgs &a, uint32_t tile_tokens, uint32_t n_cu, uint64_t max_records, PrefillPlan &plan) {
+void plan_prefill(const PrefillArgs &a, uint32_t tile_tokens, uint32_t n_cu, PrefillPlan &plan) {
     constexpr float PF_CHUNK1 = 0.59f, PF_CHUNK2 = 1.10f, PF_PIECE = 0.033f, PF_MERGE = 5.f;
     const uint32_t T = a.n_qtiles, G = a.n_kv_heads;
     if (!n_cu || T > MOEARC_PF_MAX_TILES || (uint64_t) T * G >= 2ull * n_cu) return;
@@ -1444,7 +1448,7 @@ void plan_prefill(const PrefillArgs &a, uint32_t tile_tokens, uint32_t n_cu, uin
             else lo = mid + 1;
         }
         const uint64_t n = pieces_at(lo) * G;
-        if (n > wgs || n > max_records) continue;
+        if (n > wgs) continue;
         const float t = (n <= n_cu ? PF_CHUNK1 : PF_CHUNK2) * lo + PF_MERGE + PF_PIECE * n;
         if (t < best) {
             best = t;
@@ -1510,17 +1514,14 @@ int prefill_launch(moearc_ctx *c, void *out, unsigned int out_type, uint16_t *ou
     a.boost_b = c->pf_boost_b;
     if (wgs > 0x7FFFFFFFull) return ERR_ARG;
     PrefillPlan plan;
-    const bool fixed = !precise && capturing(c);
-    if (!precise)
-        plan_prefill(a, rows_per_tile / (uint32_t) group, c->n_cu,
-                     fixed ? c->scratch_floats / MOEARC_PF_RECORD_FLOATS : ~0ull, plan);
+    if (!precise && !capturing(c)) plan_prefill(a, rows_per_tile / (uint32_t) group, c->n_cu, plan);
     if (plan.items) {
         const uint64_t n = (uint64_t) plan.items * n_kv_heads;
         PrefillSplitArgs s{};
         a.pair_half = n > c->n_cu ? c->n_cu : 0u;
         s.a = a;
-        if (!fixed && ensure_floats(c, c->pf_ws, c->pf_ws_floats, n * MOEARC_PF_RECORD_FLOATS)) return ERR;
-        s.rec_o = fixed ? c->scratch : c->pf_ws;
+        if (ensure_floats(c, c->pf_ws, c->pf_ws_floats, n * MOEARC_PF_RECORD_FLOATS)) return ERR;
+        s.rec_o = c->pf_ws;
         s.rec_ml = s.rec_o + n * MOEARC_PREFILL_FAST_ROWS * 64u;
         s.n_items = plan.items;
         s.tile_tokens = rows_per_tile / (uint32_t) group;

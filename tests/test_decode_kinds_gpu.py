@@ -140,7 +140,8 @@ def test_records_past_the_fixed_array_widen_the_splits(monkeypatch):
 @pytest.mark.parametrize("kv,D", KINDS)
 def test_capture_needs_no_memory(kv, D):
     # the first call on a context is a captured one; the graph then replays beside the context's own
-    # eager calls, whose larger batch makes the workspace grow
+    # eager calls, whose larger batch makes the workspace grow; it is one launch without records, so
+    # graphs on several streams share nothing
     hip = ctypes.CDLL("libamdhip64.so")
     B, big = Batch(11, kv, D, [3000], 256, 4, 8), Batch(12, kv, D, [9000, 9000, 9000], 256, 4, 8)
     with Context() as cx:
@@ -150,6 +151,8 @@ def test_capture_needs_no_memory(kv, D):
         assert hip.hipStreamBeginCapture(stream, 1) == 0
         cx.attn_decode_ext(out, q, k, v, bt, s, B.H, B.G, D, 0, 3000, 256, B.scale, B.type)
         assert hip.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+        nodes = ctypes.c_size_t()
+        assert hip.hipGraphGetNodes(graph, None, ctypes.byref(nodes)) == 0 and nodes.value == 1
         assert hip.hipGraphInstantiate(ctypes.byref(exe), graph, None, None, ctypes.c_size_t(0)) == 0
         bigger = big.upload(cx)
         for _ in range(3):

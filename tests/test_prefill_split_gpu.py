@@ -80,7 +80,8 @@ def test_profile_counts_a_split_prefill_once(monkeypatch):
 
 
 def test_capture_needs_no_memory():
-    # a captured call on a fresh context, replayed beside eager calls that grow the workspace
+    # a captured call on a fresh context, replayed beside eager calls that grow the workspace; it is
+    # one launch without records, so graphs on several streams share nothing
     hip = ctypes.CDLL("libamdhip64.so")
     pc, big = (fx.prefill_case(s, n_q=n, pos0=4000, pt=256, H=16, G=2) for s, n in ((0x5BB, 40), (0x5BC, 200)))
     with Context() as cx:
@@ -90,6 +91,8 @@ def test_capture_needs_no_memory():
         assert hip.hipStreamBeginCapture(stream, 1) == 0
         cx.attn_prefill(out, *bufs, pc.n_q, pc.pos0, 0, 16, 2, 64, 256, 0.125, KvType.F16)
         assert hip.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+        nodes = ctypes.c_size_t()
+        assert hip.hipGraphGetNodes(graph, None, ctypes.byref(nodes)) == 0 and nodes.value == 1
         assert hip.hipGraphInstantiate(ctypes.byref(exe), graph, None, None, ctypes.c_size_t(0)) == 0
         want, want_big = _want(pc, 0), _want(big, 0)
         for _ in range(3):
