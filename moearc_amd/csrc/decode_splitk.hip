@@ -430,7 +430,7 @@ __device__ __forceinline__ void store_out(void *out, uint32_t out_f16, uint64_t 
 }
 
 // The split kernel. Geometry words: geo0 = pt_shift | MOEARC_DECODE_UNIFORM if
-// every sequence has the same number of items | n_kv_heads << 16, geo1 = nkb | group << 16,
+// every sequence has the same number of items | MOEARC_DECODE_MANY past 24 sequences | n_kv_heads << 16, geo1 = nkb | group << 16,
 // nkb being the KV-head blocks (of KB heads) per work item.
 template <class P, int KB, int WPK, int TILES>
 __device__ __forceinline__ void decode_body(const typename P::Elem *k_pages, const typename P::Elem *v_pages,
@@ -450,7 +450,7 @@ __device__ __forceinline__ void decode_body(const typename P::Elem *k_pages, con
 
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t sh = geo0 & (MOEARC_DECODE_UNIFORM - 1u), G = geo0 >> 16;
+    const uint32_t sh = geo0 & (MOEARC_DECODE_MANY - 1u), G = geo0 >> 16;
     const uint32_t nkb = geo1 & 0xFFFFu, group = geo1 >> 16;
     const uint32_t kbi = blockIdx.x % nkb;
     const uint32_t item = blockIdx.x / nkb;
@@ -471,7 +471,20 @@ __device__ __forceinline__ void decode_body(const typename P::Elem *k_pages, con
             kvb = a.kv_begin[b];
             nkv = a.n_kv[b];
         } else {
-            do ++b; while (item >= a.item_begin[b + 1]);
+            if (geo0 & MOEARC_DECODE_MANY) {
+                // Past 24 sequences the walk's length outweighs two trips to the scalar cache, eight entries
+                // each: every eighth, then the group's. 32 sequences of 200-2000 keys (graph replay)
+                // 27.5 -> 26.5 us, 60: 37.4 -> 36.5; 8 and 17 lost 0.5-1% to the walk.
+                static_assert(MOEARC_MAX_SEQS_PER_LAUNCH == 64, "eight groups of eight sequences");
+                uint32_t g = 0;
+#pragma unroll
+                for (uint32_t i = 1; i < 8u; ++i) g += item >= a.item_begin[8u * i];
+                b = 8u * g;
+#pragma unroll
+                for (uint32_t i = 1; i < 8u; ++i) b += item >= a.item_begin[8u * g + i];
+            } else {
+                do ++b; while (item >= a.item_begin[b + 1]);
+            }
             ib = a.item_begin[b];
             next = a.item_begin[b + 1];
             kvb = a.kv_begin[b];

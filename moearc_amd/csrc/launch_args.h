@@ -28,6 +28,8 @@
 // Set in the split kernel's geometry word geo0 (above the page shift, at most 30) when every sequence
 // of the launch has as many work items as sequence 0.
 #define MOEARC_DECODE_UNIFORM 0x8000u
+// Set there when the launch has more than 24 sequences.
+#define MOEARC_DECODE_MANY 0x4000u
 
 // Kernel arguments of the split-K decode that are not preloaded scalars (the leading kernel
 // arguments carry the KV and block-table bases, q, sequence 0's span, split and item count, and

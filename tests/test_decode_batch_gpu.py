@@ -13,6 +13,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("n_seqs,lens", [(5, "window"), (64, "window"), (66, "window"), (16, "ragged"), (17, "ragged"),
+                                         (24, "ragged"), (25, "ragged"),
                                          (64, "ragged"), (70, "ragged"), (24, "equal"), (3, "equal")])
 @pytest.mark.parametrize("heads,kv_heads,dim", [(16, 2, 64), (8, 1, 128)])
 def test_each_sequence_as_alone(ctx, heads, kv_heads, dim, n_seqs, lens):
