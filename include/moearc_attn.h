@@ -255,7 +255,8 @@ int moearc_attn_qkv(moearc_ctx *c, const unsigned int *type_ids, float *const *o
 
 /* Extension (no counterpart in the reference, which runs one moearc_matvec_q per token): the
  * projections of a prompt chunk as one MFMA matrix product, y[t][r] = sum_c W[r][c] x[t][c]
- * (+ bias[r]) for t < n_tok, r < n_rows; x f32 [n_tok][n_cols], y f32 [n_tok][n_rows]. Weights
+ * (+ bias[r]) for t < n_tok, r < n_rows; x f32 [n_tok][n_cols], y f32 [n_tok][n_rows] (y may overlap
+ * x, which is then read before any of y is written). Weights
  * Q8_0 (8), F16 (1), Q4_K (12), Q5_K (13), Q6_K (14) or MXFP4 (39), W 2-byte aligned. x enters as an f16
  * hi + lo pair (to 2^-22 relative; each |x| must stay below 65504), quantised payloads as exact
  * f16 integers / E2M1 values, block scales (and K-quant mins, against f32 block sums of x) in f32:

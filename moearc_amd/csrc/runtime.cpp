@@ -1868,7 +1868,10 @@ int moearc_matmul_q(moearc_ctx *c, unsigned int type_id, float *y, const void *w
     if (const int rc = mm_check(type_id, w, n_tok, n_rows, n_cols)) return rc;
     if (n_rows == 0 || n_tok == 0) return OK;
     const MmMat mat{w, bias, y, n_rows, n_rows};
-    if (mm_takes_f32(c, n_tok, n_cols, (n_rows + 15) / 16)) return mm_small_launch(c, type_id, &mat, 1, x, n_tok, n_cols, "matmul");
+    // y over x: rows may be written only once x is in the workspace (the one launch reads x throughout)
+    const bool apart = (uintptr_t) (y + n_tok * n_rows) <= (uintptr_t) x || (uintptr_t) (x + n_tok * n_cols) <= (uintptr_t) y;
+    if (apart && mm_takes_f32(c, n_tok, n_cols, (n_rows + 15) / 16))
+        return mm_small_launch(c, type_id, &mat, 1, x, n_tok, n_cols, "matmul");
     uint16_t *xh, *xl;
     float *xs;
     if (const int rc = mm_split(c, x, n_tok * n_cols, &xh, &xl, &xs, mm_needs_sums(type_id), n_tok)) return rc;

@@ -1,0 +1,43 @@
+"""Which kernels the entry points launch, and what memory they take for it, on the host alone (host_hip.py)."""
+from __future__ import annotations
+
+import pytest
+
+import host_hip
+from host_hip import at, names
+from moearc_amd import Context, QuantType, native
+
+MM = [QuantType.F16, QuantType.Q8_0, QuantType.MXFP4, QuantType.Q4_K, QuantType.Q5_K, QuantType.Q6_K]
+
+
+@pytest.fixture(scope="module")
+def built(tmp_path_factory):
+    return host_hip.build(tmp_path_factory.mktemp("host"))
+
+
+@pytest.fixture
+def lib(built, monkeypatch):
+    monkeypatch.setattr(native, "_lib", built)
+    built.host_hip_reset()
+    yield built
+    built.host_hip_reset()
+
+
+@pytest.mark.parametrize("n_tok", [1, 2, 17, 32, 33, 64])
+@pytest.mark.parametrize("ty", MM, ids=lambda t: t.name)
+def test_a_product_over_its_own_input_reads_it_first(lib, ty, n_tok):
+    # y may overlap x: the activations are then split into the workspace before any row is written; the
+    # one-launch form, whose work-groups read x while others write y, is for buffers apart
+    n, size = 512, 64 * 512 * 4
+    with Context() as cx:
+        def call(y, x):
+            lib.host_hip_reset()
+            cx.matmul_q(ty, at(cx, y, size), at(cx, 1 << 33, ty.row_bytes(n) * n), at(cx, x, size), None, n_tok, n, n)
+            return names(lib)
+        x = 1 << 32
+        used = n_tok * n * 4
+        for y in (x - used, x + used):
+            assert [k.rsplit("_t", 1)[0] for k in call(y, x)] == [f"moearc_matmul_small_{ty.name.lower()}"]
+        for y in (x, x + 4, x - 4, x + used - 4, x - used + 4):
+            got = call(y, x)
+            assert any(k.startswith("moearc_split") for k in got) and not any("small" in k for k in got), got

@@ -62,6 +62,23 @@ def test_unaligned_buffers(ctx, ty):
     _check(ctx, ty, 18, 40, 768, w_off=2, x_off=4)
 
 
+@pytest.mark.parametrize("n_tok,shift", [(2, 0), (17, 0), (32, 512), (64, -1024)])
+@pytest.mark.parametrize("ty", BLOCKS + SUPER, ids=lambda t: t.name)
+def test_over_its_own_input(ctx, ty, n_tok, shift):
+    # y on x, and y starting a row after x or two rows before it (shift floats)
+    n = 512
+    w, _ = fx.synth_blocks(int(ty), n * n // ty.block_elems, 0x3C8)
+    x = fx.synth.unit(0x3C9, n_tok * n).reshape(n_tok, n)
+    at_x, at_y = max(0, -shift), max(0, shift)
+    raw = ctx.upload(np.concatenate([np.zeros(at_x, np.float32), x.reshape(-1), np.zeros(at_y, np.float32)]))
+    ctx.matmul_q(ty, DeviceView(raw, 4 * at_y), ctx.upload(w), DeviceView(raw, 4 * at_x), None, n_tok, n, n)
+    got = ctx.download(raw, np.float32, n_tok * n + abs(shift))[at_y:at_y + n_tok * n].reshape(n_tok, n)
+    for t in range(n_tok):
+        want, absum = oracle.matvec_q(int(ty), w, x[t], n, n, n_threads=8)
+        tol = fx.matvec_tolerance(n, absum) + 2.0 * 64 * 2.0 ** -24 * absum
+        assert np.all(np.abs(got[t] - want) <= tol)
+
+
 def test_same_product_in_any_chunk_of_a_tile(ctx):
     # a token's result does not depend on its neighbours: rows of a 32-token product equal those of a
     # 7-token one (one or two token tiles, the same reduction)
