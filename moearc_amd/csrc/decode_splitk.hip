@@ -38,8 +38,8 @@
 //
 // The 128-channel and f32 kinds took the general kernel (decode_general.hip) before, a work-group per
 // query head with neither splits nor a shared KV read: four sequences of 2K-8K keys at 32 heads over
-// 4 KV heads of 128 f16 channels (34 MB) went from 2360 to 15.3 µs, 17 of 2K-30K reach 4.8 TB/s
-// (114.6 µs, a large copy's rate), eight of 3K-30K over f32 caches 5.2-5.4 TB/s (106.6 and 112 µs).
+// 4 KV heads of 128 f16 channels (34 MB) went from 2360 to 14.8 µs, 17 of 2K-30K reach 4.8 TB/s
+// (123 µs, a large copy's rate), eight of 3K-30K over f32 caches 5.2-5.4 TB/s (106.6 and 112 µs).
 // Their error against float64 is a quarter of that kernel's (2.8e-7 against 1.2e-6).
 //
 // Kernel arguments: the fields the first loads depend on (KV and block-table bases, q, sequence
@@ -67,6 +67,12 @@ __device__ __forceinline__ float wave_max_16_32(float x) {
     x = fmaxf(x, __shfl_xor(x, 16));
     x = fmaxf(x, __shfl_xor(x, 32));
     return x;
+}
+
+// the value of the lane that DPP control CTRL names, within its 16 lanes
+template <int CTRL>
+__device__ __forceinline__ float dpp(float x) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xF, 0xF, false));
 }
 
 __device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
@@ -116,16 +122,16 @@ __device__ __forceinline__ void softmax_tile(SoftmaxState<NO> &st, float4_t (&S)
     st.l += psum;
 }
 
-// q as two f16 operands per 32 channels, q = (hi + lo) 2^(qexp - 1), and the score multiplier with
-// the power of two folded in: each head's q is normalised by a power of two (exact) so that the
-// split keeps full relative precision whatever q's magnitude.
+// A head's q, normalised by a power of two (exact) so that a split into f16 pieces does not depend on
+// the head's magnitude, and the score multiplier with that power folded in.
 template <int NQ>
 struct SplitQuery {
-    half8_t hi[NQ], lo[NQ];
     float c;
     float v[8 * NQ];
     // lane (g, n): channels 32 i + 8 g .. + 7 of head n, 0 for columns past the group
-    __device__ __forceinline__ void load(const float *qrow, uint32_t g, bool head_ok) {
+    __device__ __forceinline__ void load(const float *q, uint32_t group, uint32_t dim, uint32_t g, uint32_t n) {
+        const bool head_ok = n < group;
+        const float *const qrow = q + (head_ok ? n : 0u) * dim;
 #pragma unroll
         for (int i = 0; i < NQ; ++i) {
             const float4_t x0 = *(const float4_t *) (qrow + 32 * i + 8 * g);
@@ -137,38 +143,42 @@ struct SplitQuery {
             }
         }
     }
-    __device__ __forceinline__ void ready(float scale_log2e) {
+    // qexp and c for q 2^(top - qexp), whose largest channel is in [2^(top - 1), 2^top)
+    __device__ __forceinline__ int normalise(float scale_log2e, int top) {
         float amax = 0.f;
 #pragma unroll
         for (int i = 0; i < 8 * NQ; ++i) amax = fmaxf(amax, fabsf(v[i]));
         amax = wave_max_16_32(amax);
         int qexp = 0;
         if (amax > 0.f && amax < INFINITY) (void) frexpf(amax, &qexp);
-        c = ldexpf(scale_log2e, qexp - 1);  // score multiplier in the log2 domain
-#pragma unroll
-        for (int i = 0; i < NQ; ++i)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float x = ldexpf(v[8 * i + e], 1 - qexp);
-                const _Float16 h = (_Float16) x;
-                hi[i][e] = h;
-                lo[i][e] = (_Float16) (x - (float) h);
-            }
+        c = ldexpf(scale_log2e, qexp - top);  // score multiplier in the log2 domain
+        return qexp;
     }
 };
 
 // ---- f16 cache, 64 channels ----------------------------------------------------------------------
 struct F16D64 {
-    static constexpr int D = 64, NO = 4;
+    static constexpr int D = 64, NO = 4, Q_LDS = 0;
     using Elem = uint16_t;
     struct Tile {
         u32x4_t k[2][2];  // [key block][channel half], A-operand layout
         u32x4_t v[2][2];
     };
     struct Query : SplitQuery<2> {
+        // q = hi + lo: 22 bits of the channels down to 2^-3 of the head's largest, 2^-25 of it below
+        half8_t hi[2], lo[2];
         half8_t sel[2];  // selection operands: sel[s] lane (g, n) item i = 1 where 8g + i == 16s + n
-        __device__ __forceinline__ void ready(float scale_log2e, uint32_t g, uint32_t n) {
-            SplitQuery<2>::ready(scale_log2e);
+        __device__ __forceinline__ void ready(float scale_log2e, uint32_t g, uint32_t n, uint32_t *) {
+            const int qexp = normalise(scale_log2e, 1);
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float x = ldexpf(v[8 * i + e], 1 - qexp);
+                    const _Float16 h = (_Float16) x;
+                    hi[i][e] = h;
+                    lo[i][e] = (_Float16) (x - (float) h);
+                }
 #pragma unroll
             for (int s = 0; s < 2; ++s)
 #pragma unroll
@@ -242,21 +252,96 @@ __device__ __forceinline__ uint32_t v_row(const uint32_t (&row)[2], int blk, uin
 }
 
 // ---- f16 cache, 128 channels: HBM-bound like the 64-channel kind, 512 bytes per key and KV head.
-// Scores as there, q in two f16 operands per 32 channels. For P.V, lane (g, m) loads channels
+// Scores as there, but with q whole in three f16 operands per 32 channels, q = hi + mid / 2^11 +
+// lo / 2^22, each with sums of its own: f32's 24 bits for every channel down to 2^-38 of the head's
+// largest (the general kernel multiplies in f32; two pieces kept about 7 bits of a channel 2^18 below the
+// largest). FOLD, for groups of up to 8 heads: lo takes the idle columns 8 .. 15 of hi's product, so the
+// third piece costs neither an MFMA nor a register. (In f32 MFMAs instead, four sequences of 2K-8K keys
+// take 17.4 us for 15.7, and their 32-step chains err by 4.2e-7 for 2.5e-7.) For P.V, lane (g, m) loads channels
 // 8 m .. 8 m + 7 of key 16 blk + 4 g + r: a 16-lane group reads a whole 256-byte row, and element e
 // of the 16 lanes, widened to f32, is the A operand of a 16x16x4 f32 MFMA over keys {4 g + r} whose
 // B operand is the softmax register r as it stands: no transposition, weights in f32, at the price of
 // 4x the matrix time of the f16 product, which still leaves the matrix cores over half idle at the
 // HBM rate.
+typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+
+template <bool FOLD_>
 struct F16D128 {
-    static constexpr int D = 128, NO = 8;
+    static constexpr bool FOLD = FOLD_;
+    static constexpr int D = 128, NO = 8, Q_LDS = 256 * 4 * (FOLD ? 2 : 3) + 16;  // dwords: q's operands, the heads' c
     using Elem = uint16_t;
     struct Tile {
         u32x4_t k[2][4];  // [key block][channel quarter]
         u32x4_t v[2][4];  // [key block][r]: channels 8 m .. of key 4 g + r
     };
-    struct Query : SplitQuery<4> {
-        __device__ __forceinline__ void ready(float scale_log2e, uint32_t, uint32_t) { SplitQuery<4>::ready(scale_log2e); }
+    // The four waves work for one KV head and make its operands together: a thread takes 4 channels of one
+    // head, the 32 threads of a head share its largest channel, and the pieces meet in LDS. That is one
+    // coalesced load; in operand layout, eight per wave of 64 scattered pieces each, q's loads and the third
+    // piece's arithmetic in every wave cost more: four sequences of 2K-8K keys 15.9 us with the mid and low
+    // pieces in LDS, 17.9 with FOLD, 14.8 this way (15.4 with two pieces), eight of 200-2000 13.0 -> 12.6.
+    // At one query head per KV head, where the scattered load had one row to fetch, up to 2.5% longer.
+    struct Query {
+        static constexpr int ROUNDS = FOLD ? 1 : 2, PARTS = FOLD ? 2 : 3;  // heads / 8; hi (and lo), mid; or hi, mid, lo
+        float c;
+        float4_t raw[ROUNDS];
+        half8_t hi[4], mid[FOLD ? 4 : 1];
+        const half8_t *rest;  // !FOLD: mid and lo of 32 channels at [192 i], [192 i + 64], in LDS (registers would spill)
+        bool own;             // FOLD: a column of the heads' hi and mid
+        __device__ __forceinline__ void load(const float *q, uint32_t group, uint32_t, uint32_t, uint32_t) {
+#pragma unroll
+            for (int r = 0; r < ROUNDS; ++r) {
+                const uint32_t head = 8u * r + (threadIdx.x >> 5);
+                const float4_t x = *(const float4_t *) (q + min(head, group - 1u) * 128u + 4u * (threadIdx.x & 31u));
+                raw[r] = head < group ? x : (float4_t){0.f, 0.f, 0.f, 0.f};
+            }
+        }
+        __device__ __forceinline__ void ready(float scale_log2e, uint32_t g, uint32_t n, uint32_t *lds) {
+            half4_t *const parts = (half4_t *) lds;       // 8-byte halves of the operands' 16-byte slots
+            float *const c_of = (float *) (lds + Q_LDS - 16);
+            const uint32_t d8 = threadIdx.x & 31u;        // channels 4 d8 .. + 3: slot [d8 / 8][part][d8 / 2 % 4], half d8 % 2
+#pragma unroll
+            for (int r = 0; r < ROUNDS; ++r) {
+                const uint32_t head = 8u * r + (threadIdx.x >> 5);
+                float amax = fmaxf(fmaxf(fabsf(raw[r][0]), fabsf(raw[r][1])), fmaxf(fabsf(raw[r][2]), fabsf(raw[r][3])));
+                amax = fmaxf(amax, dpp<0xB1>(amax));   // quads: lanes 1 0 3 2, then 2 3 0 1
+                amax = fmaxf(amax, dpp<0x4E>(amax));
+                amax = fmaxf(amax, dpp<0x141>(amax));  // eight lanes mirrored, then sixteen
+                amax = fmaxf(amax, dpp<0x140>(amax));
+                amax = fmaxf(amax, __shfl_xor(amax, 16));
+                int qexp = 0;
+                if (amax > 0.f && amax < INFINITY) (void) frexpf(amax, &qexp);
+                if (d8 == 0u) c_of[head] = ldexpf(scale_log2e, qexp - 15);
+                half4_t h, m, l;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {  // below 65504; the remainders are exact in f32
+                    const float x = ldexpf(raw[r][e], 15 - qexp);
+                    h[e] = (_Float16) x;
+                    const float rem = (x - (float) h[e]) * 2048.f;
+                    m[e] = (_Float16) rem;
+                    l[e] = (_Float16) ((rem - (float) m[e]) * 2048.f);
+                }
+                const auto put = [&](uint32_t part, uint32_t column, const half4_t &v) {
+                    parts[2u * (64u * (PARTS * (d8 >> 3) + part) + 16u * ((d8 >> 1) & 3u) + column) + (d8 & 1u)] = v;
+                };
+                put(0u, head, h);
+                put(1u, head, m);
+                if constexpr (FOLD) put(0u, head + 8u, l);  // (mid's columns past 8 hold anything, and are dropped)
+                else put(2u, head, l);
+            }
+            // LDS alone is waited for: the first chunk's loads stay in flight
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+            const half8_t *const at = (const half8_t *) lds + (16u * g + n);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                hi[i] = at[64 * PARTS * i];
+                if constexpr (FOLD) mid[i] = at[64 * PARTS * i + 64];
+            }
+            rest = at + 64;
+            own = n < 8u;
+            c = c_of[FOLD ? n & 7u : n];
+        }
     };
     static __device__ __forceinline__ void load(Tile &r, const uint32_t (&row)[2], const Elem *k_pages,
                                                 const Elem *v_pages, uint64_t row_elems, uint32_t kvh, uint32_t g,
@@ -274,18 +359,27 @@ struct F16D128 {
     }
     static __device__ __forceinline__ void tile(SoftmaxState<NO> &st, Tile &r, const Query &q, uint32_t j0,
                                                 uint32_t te, uint32_t g, uint32_t) {
-        float4_t S[2];
+        float4_t S[2] = {}, t[2] = {}, u[2] = {};
 #pragma unroll
-        for (int blk = 0; blk < 2; ++blk) {
-            float4_t s = (float4_t){0.f, 0.f, 0.f, 0.f}, t = s;
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                s = mfma16(as_half8(r.k[blk][i]), q.hi[i], s);
-                t = mfma16(as_half8(r.k[blk][i]), q.lo[i], t);
+            for (int blk = 0; blk < 2; ++blk) {
+                const half8_t k = as_half8(r.k[blk][i]);
+                S[blk] = mfma16(k, q.hi[i], S[blk]);
+                if constexpr (FOLD) {
+                    t[blk] = mfma16(k, q.mid[i], t[blk]);
+                } else {
+                    t[blk] = mfma16(k, q.rest[192 * i], t[blk]);
+                    u[blk] = mfma16(k, q.rest[192 * i + 64], u[blk]);
+                }
             }
-            // an infinite key (f16 overflow at the append) scores by q.hi's sign alone
+        // an infinite key (f16 overflow at the append) scores by q.hi's sign alone
 #pragma unroll
-            for (int i = 0; i < 4; ++i) S[blk][i] = fabsf(s[i]) == INFINITY ? s[i] : s[i] + t[i];
+        for (int i = 0; i < 8; ++i) {
+            const float s = S[i >> 2][i & 3];
+            const float lo = FOLD ? dpp<0x128>(s) : u[i >> 2][i & 3];  // (rotated by 8 columns)
+            const float full = fabsf(s) == INFINITY ? s : fmaf(fmaf(lo, 0x1p-11f, t[i >> 2][i & 3]), 0x1p-11f, s);
+            S[i >> 2][i & 3] = !FOLD || q.own ? full : 0.f;
         }
         softmax_tile(st, S, q.c, j0, te, g);
         if (j0 + 32u > te) {  // keys past the span repeat its last row: weight 0, and no 0 * inf either
@@ -321,7 +415,7 @@ struct F16D128 {
 // the matrix cores could take about three times the HBM rate.
 template <int D_>
 struct F32Kv {
-    static constexpr int D = D_, NO = D / 16, NK = D / 16, NV = D / 64;
+    static constexpr int D = D_, NO = D / 16, NK = D / 16, NV = D / 64, Q_LDS = 0;
     using Elem = float;
     struct Tile {
         float4_t k[2][NK];     // [key block][16 channels]
@@ -330,14 +424,16 @@ struct F32Kv {
     struct Query {
         float4_t v[NK];  // lane (g, n): channels 16 i + 4 g .. + 3 of head n
         float c;
-        __device__ __forceinline__ void load(const float *qrow, uint32_t g, bool head_ok) {
+        __device__ __forceinline__ void load(const float *q, uint32_t group, uint32_t, uint32_t g, uint32_t n) {
+            const bool head_ok = n < group;
+            const float *const qrow = q + (head_ok ? n : 0u) * D;
 #pragma unroll
             for (int i = 0; i < NK; ++i) {
                 const float4_t x = *(const float4_t *) (qrow + 16 * i + 4 * g);
                 v[i] = head_ok ? x : (float4_t){0.f, 0.f, 0.f, 0.f};
             }
         }
-        __device__ __forceinline__ void ready(float scale_log2e, uint32_t, uint32_t) { c = scale_log2e; }
+        __device__ __forceinline__ void ready(float scale_log2e, uint32_t, uint32_t, uint32_t *) { c = scale_log2e; }
     };
     static __device__ __forceinline__ void load(Tile &r, const uint32_t (&row)[2], const Elem *k_pages,
                                                 const Elem *v_pages, uint64_t row_elems, uint32_t kvh, uint32_t g,
@@ -444,9 +540,11 @@ __device__ __forceinline__ void decode_body(const typename P::Elem *k_pages, con
     // (16 heads, one channel quad each) then fall on 64 distinct banks (a stride of D floats put all
     // 16 heads on the same 16 banks)
     constexpr uint32_t OROW = D + 4u;
-    __shared__ float o_lds[WAVES][16 * OROW];
+    __shared__ __attribute__((aligned(16))) float o_lds[WAVES][16 * OROW];
     __shared__ float m_lds[WAVES][16];
     __shared__ float l_lds[WAVES][16];
+    __shared__ __attribute__((aligned(16))) uint32_t q_lds[P::Q_LDS ? P::Q_LDS : 1];
+    static_assert(!P::Q_LDS || (KB == 1 && WPK == 4), "four waves that share q");
 
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -503,7 +601,6 @@ __device__ __forceinline__ void decode_body(const typename P::Elem *k_pages, con
     const uint32_t kvh = min(kvh_raw, G - 1u);
     const uint32_t g = lane >> 4, n = lane & 15u, m16 = lane & 15u;
     const bool head_ok = kvh_ok && n < group;
-    const uint32_t h = kvh * group + (n < group ? n : 0u);
     const uint64_t row_elems = (uint64_t) G * D;
     const uint32_t pmask = (1u << sh) - 1u;
 
@@ -540,13 +637,13 @@ __device__ __forceinline__ void decode_body(const typename P::Elem *k_pages, con
         // ---- start-up: q and the first chunk's block-table entries leave together; the chunk's KV
         // loads leave as soon as the entries arrive, before the q arithmetic.
         typename P::Query q;
-        q.load(qb + (uint64_t) h * D, g, head_ok);
+        q.load(qb + (uint64_t) kvh * group * D, group, D, g, n);
         uint32_t pid[TILES][2];
         pages_of(jw, pid);
         typename P::Tile r[TILES];
         load_chunk(jw, r, pid);
         __builtin_amdgcn_sched_barrier(0);
-        q.ready(a.scale_log2e, g, n);
+        q.ready(a.scale_log2e, g, n, q_lds);
 
         // ---- key loop: every load of a chunk is issued before any of its tiles is computed, and
         // the next chunk's block-table entries leave before the computing starts. (The compiler
@@ -564,6 +661,10 @@ __device__ __forceinline__ void decode_body(const typename P::Elem *k_pages, con
             load_chunk(jw, r, pid);
             __builtin_amdgcn_sched_barrier(0);
         }
+    } else if constexpr (P::Q_LDS != 0) {  // a wave without keys makes its share of q and meets the others
+        typename P::Query q;
+        q.load(qb + (uint64_t) kvh * group * D, group, D, g, n);
+        q.ready(a.scale_log2e, g, n, q_lds);
     }
 
     // ---- merge the WPK waves of each KV head in LDS ---------------------------------------------
@@ -629,7 +730,8 @@ __device__ __forceinline__ void decode_body(const typename P::Elem *k_pages, con
 // f32 kind holds a 32 KiB tile per wave either way).
 DECODE_KERNEL(f16d64, F16D64, 4, 2, 4, 2)
 DECODE_KERNEL(f16d64, F16D64, 1, 4, 1, 4)
-DECODE_KERNEL(f16d128, F16D128, 1, 4, 1, 3)
+DECODE_KERNEL(f16d128, F16D128<true>, 1, 4, 1, 3)
+DECODE_KERNEL(f16d128g16, F16D128<false>, 1, 4, 1, 3)
 DECODE_KERNEL(f32d64, F32Kv<64>, 4, 2, 2, 2)
 DECODE_KERNEL(f32d64, F32Kv<64>, 1, 4, 1, 4)
 DECODE_KERNEL(f32d128, F32Kv<128>, 4, 2, 1, 2)

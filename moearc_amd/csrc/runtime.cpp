@@ -84,7 +84,7 @@ struct moearc_ctx {
     hipFunction_t f_rope_sums64 = nullptr;  // the same from the q/k/v product's split-K sums
     bool block_fused = true;  // MOEARC_BLOCK_FUSED=0: the attention block's fused steps as separate launches
     hipFunction_t f_dec_general = nullptr;
-    hipFunction_t f_dec_fast[4][2] = {};  // split kernels (kDecodeVariants): kind x variant
+    hipFunction_t f_dec_fast[5][2] = {};  // split kernels (kDecodeVariants): kind x variant
     hipFunction_t f_dec_merge[2] = {};    // head_dim 64, 128
     unsigned merge_threads = 0;  // the merge kernel's launch bound (its work-group size)
     hipFunction_t f_mv[7][4] = {};  // matvec: format (F32 F16 Q8_0 Q4_K Q5_K Q6_K MXFP4) x pieces per lane 1/2/4/8
@@ -294,7 +294,8 @@ struct SpanList {
 };
 
 // The split kernels' cache layouts: f16 and f32 entries, heads of 64 and 128 channels.
-enum DecodeKind { kF16D64, kF16D128, kF32D64, kF32D128, kNumDecodeKinds, kGeneral = -1 };
+// (128 f16 channels: with up to 8 query heads per KV head, and with up to 16.)
+enum DecodeKind { kF16D64, kF16D128, kF16D128G16, kF32D64, kF32D128, kNumDecodeKinds, kGeneral = -1 };
 
 // The split-K kernels mask keys with -inf scores before multiplying by scale*log2(e) and take
 // their running maximum on raw scores, so they need a positive, finite scale; they load rows in
@@ -309,7 +310,8 @@ DecodeKind decode_kind(const void *out, const float *q, const void *k_pages, con
         return kGeneral;
     if (kv_type == 1u && head_dim == 64) return kF16D64;
     if (((uintptr_t) out | (uintptr_t) q | (uintptr_t) k_pages | (uintptr_t) v_pages) % 16 != 0) return kGeneral;
-    return kv_type == 1u ? kF16D128 : head_dim == 64 ? kF32D64 : kF32D128;
+    if (kv_type == 1u) return n_heads / n_kv_heads <= 8 ? kF16D128 : kF16D128G16;
+    return head_dim == 64 ? kF32D64 : kF32D128;
 }
 
 unsigned long kind_dim(DecodeKind k) { return k == kF16D64 || k == kF32D64 ? 64 : 128; }
@@ -317,9 +319,9 @@ unsigned long kind_dim(DecodeKind k) { return k == kF16D64 || k == kF32D64 ? 64 
 // Split-K decode variants (moearc_attn_decode_<kind>_k<kb>w<wpk>t<tiles>): kb KV heads x wpk waves
 // per work-group, each wave computing `tiles` 32-key tiles per chunk with all of their loads in
 // flight; the work-group count the split length aims for. Each kind has a short-span variant, 4
-// waves on one KV head, whose target is what its registers let the device hold at once (104, 168, 128
-// and 230 VGPRs: 4, 3, 4 and 2 work-groups per CU). All but the 128-channel f16 kind have a long-span
-// one, 8 waves (2 per SIMD, one work-group per CU) with 32 KiB each in flight. That kind's (4x2x2)
+// waves on one KV head, whose target is what its registers let the device hold at once (102, 162 or
+// 166, 128 and 225 VGPRs: 4, 3, 4 and 2 work-groups per CU). All but the 128-channel f16 kinds have a long-span
+// one, 8 waves (2 per SIMD, one work-group per CU) with 32 KiB each in flight. Theirs (4x2x2)
 // measured no better at any size, 22.5 against 19.3-20.0 µs over 32K keys of 4 KV heads and 114.9
 // against 114.5 over 17 sequences of 2K-30K; the f32 kinds' long-span shapes win from 8 such
 // sequences on (105.9 against 109.9 µs at 128 channels) and tie below.
@@ -330,6 +332,7 @@ struct DecodeVariant {
 constexpr int kNumDecodeVariants = 2;
 constexpr DecodeVariant kDecodeVariants[kNumDecodeKinds][kNumDecodeVariants] = {
     {{"4x2x4", 4, 2, 4, 256}, {"1x4x1", 1, 4, 1, 1024}},
+    {{"1x4x1", 1, 4, 1, 768}, {"1x4x1", 1, 4, 1, 768}},
     {{"1x4x1", 1, 4, 1, 768}, {"1x4x1", 1, 4, 1, 768}},
     {{"4x2x2", 4, 2, 2, 256}, {"1x4x1", 1, 4, 1, 1024}},
     {{"4x2x1", 4, 2, 1, 256}, {"1x4x1", 1, 4, 1, 512}},
@@ -679,6 +682,8 @@ moearc_ctx *moearc_ctx_create(void) {
         {&c->f_dec_fast[kF16D64][1], "moearc_attn_decode_f16d64_k1w4t1"},
         {&c->f_dec_fast[kF16D128][0], "moearc_attn_decode_f16d128_k1w4t1"},
         {&c->f_dec_fast[kF16D128][1], "moearc_attn_decode_f16d128_k1w4t1"},
+        {&c->f_dec_fast[kF16D128G16][0], "moearc_attn_decode_f16d128g16_k1w4t1"},
+        {&c->f_dec_fast[kF16D128G16][1], "moearc_attn_decode_f16d128g16_k1w4t1"},
         {&c->f_dec_fast[kF32D64][0], "moearc_attn_decode_f32d64_k4w2t2"},
         {&c->f_dec_fast[kF32D64][1], "moearc_attn_decode_f32d64_k1w4t1"},
         {&c->f_dec_fast[kF32D128][0], "moearc_attn_decode_f32d128_k4w2t1"},

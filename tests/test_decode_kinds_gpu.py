@@ -185,6 +185,25 @@ def test_unaligned_buffers(kv, D):
             B.check(cx.download(o, np.float32, B.H * D), 0)
 
 
+@pytest.mark.parametrize("octaves", [10, 18, 26])
+@pytest.mark.parametrize("kv,D,group", [(*k, 8) for k in KINDS] + [("f16", 128, 1), ("f16", 128, 12)])
+def test_one_channel_far_above_the_others(kv, D, group, octaves):
+    # one channel of q some 2^octaves above the rest, its keys as far below: every channel has its share of
+    # the scores, so the small ones must keep their f32 precision beside the large one
+    B = Batch(19, kv, D, [300], 16, 4, group)
+    dt = np.float16 if kv == "f16" else np.float32
+    k = B.k.view(dt).reshape(-1, D).astype(np.float32) * np.float32(2.0 ** 12)
+    k[:, 0] *= np.float32(2.0 ** -octaves)
+    B.k = np.ascontiguousarray(fx.synth.f16_bits(k.ravel()) if kv == "f16" else k)
+    B.q = (B.q.reshape(-1, D) * np.where(np.arange(D) == 0, 1.0, 2.0 ** -octaves)).astype(np.float32).ravel()
+    B.scale = float(np.float32(2.0 ** (octaves - 12) / np.sqrt(D)))
+    with Context() as cx:
+        q, dk, dv, bt, s = B.upload(cx)
+        out = cx.alloc(B.H * D * 4)
+        cx.attn_decode_ext(out, q, dk, dv, bt, s, B.H, B.G, D, 0, 300, 16, B.scale, B.type)
+        B.check(cx.download(out, np.float32, B.H * D), 0)
+
+
 @pytest.mark.parametrize("kv,D", KINDS)
 def test_infinities(kv, D):
     # a key of -inf in a whole first tile weighs nothing; an infinite value shows in its channel alone;
