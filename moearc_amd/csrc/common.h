@@ -17,6 +17,12 @@ typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 // log2(e) in f32: exp(x) = exp2(x * log2(e)).
 #define MOEARC_LOG2E 1.4426950408889634f
 
+// The value of the lane that DPP control CTRL names, within the lane's 16.
+template <int CTRL>
+__device__ __forceinline__ float dpp(float x) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, true));
+}
+
 // A 16-byte store written through to the device-coherent level (sc1, as an agent-scope store): a
 // kernel's end then has no dirty L2 lines of it to write back, which for outputs of tens of MB is
 // microseconds of the dispatch. It pays for whole-line writes (the prefill's output rows); 4-byte

@@ -69,12 +69,6 @@ __device__ __forceinline__ float wave_max_16_32(float x) {
     return x;
 }
 
-// the value of the lane that DPP control CTRL names, within its 16 lanes
-template <int CTRL>
-__device__ __forceinline__ float dpp(float x) {
-    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xF, 0xF, false));
-}
-
 __device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // What the scores of a head start from: below any score in the log2 domain, and finite, so that a
@@ -253,7 +247,7 @@ __device__ __forceinline__ uint32_t v_row(const uint32_t (&row)[2], int blk, uin
 
 // ---- f16 cache, 128 channels: HBM-bound like the 64-channel kind, 512 bytes per key and KV head.
 // Scores as there, but with q whole in three f16 operands per 32 channels, q = hi + mid / 2^11 +
-// lo / 2^22, each with sums of its own: f32's 24 bits for every channel down to 2^-38 of the head's
+// lo / 2^22, each with sums of its own: f32's 24 bits for every channel down to 2^-28 of the head's
 // largest (the general kernel multiplies in f32; two pieces kept about 7 bits of a channel 2^18 below the
 // largest). FOLD, for groups of up to 8 heads: lo takes the idle columns 8 .. 15 of hi's product, so the
 // third piece costs neither an MFMA nor a register. (In f32 MFMAs instead, four sequences of 2K-8K keys

@@ -13,8 +13,7 @@
 // rule).
 //
 // Precision is matmul.hip's: x = hi + lo to 2^-22, payloads as exact f16 integers (E2M1 code points
-// for MXFP4), each block's f32 sum scaled in f32. The K-quants' mins multiply the block's sum of
-// hi + lo, taken by two more MFMAs against ones.
+// for MXFP4), each block's f32 sum scaled in f32. The K-quants' mins multiply the block's f32 sum of x.
 #include "common.h"
 
 namespace {
@@ -138,14 +137,17 @@ __device__ __forceinline__ float4_t mms_mfma(half8_t a, half8_t b, float4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
 
+__device__ __forceinline__ uint32_t mms_token(uint32_t q, uint32_t k) { return 2u * q + (k & 1u) + 8u * (k >> 1); }
+
 // T tiles of 16 tokens, CK k-blocks per batch of activation loads.
 template <uint32_t TY, int T, int CK>
 __device__ __forceinline__ void mms_body(const MatmulArgs &a) {
     using F = MmsFmt<TY>;
     constexpr uint32_t WB = F::WB;
+    constexpr bool Q45 = TY == 12 || TY == 13;
     static_assert(WB % (2 * CK) == 0, "activation batches alternate within a window");
     // per wave: a window of weights; a k-block's activations in f16, [tile][hi, lo][16-byte slots], and at
-    // the end the wave's sums, [tile][token 4 q + k][row n]
+    // the end the wave's sums, [tile][token][row n]
     __shared__ __attribute__((aligned(16))) uint8_t wlds[MMS_WAVES][16 * F::RS];
     __shared__ u32x4_t xlds[MMS_WAVES][T][2][64];
     const auto red = [&](uint32_t w, uint32_t t) { return (float *) xlds[w][t]; };
@@ -175,7 +177,9 @@ __device__ __forceinline__ void mms_body(const MatmulArgs &a) {
     // floats 4 (l % 8) .. + 3 of the block. (In operand layout, 16 rows per load and a row's lanes 16
     // apart, a load of either operand cost 58 clocks at the L1 whatever it fetched: only neighbouring
     // lanes' addresses are joined. 16 tokens of Q8_0 4096 x 2880 took 15.0 us that way.) They reach
-    // operand layout through LDS, as f16: token u's 16-byte slot q (k 8 q .. + 7) at q ^ (u / 4).
+    // operand layout through LDS, as f16: token u's 16-byte slot q (k 8 q .. + 7) at q ^ (u / 4). Row 4 q + k
+    // of the A operand, and of D, is token mms_token(q, k) of its tile, so that the tokens whose sums a lane's D
+    // rows need (Q4_K, Q5_K) are those that its 16 lanes loaded.
     const float *x[T][2];
 #pragma unroll
     for (int t = 0; t < T; ++t)
@@ -188,7 +192,7 @@ __device__ __forceinline__ void mms_body(const MatmulArgs &a) {
         const uint32_t u = 8u * e + (lane >> 3), c = lane & 7u;
         put[e] = 2u * (4u * u + ((c >> 1) ^ (u >> 2))) + (c & 1u);
     }
-    const uint32_t get = 4u * n + (lq ^ (n >> 2));
+    const uint32_t un = mms_token(n >> 2, n & 3u), get = 4u * un + (lq ^ (un >> 2));
     struct Batch {
         mms_f4 x[CK][T][2];
     };
@@ -228,6 +232,19 @@ __device__ __forceinline__ void mms_body(const MatmulArgs &a) {
                     ((mms_half4 *) xlds[wave][t][0])[put[e]] = hi;
                     ((mms_half4 *) xlds[wave][t][1])[put[e]] = lo;
                 }
+            float sum[T][2];  // Q4_K, Q5_K: token 8 e + lane / 8's sum, over its eight lanes
+            if constexpr (Q45) {
+#pragma unroll
+                for (int t = 0; t < T; ++t)
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        const mms_f4 &v = o.x[i][t][e];
+                        float s = (v[0] + v[1]) + (v[2] + v[3]);
+                        s += dpp<0xB1>(s);
+                        s += dpp<0x4E>(s);
+                        sum[t][e] = s + dpp<0x141>(s);
+                    }
+            }
             __builtin_amdgcn_wave_barrier();
             float s0, s1;
             const half8_t bw = mms_operand<TY>(wrow, i0 + i, lq, s0, s1);
@@ -249,12 +266,12 @@ __device__ __forceinline__ void mms_body(const MatmulArgs &a) {
                     const float4_t s = mms_mfma(lo, bw, mms_mfma(hi, bw, zero));
 #pragma unroll
                     for (int k = 0; k < 4; ++k) acc[t][k] = fmaf(s0, s[k], acc[t][k]);
-                    if constexpr (TY == 12 || TY == 13) {
-                        const _Float16 u = (_Float16) 1.f;
-                        const half8_t ones = {u, u, u, u, u, u, u, u};
-                        const float4_t m = mms_mfma(lo, ones, mms_mfma(hi, ones, zero));
-#pragma unroll
-                        for (int k = 0; k < 4; ++k) acc[t][k] = fmaf(-s1, m[k], acc[t][k]);
+                    if constexpr (Q45) {
+                        // rows 4 lq .. + 3 of D: the tokens of lanes 0-7 and 8-15 of this lane's 16
+                        acc[t][0] = fmaf(dpp<0x150>(sum[t][0]), -s1, acc[t][0]);
+                        acc[t][1] = fmaf(dpp<0x158>(sum[t][0]), -s1, acc[t][1]);
+                        acc[t][2] = fmaf(dpp<0x150>(sum[t][1]), -s1, acc[t][2]);
+                        acc[t][3] = fmaf(dpp<0x158>(sum[t][1]), -s1, acc[t][3]);
                     }
                 }
             }
@@ -291,7 +308,7 @@ __device__ __forceinline__ void mms_body(const MatmulArgs &a) {
 #pragma unroll
     for (int t = 0; t < T; ++t)
 #pragma unroll
-        for (int k = 0; k < 4; ++k) red(wave, t)[16u * (4u * lq + k) + n] = acc[t][k];
+        for (int k = 0; k < 4; ++k) red(wave, t)[16u * mms_token(lq, k) + n] = acc[t][k];
     __syncthreads();
     // element e of tile t: token 16 t + e / 16, row r0 + e % 16, the waves' sums in order
     for (uint32_t i = tid; i < 256u * T; i += 64u * MMS_WAVES) {
