@@ -227,7 +227,7 @@ struct MatmulArgs {
     MatmulSeg seg[MOEARC_MM_MAX_SEG];
     const uint16_t *xh, *xl;   // [n_tok][cols] f16: x = hi + lo to within 2^-22 |x|
     const float *xs;           // Q4_K, Q5_K: block sums of x, f32 [n_tok][cols / 32] (matmul.hip) or f16
-                               // pieces [n_tok][cols / 256][2][8] (matmul2k.hip); matmul_small.hip: x
+                               // pieces [n_tok][cols / 256][4][8] (matmul2k.hip); matmul_small.hip: x
                                // itself, f32 [n_tok][cols]; else unread
     float *part;               // split launches (grid z > 1): slice z's sums, [t][r] per matrix
     uint64_t part_stride;      // floats per slice: the sum of n_tok * rows over the matrices

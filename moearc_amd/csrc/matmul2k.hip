@@ -6,27 +6,31 @@
 // f16, so it is the matrix operand itself, and products of several sub-blocks add up in the matrix cores
 // before d scales them. The operand costs what q alone did: the 0x64 exponent trick gives 1024 + q, and
 // one packed f16 multiply-add, (1024 + q) * sc - 1024 * sc, exact, replaces the subtraction. The mins,
-// sum over sub-blocks of m * (sum of x), are a 32x32x16 MFMA per super-block and tile too: its 16-wide
-// k is the 8 sub-blocks' activation sums in two f16 pieces, v = sum / 64 = v0 + v1 / 2048 to 2^-24 |v|
-// (moearc_split_sums_k), against m and m / 2048, exact in f16.
+// sum over sub-blocks of m * (sum of x), are two 32x32x16 MFMAs per super-block and tile too: of the
+// 8 sub-blocks' activation sums in four f16 pieces, sum / 64 = v0 + v1 / 2^11 + v2 / 2^22 + v3 / 2^33
+// (moearc_split_sums_k), two side by side in a 16-wide k: v2 and v3 against m / 2^12 and m / 2^23, then v0
+// and v1 against 2^10 m and m / 2, all exact in f16. v0 and v1 are 0 rather than subnormal (the matrix cores
+// align a subnormal operand as if it were 2^-14, and its low bits drop out), so the pieces hold an f32 sum
+// whole down to 2^-19, its first 23 bits down to 2^-30.
 //
 // What bounds it: with a scale and a min per sub-block (128 f32 multiply-adds per 16 MFMAs and wave,
 // and 16-byte LDS reads of the sums for the mins) the vector unit did, at about twice the matrix time.
-// 4096 x 2048 Q4_K over 2048 tokens 130 -> 95 us, over 1000 (two k-slices and their reduction) 82 -> 64,
-// over 128 30.4 -> 25.4; Q5_K 2048 x 4096 over 300 46 -> 35.
+// Whole calls, split and sums included: 4096 x 2048 Q4_K over 2048 tokens 126 -> 96 us, over 1000 78 -> 56,
+// over 128 28.8 -> 24.4; Q5_K 2048 x 4096 over 300 44 -> 34. The mins in two pieces and one MFMA, to 2^-23 of
+// a sum, were 1.0-1.5% faster.
 //
 // Sums of a pair of sub-blocks go to the accumulators, d applied: the f32 rounding of the matrix cores'
 // running sum grows with its length. Relative error against float64 (1000 tokens of N(0, 1), 2048
-// columns): 2.3e-7 with a scale per sub-block; 2.0e-7 by pairs, 2.2e-7 by four, 2.8e-7 by super-blocks,
-// each twice as long about 1% faster. The low halves of the activations are multiplied first, while the
-// sum is still small (2.1e-7 by pairs in hi, lo order).
+// columns): 2.4e-7 with a scale per sub-block; 1.9e-7 by pairs, and, with the mins in two pieces, 2.0e-7 by
+// pairs, 2.2e-7 by four, 2.8e-7 by super-blocks, each twice as long about 1% faster. The low halves of the
+// activations are multiplied first, while the sum is still small (2.1e-7 by pairs in hi, lo order).
 #include "common.h"
 
 namespace {
 
 // LDS: three activation buffers as in matmul2.hip; two buffers of a pair of sub-blocks' 32 payload
 // bytes per row (low nibbles: the first sub-block); two of a super-block's header per row (d, dmin,
-// the 12 scale bytes; Q5_K: and the 32 bytes of fifth bits); one super-block's sums per token.
+// the 12 scale bytes; Q5_K: and the 32 bytes of fifth bits); one super-block's sums per token (v0 and v1; v2 and v3).
 template <uint32_t TY, uint32_t KS = 1>  // KS: as mm2_body's
 __device__ __forceinline__ void mm2k_body(const MatmulArgs &a) {
     constexpr bool Q5K = TY == 13;
@@ -34,7 +38,7 @@ __device__ __forceinline__ void mm2k_body(const MatmulArgs &a) {
     constexpr uint32_t HDR = Q5K ? 48u : 16u, NHDR = Q5K ? 2u : 1u;   // header bytes per row, copies per wave
     constexpr uint32_t PAIR = MM2_ROWS * 32u;
     constexpr uint32_t PAIR0 = MM2_NBUF * MM2_ACT, HDR0 = PAIR0 + 2u * PAIR, SUM0 = HDR0 + 2u * MM2_ROWS * HDR;
-    constexpr uint32_t LDS = SUM0 + MM2_TOK * 32u;
+    constexpr uint32_t LDS = SUM0 + 2u * MM2_TOK * 32u;
     __shared__ __attribute__((aligned(1024))) uint8_t tiles[KS * LDS];
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave8 = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -62,7 +66,7 @@ __device__ __forceinline__ void mm2k_body(const MatmulArgs &a) {
     const uint32_t prow = (64u * wave + lane) >> 1, pchunk = (lane & 1u) ^ ((prow >> 3) & 1u);
     const uint64_t sb0 = SB * (uint64_t) (kb0 >> 3);
     const uint8_t *psrc = sg.w + (uint64_t) min(r0 + prow, sg.rows - 1u) * sg.row_bytes + sb0 + QS + 16u * pchunk;
-    const uint8_t *ssrc = (const uint8_t *) a.xs + ((uint64_t) min(t0 + prow, a.n_tok - 1u) * (a.cols >> 8) + (kb0 >> 3)) * 32u +
+    const uint8_t *ssrc = (const uint8_t *) a.xs + ((uint64_t) min(t0 + prow, a.n_tok - 1u) * (a.cols >> 8) + (kb0 >> 3)) * 64u +
                           16u * pchunk;
     // Headers: Q4_K row 64 (w & 1) + lane (waves 2 and 3 repeat 0 and 1); Q5_K instruction i of wave w
     // fills slots 64 min(2 w + i, 5) .. + 63, slot q being row q / 3's chunk q % 3.
@@ -126,14 +130,18 @@ __device__ __forceinline__ void mm2k_body(const MatmulArgs &a) {
             const uint32_t b = 8u * sb + j;
             __builtin_amdgcn_sched_barrier(0);
             if (j == 5u) __builtin_amdgcn_s_waitcnt(mm2_vmcnt_lgkm0(5u + NHDR));
-            else if (j % 2u == 1u || j == 2u) __builtin_amdgcn_s_waitcnt(mm2_vmcnt_lgkm0(5u));
+            else if (j == 2u) __builtin_amdgcn_s_waitcnt(mm2_vmcnt_lgkm0(6u));
+            else if (j % 2u == 1u) __builtin_amdgcn_s_waitcnt(mm2_vmcnt_lgkm0(5u));
             else __builtin_amdgcn_s_waitcnt(mm2_vmcnt_lgkm0(4u));
             __builtin_amdgcn_s_barrier();
             __builtin_amdgcn_sched_barrier(0);
             const uint32_t prev = bufo == 0u ? 2u * MM2_ACT : bufo - MM2_ACT;
             copy_act(min(b + 2u, nb - 1u), prev);
             if (j % 2u == 0u) copy_pair(min(b + 2u, nb - 2u), ((j >> 1) + 1u) & 1u);
-            if (j == 1u) mm2_copy16(at(SUM0 + wave * 1024u), ssrc + 32u * (uint64_t) sb);
+            if (j == 1u)
+#pragma unroll
+                for (uint32_t i = 0; i < 2; ++i)
+                    mm2_copy16(at(SUM0 + i * MM2_TOK * 32u + wave * 1024u), ssrc + 64u * (uint64_t) sb + 32u * i);
             if (j == 4u) copy_hdr(min(sb + 1u, nsb - 1u), hpar ^ 1u);
             __builtin_amdgcn_sched_barrier(0);
 
@@ -197,17 +205,22 @@ __device__ __forceinline__ void mm2k_body(const MatmulArgs &a) {
                     }
                 }
             if (j == 7u) {  // the super-block's mins and scale
-                half8_t xs[2];
+                half8_t v01[2], v23[2];
 #pragma unroll
-                for (int tt = 0; tt < 2; ++tt) xs[tt] = __builtin_bit_cast(half8_t, mm2_lds16(soff[tt]));
+                for (int tt = 0; tt < 2; ++tt) {
+                    v01[tt] = __builtin_bit_cast(half8_t, mm2_lds16(soff[tt]));
+                    v23[tt] = __builtin_bit_cast(half8_t, mm2_lds16(soff[tt] + MM2_TOK * 32u));
+                }
 #pragma unroll
                 for (int rt = 0; rt < 2; ++rt) {
-                    const half8_t m = mm2_u4_to_f16(mm2_u32x2{mn[rt][0], mn[rt][1]}) * (h ? (_Float16) 0x1p-11f : (_Float16) 1.f);
-                    const float dm = -64.f * (float) __builtin_bit_cast(_Float16, (uint16_t) (dd[rt] >> 16));
+                    const half8_t m = mm2_u4_to_f16(mm2_u32x2{mn[rt][0], mn[rt][1]});
+                    const half8_t m01 = m * (h ? (_Float16) 0.5f : (_Float16) 1024.f), m23 = m * (h ? (_Float16) 0x1p-23f : (_Float16) 0x1p-12f);
+                    const float dm = -0.0625f * (float) __builtin_bit_cast(_Float16, (uint16_t) (dd[rt] >> 16));
 #pragma unroll
                     for (int tt = 0; tt < 2; ++tt) {
                         mm2_f32x16 M = {};
-                        M = __builtin_amdgcn_mfma_f32_32x32x16_f16(xs[tt], m, M, 0, 0, 0);
+                        M = __builtin_amdgcn_mfma_f32_32x32x16_f16(v23[tt], m23, M, 0, 0, 0);
+                        M = __builtin_amdgcn_mfma_f32_32x32x16_f16(v01[tt], m01, M, 0, 0, 0);
 #pragma unroll
                         for (int e = 0; e < 16; ++e)
                             acc[tt][rt][e] = fmaf(dm, M[e], acc[tt][rt][e]);
@@ -241,9 +254,9 @@ extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_pe
 moearc_matmul2x_q5_k_k(MatmulArgs a) { mm2k_body<13, 2>(a); }
 
 // The f16 hi / lo split of x (as moearc_split_f16_k) and, in the same pass, each super-block's eight
-// 32-wide sums as two f16 pieces for the mins' MFMA: piece 0 f16(v), piece 1 f16((v - f32(piece 0)) *
-// 2048), v = sum / 64 (an f16 sum of 32 activations could overflow). A thread takes eight elements, four
-// lanes a sub-block. xs: [n / 256][piece][8]. ALIGNED: x on 16 bytes, else element loads.
+// 32-wide sums in f32 as the four f16 pieces of v = sum / 64 (an f16 sum of 32 activations could overflow):
+// v0 = f16(v), v1 = f16 of the remainder times 2^11 and so on; the remainders are exact. A thread takes eight
+// elements, four lanes a sub-block. xs: [n / 256][piece][8]. ALIGNED: x on 16 bytes, else element loads.
 template <bool ALIGNED>
 __device__ __forceinline__ void split_sums(const float *x, uint16_t *hi, uint16_t *lo, uint16_t *xs, uint64_t n8) {
     for (uint64_t i = (uint64_t) blockIdx.x * blockDim.x + threadIdx.x; i < n8; i += (uint64_t) gridDim.x * blockDim.x) {
@@ -272,9 +285,15 @@ __device__ __forceinline__ void split_sums(const float *x, uint16_t *hi, uint16_
         t += __shfl_xor(t, 1);  // n8 is a multiple of 32: a sub-block's four lanes are all here
         t += __shfl_xor(t, 2);
         t *= 0x1p-6f;
-        const _Float16 p0 = (_Float16) t, p1 = (_Float16) ((t - (float) p0) * 2048.f);
-        if ((i & 3u) < 2u)
-            xs[(i >> 5) * 16u + 8u * (uint32_t) (i & 3u) + (uint32_t) ((i >> 2) & 7u)] = __builtin_bit_cast(uint16_t, (i & 3u) ? p1 : p0);
+        _Float16 part[4];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            part[p] = p < 2 && fabsf(t) < 0x1p-14f ? (_Float16) 0.f : (_Float16) t;
+            t = (t - (float) part[p]) * 2048.f;
+        }
+        const uint32_t p = (uint32_t) (i & 3u);
+        xs[(i >> 5) * 32u + 8u * p + (uint32_t) ((i >> 2) & 7u)] =
+            __builtin_bit_cast(uint16_t, p == 0u ? part[0] : p == 1u ? part[1] : p == 2u ? part[2] : part[3]);
     }
 }
 extern "C" __global__ void moearc_split_sums_k(const float *x, uint16_t *hi, uint16_t *lo, uint16_t *xs, uint64_t n8) {

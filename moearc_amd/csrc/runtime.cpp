@@ -1816,7 +1816,7 @@ bool mm_needs_sums(unsigned ty) { return ty == 12u || ty == 13u; }
 // (the K-quants: n a multiple of 256), its 32-element block sums behind it: in f32 for the kernels of up
 // to 32 tokens, as f16 pieces per super-block for the 128 x 128 tiles (MatmulArgs::xs; the same space).
 int mm_split_space(moearc_ctx *c, size_t n, uint16_t **xh, uint16_t **xl, float **xs) {
-    const size_t halves = 2 * n + n / 16;  // hi, lo, then n / 32 floats
+    const size_t halves = 2 * n + 4 * (n / 32);  // hi, lo, then n / 32 sums of four f16 pieces (or of one float)
     if (halves > c->mm_ws_halves) {
         if (c->mm_ws) {
             if (hipStreamSynchronize(c->stream) != hipSuccess || hipFree(c->mm_ws) != hipSuccess) return ERR;

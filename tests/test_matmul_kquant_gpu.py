@@ -36,7 +36,8 @@ def test_super_blocks(ctx, ty, n_tok, rows, cols, x_off):
     assert worst <= 1.0
 
 
-@pytest.mark.parametrize("n_tok,rows,cols", [(5, 40, 512), (24, 33, 256), (64, 50, 768)])  # matmul_small.hip
+@pytest.mark.parametrize("n_tok,rows,cols", [(5, 40, 512), (24, 33, 256), (64, 50, 768),  # matmul_small.hip
+                                             (70, 129, 512), (130, 40, 2304), (400, 6017, 512)])
 @pytest.mark.parametrize("size", [1.0, 2.0 ** -20])
 @pytest.mark.parametrize("ty", [QuantType.Q4_K, QuantType.Q5_K], ids=lambda t: t.name)
 def test_mins_take_f32_sums(ctx, ty, size, n_tok, rows, cols):
