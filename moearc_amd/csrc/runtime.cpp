@@ -268,7 +268,11 @@ int ensure_floats(moearc_ctx *c, float *&ws, size_t &have, size_t floats) {
         ws = nullptr;
         have = 0;
     }
-    if (hipMalloc((void **) &ws, floats * sizeof(float)) != hipSuccess) return ERR;
+    if (hipMalloc((void **) &ws, floats * sizeof(float)) != hipSuccess) {
+        (void) hipGetLastError();  // a caller that does without leaves no error for the program's next check
+        ws = nullptr;
+        return ERR;
+    }
     have = floats;
     return OK;
 }
@@ -1520,12 +1524,12 @@ int prefill_launch(moearc_ctx *c, void *out, unsigned int out_type, uint16_t *ou
     if (wgs > 0x7FFFFFFFull) return ERR_ARG;
     PrefillPlan plan;
     if (!precise && !capturing(c)) plan_prefill(a, rows_per_tile / (uint32_t) group, c->n_cu, plan);
-    if (plan.items) {
-        const uint64_t n = (uint64_t) plan.items * n_kv_heads;
+    const uint64_t n = (uint64_t) plan.items * n_kv_heads;
+    // without memory for the records (up to 35 MB) the one launch, which needs none
+    if (plan.items && ensure_floats(c, c->pf_ws, c->pf_ws_floats, n * MOEARC_PF_RECORD_FLOATS) == OK) {
         PrefillSplitArgs s{};
         a.pair_half = n > c->n_cu ? c->n_cu : 0u;
         s.a = a;
-        if (ensure_floats(c, c->pf_ws, c->pf_ws_floats, n * MOEARC_PF_RECORD_FLOATS)) return ERR;
         s.rec_o = c->pf_ws;
         s.rec_ml = s.rec_o + n * MOEARC_PREFILL_FAST_ROWS * 64u;
         s.n_items = plan.items;

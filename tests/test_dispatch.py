@@ -41,3 +41,20 @@ def test_a_product_over_its_own_input_reads_it_first(lib, ty, n_tok):
         for y in (x, x + 4, x - 4, x + used - 4, x - used + 4):
             got = call(y, x)
             assert any(k.startswith("moearc_split") for k in got) and not any("small" in k for k in got), got
+
+
+BIG = 1 << 44
+
+
+def _prefill(cx, n_q=200, pos0=16301):
+    cx.attn_prefill(*(at(cx, (1 << 33) + i * BIG, BIG) for i in range(6)), n_q, pos0, 0, 64, 8, 64, 256, 0.125)
+
+
+def test_prefill_without_memory_for_records_is_not_split(lib):
+    with Context() as cx:
+        lib.host_hip_largest(1 << 16)
+        _prefill(cx)
+        assert names(lib) == ["moearc_attn_prefill_g8"] and lib.host_hip_last_error() == 0
+        lib.host_hip_reset()
+        _prefill(cx)
+        assert names(lib) == ["moearc_attn_prefill_split_g8", "moearc_attn_prefill_merge_k"]
