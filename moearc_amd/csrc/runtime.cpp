@@ -516,6 +516,16 @@ int decode_launch_body(moearc_ctx *c, void *out, unsigned int out_f16, const flo
         int variant = 0;
         uint32_t split_len = 0;
         if (kind != kGeneral) plan_group(c, kind, sub, cnt, n_heads, n_kv_heads, rs, variant, split_len);
+        if (kind != kGeneral && kind != kF16D64 && !rs.fixed) {
+            // without memory for their records these kinds run one split per sequence, as when captured (the
+            // general kernel, which served them before, needed none)
+            const uint64_t items = group_items(sub, cnt, split_len);
+            if (items > cnt && ensure_floats(c, c->ws_kinds, c->ws_kinds_floats, (size_t) (n_heads * items * rec_floats))) {
+                rs.fixed = c->scratch;
+                rs.cap = 0;
+                plan_group(c, kind, sub, cnt, n_heads, n_kv_heads, rs, variant, split_len);
+            }
+        }
         if (kind == kGeneral) {
             DecodeGeneralArgs a{};
             a.q = qb;

@@ -5,7 +5,7 @@ import pytest
 
 import host_hip
 from host_hip import at, names
-from moearc_amd import Context, QuantType, native
+from moearc_amd import Context, KvType, QuantType, native
 
 MM = [QuantType.F16, QuantType.Q8_0, QuantType.MXFP4, QuantType.Q4_K, QuantType.Q5_K, QuantType.Q6_K]
 
@@ -46,8 +46,33 @@ def test_a_product_over_its_own_input_reads_it_first(lib, ty, n_tok):
 BIG = 1 << 44
 
 
+def _decode(cx, kv, dim, n_kv, heads=32, kv_heads=4, page=256, base=1 << 33):
+    cx.attn_decode_ext(*(at(cx, base + i * BIG, BIG) for i in range(6)), heads, kv_heads, dim, 0, n_kv, page, 0.125,
+                       KvType.F16 if kv == "f16" else KvType.F32)
+
+
 def _prefill(cx, n_q=200, pos0=16301):
     cx.attn_prefill(*(at(cx, (1 << 33) + i * BIG, BIG) for i in range(6)), n_q, pos0, 0, 64, 8, 64, 256, 0.125)
+
+
+KINDS = [("f16", 128), ("f32", 64), ("f32", 128)]
+
+
+@pytest.mark.parametrize("kv,dim", KINDS)
+def test_decode_without_memory_for_records_is_not_split(lib, kv, dim):
+    # the general kernel, which took these caches before, needed no memory: neither may they
+    with Context() as cx:
+        lib.host_hip_largest(1 << 16)
+        _decode(cx, kv, dim, 20000)
+        one = names(lib)
+        assert len(one) == 1 and f"{kv}d{dim}" in one[0] and lib.host_hip_last_error() == 0
+        lib.host_hip_reset()
+        _decode(cx, kv, dim, 20000)
+        assert len(names(lib)) == 2 and "merge" in names(lib)[1]
+        lib.host_hip_reset()
+        lib.host_hip_largest(1 << 16)  # a workspace that cannot grow
+        _decode(cx, kv, dim, 20000, heads=64)
+        assert len(names(lib)) == 1
 
 
 def test_prefill_without_memory_for_records_is_not_split(lib):
