@@ -457,7 +457,7 @@ int decode_launch(moearc_ctx *c, void *out, unsigned int out_f16, const float *q
                   unsigned long page_tokens, float scale, unsigned int kv_type, RecordSpace rs = {}) {
     // A fixed record buffer must hold every launch group's records: checked for all groups before
     // anything is enqueued, so a refusal leaves the stream untouched.
-    const DecodeKind kind =
+    DecodeKind kind =
         decode_kind(out, q, k_pages, v_pages, n_heads, n_kv_heads, head_dim, page_tokens, kv_type, scale);
     // Under stream capture the kinds that the general kernel used to serve keep no records (one split
     // per sequence): that kernel needed no memory, so a captured call of theirs must neither allocate,
@@ -476,7 +476,11 @@ int decode_launch(moearc_ctx *c, void *out, unsigned int out_f16, const float *q
             uint32_t split_len = 0;
             plan_group(c, kind, sub, cnt, n_heads, n_kv_heads, rs, variant, split_len);
             const uint64_t items = group_items(sub, cnt, split_len);
-            if (items > cnt && (uint64_t) n_heads * items * record_floats(kind) > rs.cap) return ERR_ARG;
+            if (items > cnt && (uint64_t) n_heads * items * record_floats(kind) > rs.cap) {
+                if (kind == kF16D64) return ERR_ARG;
+                kind = kGeneral;  // a span of more keys than the longest split
+                break;
+            }
         }
     }
     // With profiling on, the whole call (split and merge launches, SWA and full layers alike) is
@@ -524,6 +528,7 @@ int decode_launch_body(moearc_ctx *c, void *out, unsigned int out_f16, const flo
                 rs.fixed = c->scratch;
                 rs.cap = 0;
                 plan_group(c, kind, sub, cnt, n_heads, n_kv_heads, rs, variant, split_len);
+                if (group_items(sub, cnt, split_len) > cnt) kind = kGeneral;  // more keys than the longest split
             }
         }
         if (kind == kGeneral) {

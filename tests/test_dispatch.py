@@ -83,3 +83,17 @@ def test_prefill_without_memory_for_records_is_not_split(lib):
         lib.host_hip_reset()
         _prefill(cx)
         assert names(lib) == ["moearc_attn_prefill_split_g8", "moearc_attn_prefill_merge_k"]
+
+
+@pytest.mark.parametrize("kv,dim", KINDS)
+def test_a_span_too_long_for_one_split_takes_the_general_kernel(lib, kv, dim):
+    # a split holds at most 2^30 keys; where records are not to be had, longer spans stay with the general kernel
+    n_kv = 3 << 30
+    with Context() as cx:
+        _decode(cx, kv, dim, n_kv, page=1 << 20)
+        assert len(names(lib)) == 2
+        for prepare in (lambda: lib.host_hip_capture(1, 0), lambda: lib.host_hip_largest(1 << 10)):
+            lib.host_hip_reset()
+            prepare()
+            _decode(cx, kv, dim, n_kv, heads=64, page=1 << 20)
+            assert names(lib) == ["moearc_attn_decode_general_k"]
