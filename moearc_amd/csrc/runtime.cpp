@@ -259,8 +259,28 @@ int launch(moearc_ctx *c, hipFunction_t f, unsigned grid, unsigned block, const 
     return launch2d(c, f, grid, 1, block, args, what, r, m, 0, kernel);
 }
 
+bool capturing(moearc_ctx *c) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(c->stream, &status) == hipSuccess && status == hipStreamCaptureStatusActive;
+}
+
+// Lets this thread allocate and free while another stream than the context's, another context's say, is being
+// captured: in the default mode such a call fails and breaks that capture. Under a capture of the context's
+// own stream the program's mode stays, and refuses what it refused.
+struct RelaxedCapture {
+    const bool on;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    explicit RelaxedCapture(moearc_ctx *c) : on(!capturing(c)) {
+        if (on) (void) hipThreadExchangeStreamCaptureMode(&mode);
+    }
+    ~RelaxedCapture() {
+        if (on) (void) hipThreadExchangeStreamCaptureMode(&mode);
+    }
+};
+
 int ensure_floats(moearc_ctx *c, float *&ws, size_t &have, size_t floats) {
     if (floats <= have) return OK;
+    const RelaxedCapture relaxed(c);
     if (ws) {
         // the previous workspace may still be read by queued launches
         if (hipStreamSynchronize(c->stream) != hipSuccess) return ERR;
@@ -275,11 +295,6 @@ int ensure_floats(moearc_ctx *c, float *&ws, size_t &have, size_t floats) {
     }
     have = floats;
     return OK;
-}
-
-bool capturing(moearc_ctx *c) {
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(c->stream, &status) == hipSuccess && status == hipStreamCaptureStatusActive;
 }
 
 // ---- decode dispatch ----------------------------------------------------------------------------

@@ -6,6 +6,7 @@ import pytest
 import host_hip
 from host_hip import at, names
 from moearc_amd import Context, KvType, QuantType, native
+from moearc_amd.context import Failed
 
 MM = [QuantType.F16, QuantType.Q8_0, QuantType.MXFP4, QuantType.Q4_K, QuantType.Q5_K, QuantType.Q6_K]
 
@@ -97,3 +98,32 @@ def test_a_span_too_long_for_one_split_takes_the_general_kernel(lib, kv, dim):
             prepare()
             _decode(cx, kv, dim, n_kv, heads=64, page=1 << 20)
             assert names(lib) == ["moearc_attn_decode_general_k"]
+
+
+def test_growing_a_workspace_leaves_another_capture_alone(lib):
+    # a program may capture one stream while a context calls eagerly on its own: allocations then need a relaxed
+    # thread, or they fail and break the capture
+    with Context() as cx:
+        lib.host_hip_capture(0, 1)
+        _prefill(cx)
+        assert names(lib) == ["moearc_attn_prefill_split_g8", "moearc_attn_prefill_merge_k"]
+        for kv, dim in KINDS:
+            _decode(cx, kv, dim, 20000)
+        _prefill(cx, 200, 30000)
+        assert lib.host_hip_broken_captures() == 0
+        assert lib.hipMalloc(None, 16) != 0 and lib.host_hip_broken_captures() == 1  # the mode is the thread's own again
+        lib.host_hip_capture(0, 0)
+
+
+def test_a_captured_call_that_needs_a_workspace_is_refused(lib):
+    # 64-channel f16 heads keep their records in the workspace: growing it under capture fails, as ever
+    with Context() as cx:
+        lib.host_hip_capture(1, 0)
+        with pytest.raises(Failed):
+            _decode(cx, "f16", 64, 20000)
+        assert names(lib) == []
+        lib.host_hip_capture(0, 0)
+        _decode(cx, "f16", 64, 20000)
+        lib.host_hip_capture(1, 0)
+        _decode(cx, "f16", 64, 20000)
+        lib.host_hip_capture(0, 0)

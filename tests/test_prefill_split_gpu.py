@@ -105,6 +105,23 @@ def test_capture_needs_no_memory():
         hip.hipGraphDestroy(graph)
 
 
+def test_workspace_grows_beside_another_contexts_capture():
+    # the eager call's allocation neither fails nor breaks the capture (mode 0: global)
+    hip = ctypes.CDLL("libamdhip64.so")
+    pc = fx.prefill_case(0x5BE, n_q=40, pos0=4000, pt=256, H=16, G=2)
+    with Context() as other, Context() as cx:
+        x, stream, graph = other.upload(np.ones(64, np.float32)), ctypes.c_void_p(other.stream), ctypes.c_void_p()
+        bufs = [cx.upload(np.ascontiguousarray(a)) for a in (pc.qp.view(np.uint16), pc.k_raw, pc.v_raw, pc.bt, pc.sinks)]
+        out = cx.alloc(pc.n_q * pc.H * 64 * 4)
+        assert hip.hipStreamBeginCapture(stream, 0) == 0
+        other.zero(x, 64)
+        cx.attn_prefill(out, *bufs, pc.n_q, pc.pos0, 0, 16, 2, 64, 256, 0.125, KvType.F16)
+        assert hip.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+        hip.hipGraphDestroy(graph)
+        got = cx.download(out, np.float32, (pc.n_q, 16, 64))
+        assert np.max(np.abs(got - _want(pc, 0))) <= TOL
+
+
 def test_block_deep_in_a_context(monkeypatch):
     # the merge writes the output projection's activation split: as the separate launches do
     E, H, G, D, pt, n, pos0 = 512, 16, 2, 64, 256, 100, 4000
