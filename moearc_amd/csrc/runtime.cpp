@@ -1649,9 +1649,6 @@ struct MmSums {
     uint32_t slices = 0;
 };
 
-// y = W x for n_mat matrices of one weight type over the same chunk x, given as its f16 split
-// (xh, xl) of n_tok x n_cols, in one launch (plus the split-K reduction, unless `sums` takes the
-// slices' sums instead; y is then not written).
 // Whether a product of a few tokens runs from the f32 activations in one launch, 16 weight rows per
 // work-group, the reduction cut over its 8 waves (matmul_small.hip): rows of at least one window (eight
 // k-blocks), and up to 32 tokens (gpt-oss attn_q, 4096 x 2880 Q8_0: 8.8 us at 8 tokens, 11.8 at 32,
@@ -1659,8 +1656,18 @@ struct MmSums {
 // work-group per CU then), 64 (17.4 us at 63 and 64 against 27.1, and 21.7 on the 128 x 128 tiles). The
 // 5120 rows of a gpt-oss block's q, k and v are 320 tiles: 64 tokens of the block take 70 us that way
 // and 58 on the 128 x 128 tiles.
-bool mm_takes_f32(const moearc_ctx *c, unsigned long n_tok, unsigned long n_cols, uint64_t tiles16) {
-    return n_tok <= c->mm_small && n_cols >= 256 && (n_tok <= 32 || tiles16 <= 256);
+// Past 8192 rows two things end it. A work-group's fixed cost is spread over its 16 rows only, so short rows
+// lose: 65536 x 512 Q8_0 48 us for 25 at 17 tokens, 35 for 24 at 16; 1024 columns are level or better but
+// for Q8_0 past 16 tokens (52 for 42), from 2048 on all are (151936 x 2048: 174 for 242). And each work-group
+// reads all activations through the L2, which in F16, whose other kernels are the fastest, costs more
+// than they save past about 41K rows at 32 tokens (65536 x 2880: 140 us for 104), 49K at 16 (103 for 95)
+// and 65K at 8 (98304: 132 for 127).
+bool mm_takes_f32(const moearc_ctx *c, unsigned ty, unsigned long n_tok, unsigned long n_cols, uint64_t tiles16) {
+    if (n_tok > c->mm_small || n_cols < 256) return false;
+    if (n_tok > 32) return tiles16 <= 256;
+    if (tiles16 <= 512) return true;
+    if (ty == 1u) return n_cols >= 1024 && tiles16 <= (n_tok <= 8 ? 4096u : n_tok <= 16 ? 3072u : 2560u);
+    return n_cols >= (ty == 8u && n_tok > 16 ? 2048u : 1024u);
 }
 
 int mm_small_launch(moearc_ctx *c, unsigned ty, const MmMat *m, unsigned n_mat, const float *x, unsigned long n_tok,
@@ -1691,6 +1698,22 @@ int mm_small_launch(moearc_ctx *c, unsigned ty, const MmMat *m, unsigned n_mat, 
     return launch2d(c, f, (unsigned) tile_end, 1, 64 * MOEARC_MM_SMALL_WAVES, a, what, rows, n_tok);
 }
 
+// Whether a product runs on the 128 x 128 tiles of the 32x32x16 MFMA (matmul2.hip, matmul2k.hip) and not on
+// the 16x16x32 kernels (matmul.hip): chunks of at least 64 tokens, or of more than 32 over rows of 1024
+// columns and more (F16: 2048). 33 to 63 tokens of a gpt-oss block's q, k and v, too many rows for
+// matmul_small.hip, took 70-79 us per block on the 16x16x32 kernels and take 57-58; over shorter rows the
+// tiles, made for 128 tokens, lose: 33 tokens of 16384 x 512 Q6_K 23 us for 20, x 256 F16 15 for 10,
+// 65536 x 1024 F16 41 for 35. Q8_0 and MXFP4 weights arrive there in pairs of k-blocks, so their rows must
+// hold an even number of them.
+bool mm_takes_tiles(unsigned ty, unsigned long n_tok, unsigned long n_cols) {
+    const bool pairs = ty == 8u || ty == 39u;
+    if (pairs && (n_cols / 32) % 2 != 0) return false;
+    return n_tok >= 64 || (n_tok > 32 && n_cols >= (ty == 1u ? 2048u : 1024u));
+}
+
+// y = W x for n_mat matrices of one weight type over the same chunk x, given as its f16 split
+// (xh, xl) of n_tok x n_cols, in one launch (plus the split-K reduction, unless `sums` takes the
+// slices' sums instead; y is then not written).
 int mm_launch(moearc_ctx *c, unsigned ty, const MmMat *m, unsigned n_mat, const uint16_t *xh, const uint16_t *xl,
               const float *xs, unsigned long n_tok, unsigned long n_cols, const char *what,
               bool accumulate = false, MmSums *sums = nullptr) {
@@ -1710,17 +1733,13 @@ int mm_launch(moearc_ctx *c, unsigned ty, const MmMat *m, unsigned n_mat, const 
         tiles128 += (m[i].rows + 127) / 128;
         tiles256 += (m[i].rows + 255) / 256;
     }
-    // Every format over chunks of more than 32 tokens: 128 x 128 tiles on the 32x32x16 MFMA (matmul2.hip;
-    // 33 to 63 tokens of a gpt-oss block's q, k and v, too many rows for matmul_small.hip, took 70-79 us
-    // per block on the 16 x 16 x 32 kernels and take 57-58; Q8_0 and MXFP4 weights arrive there in pairs of k-blocks, so their rows must
-    // hold an even number of them). Otherwise 32 rows per wave halves the activation loads per MFMA, but only
-    // pays while the launch still has about two work-groups per CU; shorter chunks take 16.
+    // The 16x16x32 kernels: 32 rows per wave halves the activation loads per MFMA, but only pays while the
+    // launch still has about two work-groups per CU; shorter chunks take 16.
     hipFunction_t f;
     unsigned long rows_per_tile;
     unsigned gy;
     const bool pairs = ty == 8u || ty == 39u;
-    const bool mm2 = (ty == 1u || ty == 12u || ty == 13u || ty == 14u || (pairs && (n_cols / 32) % 2 == 0)) &&
-                     n_tok > 32;
+    const bool mm2 = mm_takes_tiles(ty, n_tok, n_cols);
     // F16, Q8_0 and MXFP4 take work-groups of eight waves over 128 tokens x 256 rows (one per CU)
     // when those tiles alone cover every CU in whole rounds, the last at least three quarters
     // full: each k-block's copies into LDS then serve twice the rows, and the copies' volume is
@@ -1847,8 +1866,8 @@ int mm_launch(moearc_ctx *c, unsigned ty, const MmMat *m, unsigned n_mat, const 
 bool mm_needs_sums(unsigned ty) { return ty == 12u || ty == 13u; }
 
 // The f16 hi / lo split of x (n floats, n a multiple of 32) into the context's buffer, and, when `sums`
-// (the K-quants: n a multiple of 256), its 32-element block sums behind it: in f32 for the kernels of up
-// to 32 tokens, as f16 pieces per super-block for the 128 x 128 tiles (MatmulArgs::xs; the same space).
+// (the K-quants: n a multiple of 256), its 32-element block sums behind it: as f16 pieces per super-block for
+// the 128 x 128 tiles (`tiles`), else in f32 (MatmulArgs::xs; the same space).
 int mm_split_space(moearc_ctx *c, size_t n, uint16_t **xh, uint16_t **xl, float **xs) {
     const size_t halves = 2 * n + 4 * (n / 32);  // hi, lo, then n / 32 sums of four f16 pieces (or of one float)
     if (halves > c->mm_ws_halves) {
@@ -1866,9 +1885,9 @@ int mm_split_space(moearc_ctx *c, size_t n, uint16_t **xh, uint16_t **xl, float 
     return OK;
 }
 
-int mm_split(moearc_ctx *c, const float *x, size_t n, uint16_t **xh, uint16_t **xl, float **xs, bool sums, unsigned long n_tok) {
+int mm_split(moearc_ctx *c, const float *x, size_t n, uint16_t **xh, uint16_t **xl, float **xs, bool sums, bool tiles) {
     if (const int rc = mm_split_space(c, n, xh, xl, xs)) return rc;
-    if (sums && n_tok > 32) {  // one pass for both: 1000 x 2048 activations 10.2 us in two launches
+    if (sums && tiles) {  // one pass for both: 1000 x 2048 activations 10.2 us in two launches
         struct {
             const float *x;
             uint16_t *hi, *lo, *xs;
@@ -1909,11 +1928,12 @@ int moearc_matmul_q(moearc_ctx *c, unsigned int type_id, float *y, const void *w
     const MmMat mat{w, bias, y, n_rows, n_rows};
     // y over x: rows may be written only once x is in the workspace (the one launch reads x throughout)
     const bool apart = (uintptr_t) (y + n_tok * n_rows) <= (uintptr_t) x || (uintptr_t) (x + n_tok * n_cols) <= (uintptr_t) y;
-    if (apart && mm_takes_f32(c, n_tok, n_cols, (n_rows + 15) / 16))
+    if (apart && mm_takes_f32(c, type_id, n_tok, n_cols, (n_rows + 15) / 16))
         return mm_small_launch(c, type_id, &mat, 1, x, n_tok, n_cols, "matmul");
     uint16_t *xh, *xl;
     float *xs;
-    if (const int rc = mm_split(c, x, n_tok * n_cols, &xh, &xl, &xs, mm_needs_sums(type_id), n_tok)) return rc;
+    if (const int rc = mm_split(c, x, n_tok * n_cols, &xh, &xl, &xs, mm_needs_sums(type_id), mm_takes_tiles(type_id, n_tok, n_cols)))
+        return rc;
     return mm_launch(c, type_id, &mat, 1, xh, xl, xs, n_tok, n_cols, "matmul");
 }
 
@@ -1998,14 +2018,16 @@ int moearc_attn_block_chunk(moearc_ctx *c, const moearc_attn_block *b, float *h,
                         mm_check(b->w_type[0], b->w[0], n_tok, q_rows, E) == OK &&
                         mm_check(b->w_type[1], b->w[1], n_tok, kv_rows, E) == OK &&
                         mm_check(b->w_type[2], b->w[2], n_tok, kv_rows, E) == OK;
-    const bool small = mm_takes_f32(c, n_tok, E, (q_rows + 15) / 16 + 2 * ((kv_rows + 15) / 16)),
-               small_out = (small || n_tok <= 32) && mm_takes_f32(c, n_tok, q_rows, (E + 15) / 16);
+    bool small = true;
+    for (int i = 0; i < 3; ++i)
+        small = small && mm_takes_f32(c, b->w_type[i], n_tok, E, (q_rows + 15) / 16 + 2 * ((kv_rows + 15) / 16));
+    const bool small_out = (small || n_tok <= 32) && mm_takes_f32(c, b->w_type[3], n_tok, q_rows, (E + 15) / 16);
     if (mm_qkv) {
         uint16_t *xh = nullptr, *xl = nullptr;
         float *xs = nullptr;
         const bool sums = mm_needs_sums(b->w_type[0]) || mm_needs_sums(b->w_type[1]) || mm_needs_sums(b->w_type[2]);
         if (!small)
-            if (const int rc = mm_split(c, x, n_tok * E, &xh, &xl, &xs, sums, n_tok)) return rc;
+            if (const int rc = mm_split(c, x, n_tok * E, &xh, &xl, &xs, sums, mm_takes_tiles(12u, n_tok, E))) return rc;
         float *outs[3] = {q, k, v};
         const unsigned long rows[3] = {q_rows, kv_rows, kv_rows};
         // the projections of one weight type in one launch (a block's q, k and v usually share it)
@@ -2121,7 +2143,8 @@ int moearc_attn_block_chunk(moearc_ctx *c, const moearc_attn_block *b, float *h,
         uint16_t *xh = axh, *xl = axl;
         float *xs = axs;
         if (!att_split)
-            if (const int rc = mm_split(c, att, nq, &xh, &xl, &xs, mm_needs_sums(b->w_type[3]), n_tok)) return rc;
+            if (const int rc = mm_split(c, att, nq, &xh, &xl, &xs, mm_needs_sums(b->w_type[3]), mm_takes_tiles(12u, n_tok, q_rows)))
+                return rc;
         return mm_launch(c, b->w_type[3], &mat, 1, xh, xl, xs, n_tok, q_rows, "attn_proj_mm", true);
     }
     std::vector<MvJob> jobs;

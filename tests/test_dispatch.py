@@ -44,6 +44,55 @@ def test_a_product_over_its_own_input_reads_it_first(lib, ty, n_tok):
             assert any(k.startswith("moearc_split") for k in got) and not any("small" in k for k in got), got
 
 
+def _product(cx, lib, ty, n_tok, rows, cols):
+    lib.host_hip_reset()
+    size = 1 << 40
+    cx.matmul_q(ty, at(cx, 1 << 41, size), at(cx, 1 << 42, size), at(cx, 1 << 43, size), None, n_tok, rows, cols)
+    got = [k for k in names(lib) if "split" not in k and "sums" not in k and "reduce" not in k]
+    assert len(got) == 1
+    return got[0]
+
+
+Q = QuantType
+
+
+@pytest.mark.parametrize("ty,n_tok,rows,cols,form", [
+    # up to 32 tokens: the one launch while the rows are few, or long enough; F16 not past its row counts
+    (Q.Q8_0, 32, 8192, 256, "small"), (Q.Q8_0, 1, 8193, 256, "16"), (Q.Q8_0, 16, 8193, 1024, "small"),
+    (Q.Q8_0, 17, 8193, 1024, "16"), (Q.Q8_0, 17, 151936, 2048, "small"), (Q.MXFP4, 32, 8193, 1024, "small"),
+    (Q.MXFP4, 2, 8193, 992, "16"), (Q.Q4_K, 32, 262144, 1024, "small"), (Q.Q4_K, 32, 8193, 768, "16"),
+    (Q.Q5_K, 3, 8193, 768, "16"), (Q.Q6_K, 3, 8193, 768, "16"), (Q.F16, 32, 40960, 2880, "small"),
+    (Q.F16, 17, 40961, 2880, "16"), (Q.F16, 16, 49152, 2880, "small"), (Q.F16, 9, 49153, 2880, "16"),
+    (Q.F16, 8, 65536, 2880, "small"), (Q.F16, 8, 65537, 2880, "16"), (Q.F16, 8, 8193, 1000 - 1000 % 32, "16"),
+    (Q.Q8_0, 32, 64, 224, "16"),
+    # 33 to 64: in one round of work-groups the one launch, else the tiles, over short rows the 16 x 16 kernels
+    (Q.Q8_0, 64, 4096, 2880, "small"), (Q.Q8_0, 63, 4097, 2880, "tiles"), (Q.Q8_0, 63, 4097, 960, "16"),
+    (Q.Q4_K, 33, 4097, 1024, "tiles"), (Q.Q4_K, 63, 4097, 768, "16"), (Q.Q6_K, 33, 4097, 512, "16"),
+    (Q.F16, 33, 4097, 2048, "tiles"), (Q.F16, 63, 4097, 2016, "16"), (Q.F16, 64, 4097, 256, "tiles"),
+    # 65 and more: the tiles, but for rows of an odd number of Q8_0 or MXFP4 blocks
+    (Q.Q6_K, 65, 16, 256, "tiles"), (Q.Q8_0, 65, 16, 288, "16"), (Q.MXFP4, 500, 16, 96, "16"),
+    # a grid of about one tile per CU halves its reduction inside the work-group; F16, Q8_0 and MXFP4 go wide
+    (Q.Q4_K, 1000, 4096, 2048, "halves"), (Q.Q4_K, 1000, 2944, 2048, "tiles"), (Q.Q8_0, 400, 6017, 576, "halves"),
+    (Q.Q6_K, 2048, 4096, 2048, "tiles"), (Q.Q8_0, 2048, 4096, 2880, "wide"),
+], ids=str)
+def test_product_forms(lib, ty, n_tok, rows, cols, form):
+    name = ty.name.lower()
+    want = {"small": f"moearc_matmul_small_{name}_t{-(-n_tok // 16)}_k", "tiles": f"moearc_matmul2_{name}_k",
+            "halves": f"moearc_matmul2x_{name}_k", "wide": f"moearc_matmul2w_{name}_k", "16": f"moearc_matmul_{name}_r"}
+    with Context() as cx:
+        got = _product(cx, lib, ty, n_tok, rows, cols)
+        assert got.startswith(want[form]), got
+
+
+def test_without_the_small_form(lib, monkeypatch):
+    # MOEARC_MM_SMALL=0: the kernels that it replaced
+    monkeypatch.setenv("MOEARC_MM_SMALL", "0")
+    with Context() as cx:
+        for ty in MM:
+            assert _product(cx, lib, ty, 8, 4096, 2048).startswith(f"moearc_matmul_{ty.name.lower()}_r")
+            assert _product(cx, lib, ty, 40, 4096, 2048) == f"moearc_matmul2_{ty.name.lower()}_k"
+
+
 BIG = 1 << 44
 
 

@@ -18,7 +18,7 @@ BLOCKS = [QuantType.F16, QuantType.Q8_0, QuantType.MXFP4]
 SUPER = [QuantType.Q4_K, QuantType.Q5_K, QuantType.Q6_K]
 
 
-def _check(ctx, ty, n_tok, rows, cols, bias=True, w_off=0, x_off=0):
+def _check(ctx, ty, n_tok, rows, cols, bias=True, w_off=0, x_off=0, run=32):
     w, _ = fx.synth_blocks(int(ty), rows * cols // ty.block_elems, 0x3C3 + rows)
     x = fx.synth.unit(0x3C4 + cols, n_tok * cols).reshape(n_tok, cols)
     b = fx.synth.unit(0x3C5, rows)
@@ -30,7 +30,7 @@ def _check(ctx, ty, n_tok, rows, cols, bias=True, w_off=0, x_off=0):
     for t in range(n_tok):
         want, absum = oracle.matvec_q(int(ty), w, x[t], rows, cols, n_threads=8)
         want = want.astype(np.float64) + (b if bias else 0.0)
-        tol = fx.matvec_tolerance(cols, absum) + 2.0 * 32 * 2.0 ** -24 * absum + 2.0 ** -23 * np.abs(want)
+        tol = fx.matvec_tolerance(cols, absum) + 2.0 * run * 2.0 ** -24 * absum + 2.0 ** -23 * np.abs(want)
         worst = max(worst, float(np.max(np.abs(got[t] - want) / tol)))
     print(f"{ty.name} {n_tok} x {rows} x {cols}: worst / bound = {worst:.3f}", flush=True)
     assert worst <= 1.0
@@ -77,6 +77,15 @@ def test_over_its_own_input(ctx, ty, n_tok, shift):
         want, absum = oracle.matvec_q(int(ty), w, x[t], n, n, n_threads=8)
         tol = fx.matvec_tolerance(n, absum) + 2.0 * 64 * 2.0 ** -24 * absum
         assert np.all(np.abs(got[t] - want) <= tol)
+
+
+@pytest.mark.parametrize("n_tok,rows,cols", [(5, 8200, 256), (20, 8200, 768), (40, 4112, 768),  # matmul.hip
+                                             (40, 4112, 2048), (63, 4100, 1024), (66, 130, 256)])  # 128 x 128 tiles
+@pytest.mark.parametrize("ty", BLOCKS + SUPER, ids=lambda t: t.name)
+def test_where_the_form_ends(ctx, ty, n_tok, rows, cols):
+    # more rows or tokens than it takes (tests/test_dispatch.py has the rule): the other kernels of few tokens.
+    # The tiles' K-quants add up pairs of blocks in the matrix cores (run)
+    _check(ctx, ty, n_tok, rows, cols, run=64)
 
 
 def test_same_product_in_any_chunk_of_a_tile(ctx):
