@@ -219,7 +219,8 @@ __device__ __forceinline__ void mm2_store_halves(const MatmulArgs &a, const MmSe
 }
 
 // The k-blocks [kb0, kb0 + nb) of wave group `group` (of KS) of this work-group's k-slice, cut on a multiple
-// of GRAN; most: the larger group's count, which is the steps (barriers) that every wave goes through.
+// of GRAN (the host halves only slices of two and more); most: the larger group's count, which is the steps
+// (barriers) that every wave goes through.
 struct Mm2Span {
     uint32_t kb0, nb, most;
 };
@@ -653,7 +654,6 @@ __device__ __forceinline__ void mm2_body(const MatmulArgs &a) {
         if (b + 1u < nb) pstep(b + 1u, 1u);
         __builtin_amdgcn_s_waitcnt(mm2_vmcnt(0));  // no copy outlives the work-group
     } else {
-    if (KS == 1 || nb > 0u) {  // (the last k-slice may leave group 1 without a block)
     copy(0, 0);
     if constexpr (Q8) qcopy(0, 0);
     if constexpr (Q6K) k6copy(0);
@@ -678,7 +678,7 @@ __device__ __forceinline__ void mm2_body(const MatmulArgs &a) {
         copy(min(b + 2u, nb - 1u), (buf + 2u) % 3u);
         if constexpr (Q8)
             if (!odd) qcopy(min(b + 2u, nb - 2u), (qb + 1u) % 3u);
-            if constexpr (Q6K) k6copy(min(b + 2u, nb - 1u));
+        if constexpr (Q6K) k6copy(min(b + 2u, nb - 1u));
         if constexpr (MX) xcopy(min(b + 2u, nb - 1u), (qb + 1u) % 3u);
         __builtin_amdgcn_sched_barrier(0);
         compute(buf, qb, odd, b);
@@ -697,7 +697,6 @@ __device__ __forceinline__ void mm2_body(const MatmulArgs &a) {
     if (b + 2u < nb) step(b + 2u, 2, 1, false);
     if (b + 3u < nb) step(b + 3u, 0, 1, true);
     if (b + 4u < nb) step(b + 4u, 1, 2, false);
-    }
     if constexpr (KS == 2)
         for (uint32_t i = nb; i < span.most; ++i) __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_s_waitcnt(mm2_vmcnt(0));  // no copy outlives the work-group

@@ -110,12 +110,10 @@ __device__ __forceinline__ void mm2k_body(const MatmulArgs &a) {
 #pragma unroll
             for (int j = 0; j < 16; ++j) acc[tt][rt][j] = 0.f;
 
-    if (KS == 1 || nsb > 0u) {  // (the last k-slice may leave group 1 without a super-block)
-        copy_hdr(0u, 0u);
-        copy_pair(0u, 0u);
-        copy_act(0u, 0u);
-        copy_act(1u, MM2_ACT);
-    }
+    copy_hdr(0u, 0u);
+    copy_pair(0u, 0u);
+    copy_act(0u, 0u);
+    copy_act(1u, MM2_ACT);
     uint32_t bufo = 0u;              // k-block b's activation buffer, b % 3, as an offset
     for (uint32_t sb = 0; sb < nsb; ++sb) {
         const uint32_t hpar = sb & 1u;

@@ -621,7 +621,8 @@ int decode_launch_body(moearc_ctx *c, void *out, unsigned int out_f16, const flo
         L.nkv0 = a.n_kv[0];
         L.slen0 = split_len;
         L.next0 = a.item_begin[1];
-        L.geo0 = log2u(page_tokens) | (uniform ? MOEARC_DECODE_UNIFORM : 0u) | (cnt > 24 ? MOEARC_DECODE_MANY : 0u) | (uint32_t) n_kv_heads << 16;
+        L.geo0 = log2u(page_tokens) | (uniform ? MOEARC_DECODE_UNIFORM : 0u) | (cnt > 24 ? MOEARC_DECODE_MANY : 0u) |
+                 (uint32_t) n_kv_heads << 16;
         L.geo1 = (uint32_t) nkb | (uint32_t) (n_heads / n_kv_heads) << 16;
         const int rc = launch(c, c->f_dec_fast[kind][variant], (unsigned) wgs, 64u * dv.kb * dv.wpk, L,
                               "attn_decode.split", n_heads, head_dim);

@@ -200,8 +200,8 @@ def test_fused_launches_equal_separate_ones(monkeypatch, dims):
     # the RoPE of q and the K/V append as one launch (moearc_rope_qkv_chunk64_k; after a split q/k/v
     # product moearc_rope_qkv_sums64_k, which also adds the product's k-slice sums and biases in
     # place of its reduction launch), and the prefill writing the output projection's f16 hi + lo
-    # split instead of f32 rows and a split launch. The residual after a 45-token chunk (the
-    # 16-token product), a 128-token one (the MFMA product) and a decode step, and both pools,
+    # split instead of f32 rows and a split launch. The residual after a 45-token chunk, a
+    # 128-token one (at gpt-oss's shape both on the 128 x 128 tiles) and a decode step, and both pools,
     # bit-identical.
     from moearc_amd import Context
     d = GPT_OSS if dims == "gpt_oss" else TOY

@@ -210,7 +210,7 @@ def test_matvec_refusals_and_empty_shapes(ctx):
     (QuantType.Q8_0, 2, 4096, 2880), (QuantType.F16, 129, 2880, 4096),
     # enough work-groups for the 32-rows-per-wave kernels
     (QuantType.Q8_0, 512, 8192, 256), (QuantType.F16, 256, 16384, 128),
-    # the 128 x 128-tile kernels (Q8_0 and F16 from 64 tokens): ragged tiles, k-block counts around
+    # the 128 x 128-tile kernels (from 65 tokens at these few rows): ragged tiles, k-block counts around
     # the three-deep pipeline and its six-block unroll (Q8_0 there only with an even count: its
     # weights travel in pairs of blocks; odd counts, as 224 and 96 columns, take the 16x16 kernels)
     (QuantType.Q8_0, 200, 300, 64), (QuantType.Q8_0, 64, 128, 224), (QuantType.F16, 100, 200, 32),
@@ -221,7 +221,7 @@ def test_matvec_refusals_and_empty_shapes(ctx):
     (QuantType.Q4_K, 37, 200, 1024), (QuantType.Q4_K, 512, 8192, 256), (QuantType.Q5_K, 67, 96, 2048),
     (QuantType.Q5_K, 512, 8192, 256), (QuantType.MXFP4, 37, 200, 1024), (QuantType.MXFP4, 512, 8192, 96),
     (QuantType.Q6_K, 37, 200, 1024), (QuantType.Q6_K, 512, 8192, 256),
-    # Q4_K on the 128 x 128 tiles (from 64 tokens): ragged tiles, super-block counts around the
+    # Q4_K on the 128 x 128 tiles (from 65 tokens here: fewer, and so few rows, take matmul_small.hip): ragged tiles, super-block counts around the
     # three-deep pipeline and its six-block unroll, and a split launch (slices on super-blocks)
     (QuantType.Q4_K, 64, 128, 256), (QuantType.Q4_K, 200, 300, 512), (QuantType.Q4_K, 130, 257, 768),
     (QuantType.Q4_K, 96, 160, 1280), (QuantType.Q4_K, 128, 512, 2048),
