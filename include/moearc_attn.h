@@ -95,7 +95,13 @@ int moearc_kv_append(moearc_ctx *c, void *k_pages, void *v_pages, const float *k
  * n_heads % n_kv_heads != 0 -> -2; kv_begin >= n_kv -> -2; head_dim > 1024 -> -2.
  * Paths: head_dim 64 or 128 with a group of at most 16 heads, a power-of-two page size and a positive
  * scale run the split-K MFMA kernels (f32 KV and head_dim 128 also need out, q and the pages 16-byte
- * aligned); every other accepted shape runs a general f32 kernel. */
+ * aligned); every other accepted shape runs a general f32 kernel.
+ * Under stream capture: with f16 KV and head_dim 64 a call splits as it does eagerly, over the context's
+ * workspace, which an eager call must have grown (else -1). f32 KV and head_dim 128 run one split per
+ * sequence, without memory: a graph of one launch, far slower over long spans (four sequences of 2K-8K keys,
+ * 32 heads over 4 KV heads: 122 us replayed, 14 eager), whose outputs may differ from an eager call's in
+ * their last bits. moearc_attn_decode_batched_noalloc splits them under capture too (19 us). The same happens
+ * eagerly when the device has no memory for the records. */
 int moearc_attn_decode(moearc_ctx *c, float *out, const float *q, const void *k_pages,
                        const void *v_pages, const unsigned int *block_table, const float *sinks,
                        unsigned long n_heads, unsigned long n_kv_heads, unsigned long head_dim,
@@ -115,7 +121,8 @@ int moearc_attn_decode(moearc_ctx *c, float *out, const float *q, const void *k_
  * engine keeps sequence lengths on the host, moe.rs:1890-1912); every other pointer is device
  * memory. Each sequence must equal the single call with the same arguments.
  * Refusals: as moearc_attn_decode per sequence (an empty span in any sequence -> -2), plus
- * n_seqs == 0, out_type not 0/1, or bt_stride < ceil(n_kv[b] / page_tokens) -> -2. */
+ * n_seqs == 0, out_type not 0/1, or bt_stride < ceil(n_kv[b] / page_tokens) -> -2. Under capture: as
+ * moearc_attn_decode. */
 int moearc_attn_decode_batched(moearc_ctx *c, void *out, unsigned int out_type, const float *q,
                                const void *k_pages, const void *v_pages,
                                const unsigned int *block_tables, unsigned long bt_stride,
@@ -133,9 +140,10 @@ int moearc_attn_decode_batched(moearc_ctx *c, void *out, unsigned int out_type, 
  * the call makes no hipMalloc, hipFree, event or host allocation. Limit: with f16 KV and head_dim 64,
  * n_heads x work items x 66 floats must fit the array (64 heads: up to 496 work items; the default
  * split plan uses at most 128); a larger call is refused with -2, checked for every launch of the call
- * before anything is enqueued. (Other shapes are never refused for it: their splits grow to fit.) Calls of one context reuse the array in stream order; calls that overlap in time on one
- * context (e.g. graphs captured from it replayed on other streams concurrently) race. Nothing in the
- * array needs clearing between calls. */
+ * before anything is enqueued. (Other shapes are never refused for it: their splits grow to fit.) Calls of
+ * one context reuse the array in stream order; calls that overlap in time on one context (e.g. graphs
+ * captured from it replayed on other streams concurrently) race. Nothing in the array needs clearing
+ * between calls. */
 int moearc_attn_decode_batched_noalloc(moearc_ctx *c, void *out, unsigned int out_type, const float *q,
                                        const void *k_pages, const void *v_pages,
                                        const unsigned int *block_tables, unsigned long bt_stride,
@@ -151,7 +159,12 @@ int moearc_attn_decode_batched_noalloc(moearc_ctx *c, void *out, unsigned int ou
  * decode per prompt token (moe.rs:1856-1862, moe.rs:2020-2027).
  * q: f16 [n_q][n_heads][head_dim]; out: [n_q][n_heads][head_dim] f32 or f16 by out_type.
  * Requires kv_type 1 (f16), head_dim 64, a group n_heads/n_kv_heads of 1, 2, 4 or 8 and a
- * power-of-two page_tokens; other shapes -> -2. */
+ * power-of-two page_tokens; other shapes -> -2.
+ * A chunk whose query tiles leave compute units idle (short, deep in a context) is cut along the keys and
+ * merged in a second launch, over a workspace of up to 35 MB that grows on demand. Captured calls, and calls
+ * for which the device has no such memory, run the one launch (200 tokens behind 16,301 keys: 312 us, 77 cut);
+ * their outputs may differ in the last bits of the softmax weights' f16 rounding (4e-4 relative; either is
+ * 3e-4 from float64). */
 int moearc_attn_prefill(moearc_ctx *c, void *out, unsigned int out_type, const void *q,
                         const void *k_pages, const void *v_pages, const unsigned int *block_table,
                         const float *sinks, unsigned long n_q, unsigned long pos0,
@@ -306,7 +319,8 @@ typedef struct moearc_attn_block {
  * them), tokens at positions pos0 .. pos0 + n_tok - 1. Working memory is the context's (grown on
  * demand, kept). Refusals: null c, b, h, x, pos, page_ids or slots -> -1; a ring too small for the
  * chunk (see ring_pages) -> -2; then those of the calls above, in that order (nothing is enqueued
- * for a refusal found before the first launch). */
+ * for a refusal found before the first launch). Under capture the working memory must have been grown by an
+ * eager call of the same size, and the attention takes its captured form (moearc_attn_prefill). */
 int moearc_attn_block_chunk(moearc_ctx *c, const moearc_attn_block *b, float *h, const float *x,
                             unsigned long n_tok, unsigned long pos0, const int *pos,
                             const unsigned int *page_ids, const unsigned int *slots);

@@ -2,7 +2,7 @@
 // tokens, straight from the f32 activations in one launch. Bound by latency: the products of matmul.hip
 // split the activations in a launch before, cut the reduction over grid z with one k-block in flight
 // per wave, and added the slices in a launch after. 8 tokens of Q8_0 4096 x 2880 (12.6 MB) went from
-// 21.9 to 8.8 us, of MXFP4 28.0 to 8.4, of Q4_K 4096 x 2048 25.7 to 6.5.
+// 21.9 to 8.8 us, of MXFP4 28.0 to 8.4, of Q4_K 4096 x 2048 25.4 to 6.6.
 //
 // Work-group: 16 weight rows and all tokens; its 8 waves cut the reduction between them (whole
 // super-blocks for the K-quants) and meet once, in LDS, at the end. A wave has CK k-blocks of both

@@ -1806,7 +1806,7 @@ int mm_launch(moearc_ctx *c, unsigned ty, const MmMat *m, unsigned n_mat, const 
         uint64_t want = std::max<uint64_t>(1, std::min<uint64_t>(aim * kMmCUs / tiles, nb / 4));
         // Tiles that fill three quarters of the CUs or more by themselves are not sliced: eight waves to
         // a work-group keep two per SIMD, the two fours halve the reduction between them and meet in LDS, and
-        // there are no partial sums to write, read and add (1000 x 4096 x 2048 Q4_K, 256 tiles: 67 -> 60.5 us,
+        // there are no partial sums to write, read and add (1000 x 4096 x 2048 Q4_K, 256 tiles: 62 -> 55 us,
         // 1000 x 4096 x 2880 Q8_0 77.4 -> 72.5 and F16 75 -> 69, 900 MXFP4 86 -> 80; 192 tiles 66.1 -> 65.3;
         // 160 tiles lose, 48.2 -> 55 and, Q6_K, 65 -> 77). Two slices of such halves tie with four of four
         // waves (128 tiles: 48.5 against 49.9, 44.6 against 45.0, 39.5 against 39.4).
