@@ -84,6 +84,17 @@ def test_product_forms(lib, ty, n_tok, rows, cols, form):
         assert got.startswith(want[form]), got
 
 
+def test_forms_that_the_gpu_tests_mean(lib):
+    # the shapes of test_matmul_halves_gpu.py and test_matmul_kquant_gpu.py run the kernels that those are about
+    with Context() as cx:
+        for ty, cols in [(Q.F16, 544), (Q.Q8_0, 576), (Q.MXFP4, 320), (Q.Q4_K, 768), (Q.Q5_K, 512), (Q.Q6_K, 768)]:
+            for rows in (6017, 8192):
+                assert _product(cx, lib, ty, 400, rows, cols) == f"moearc_matmul2x_{ty.name.lower()}_k"
+        for n_tok, rows, cols in [(65, 1, 256), (70, 129, 512), (128, 128, 2304), (129, 300, 768), (300, 257, 2048)]:
+            for ty in (Q.Q4_K, Q.Q5_K):
+                assert _product(cx, lib, ty, n_tok, rows, cols) == f"moearc_matmul2_{ty.name.lower()}_k"
+
+
 def test_without_the_small_form(lib, monkeypatch):
     # MOEARC_MM_SMALL=0: the kernels that it replaced
     monkeypatch.setenv("MOEARC_MM_SMALL", "0")
