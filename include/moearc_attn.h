@@ -119,7 +119,8 @@ int moearc_attn_decode(moearc_ctx *c, float *out, const float *q, const void *k_
  * out_type), attends [kv_begin[b], n_kv[b]) through block-table row
  * block_tables[b * bt_stride ...]. kv_begin and n_kv are HOST arrays of n_seqs entries (the
  * engine keeps sequence lengths on the host, moe.rs:1890-1912); every other pointer is device
- * memory. Each sequence must equal the single call with the same arguments.
+ * memory. Each sequence equals the single call with the same arguments, to rounding (on the split kernels the
+ * batch as a whole decides how many splits a span has).
  * Refusals: as moearc_attn_decode per sequence (an empty span in any sequence -> -2), plus
  * n_seqs == 0, out_type not 0/1, or bt_stride < ceil(n_kv[b] / page_tokens) -> -2. Under capture: as
  * moearc_attn_decode. */
