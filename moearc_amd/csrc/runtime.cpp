@@ -328,6 +328,7 @@ DecodeKind decode_kind(const void *out, const float *q, const void *k_pages, con
         !is_pow2(page_tokens) || page_tokens > (1ul << 30) || !(scale > 0.f && scale <= 3.0e38f))
         return kGeneral;
     if (kv_type == 1u && head_dim == 64) return kF16D64;
+    if (!(scale * 1.4426950408889634f <= 3.0e38f)) return kGeneral;  // the multiplier in the log2 domain
     if (((uintptr_t) out | (uintptr_t) q | (uintptr_t) k_pages | (uintptr_t) v_pages) % 16 != 0) return kGeneral;
     if (kv_type == 1u) return n_heads / n_kv_heads <= 8 ? kF16D128 : kF16D128G16;
     return head_dim == 64 ? kF32D64 : kF32D128;

@@ -107,8 +107,8 @@ def test_without_the_small_form(lib, monkeypatch):
 BIG = 1 << 44
 
 
-def _decode(cx, kv, dim, n_kv, heads=32, kv_heads=4, page=256, base=1 << 33):
-    cx.attn_decode_ext(*(at(cx, base + i * BIG, BIG) for i in range(6)), heads, kv_heads, dim, 0, n_kv, page, 0.125,
+def _decode(cx, kv, dim, n_kv, heads=32, kv_heads=4, page=256, base=1 << 33, scale=0.125):
+    cx.attn_decode_ext(*(at(cx, base + i * BIG, BIG) for i in range(6)), heads, kv_heads, dim, 0, n_kv, page, scale,
                        KvType.F16 if kv == "f16" else KvType.F32)
 
 
@@ -134,6 +134,16 @@ def test_decode_without_memory_for_records_is_not_split(lib, kv, dim):
         lib.host_hip_largest(1 << 16)  # a workspace that cannot grow
         _decode(cx, kv, dim, 20000, heads=64)
         assert len(names(lib)) == 1
+
+
+@pytest.mark.parametrize("kv,dim", KINDS)
+def test_scales_past_the_log2_domain_take_the_general_kernel(lib, kv, dim):
+    # the split kernels multiply scores by scale * log2(e), which must be finite
+    with Context() as cx:
+        for scale, general in ((2.0e38, False), (2.4e38, True), (0.0, True), (-1.0, True), (1.0e-40, False)):
+            lib.host_hip_reset()
+            _decode(cx, kv, dim, 100, scale=scale)
+            assert (names(lib) == ["moearc_attn_decode_general_k"]) == general
 
 
 def test_prefill_without_memory_for_records_is_not_split(lib):
